@@ -2224,7 +2224,8 @@ int nbg_selftest_pair_host(const double* x0, const double* v0, double k, double 
                            double* out) {
   if (!x0 || !v0 || !out) return -1;
   double delxv[6];
-  const nbg::KParams P = nbg::jac_delxv_gamma(x0, v0, delxv, k, h, drift_first != 0);
+  const nbg::KParams P = drift_first ? nbg::kepler_drift<true>(x0, v0, delxv, k, h)
+                                     : nbg::kepler_drift<false>(x0, v0, delxv, k, h);
   double kep[48], jm[6];
   for (int q = 0; q < 48; ++q) kep[q] = 0.0;
   for (int q = 0; q < 6; ++q) jm[q] = 0.0;

@@ -174,8 +174,17 @@ __device__ inline double jij_coef(const PairSlot& sl, bool rowi, int rk, int k) 
 // no longer fit the instruction cache.  Inputs and outputs pass through the
 // pair's slot in LDS; the arithmetic runs in registers.
 // ---------------------------------------------------------------------------
-static __device__ __attribute__((noinline)) void pair_drift(PairSlot* sl, double gm, double hh, bool drift_first) {
+// The slot is named by its LDS offset, so that its accesses are LDS
+// instructions rather than flat ones.
+typedef __attribute__((address_space(3))) PairSlot LdsSlot;
+__device__ __forceinline__ uint32_t lds_slot(PairSlot* sl) { return (uint32_t)(uintptr_t)(LdsSlot*)sl; }
+__device__ __forceinline__ PairSlot* slot_at(uint32_t off) { return (PairSlot*)(LdsSlot*)(uintptr_t)off; }
+
+// The drift by the general formulas: waves with a lane outside the common
+// case of nbg_pair.h (a long step, a nearly parabolic or radial orbit).
+static __device__ __attribute__((noinline)) void pair_drift_general(uint32_t slot, double gm, double hh, bool drift_first) {
   drift_first = __builtin_amdgcn_readfirstlane((int)drift_first) != 0;  // the same for the whole sweep
+  PairSlot* sl = slot_at(slot);
   double x0[3], v0[3], delxv[6];
   for (int k = 0; k < 3; ++k) {
     x0[k] = sl->x0[k];
@@ -186,8 +195,24 @@ static __device__ __attribute__((noinline)) void pair_drift(PairSlot* sl, double
   for (int k = 0; k < 6; ++k) sl->delxv[k] = delxv[k];
 }
 
-static __device__ __attribute__((noinline)) void pair_jacobian(PairSlot* sl, bool drift_first) {
-  drift_first = __builtin_amdgcn_readfirstlane((int)drift_first) != 0;  // the same for the whole sweep
+template <bool DF> static __device__ __attribute__((noinline)) void pair_drift(uint32_t slot, double gm, double hh) {
+  PairSlot* sl = slot_at(slot);
+  double x0[3], v0[3], delxv[6];
+  for (int k = 0; k < 3; ++k) {
+    x0[k] = sl->x0[k];
+    v0[k] = sl->v0[k];
+  }
+  KParams P;
+  if (jac_delxv_gamma_fast<DF>(x0, v0, delxv, gm, hh, P)) {
+    sl->P = P;
+    for (int k = 0; k < 6; ++k) sl->delxv[k] = delxv[k];
+  } else {
+    pair_drift_general(slot, gm, hh, DF);
+  }
+}
+
+template <bool DF> static __device__ __attribute__((noinline)) void pair_jacobian(uint32_t slot) {
+  PairSlot* sl = slot_at(slot);
   double x0[3], v0[3], kep[48], jm[6];
   for (int k = 0; k < 3; ++k) {
     x0[k] = sl->x0[k];
@@ -199,7 +224,7 @@ static __device__ __attribute__((noinline)) void pair_jacobian(PairSlot* sl, boo
   const double mi = sl->mi, mj = sl->mj, mijinv = sl->mijinv, m_i = sl->m_i, m_j = sl->m_j;
   double dl[6];
   for (int q = 0; q < 6; ++q) dl[q] = sl->delxv[q];
-  compute_jacobian_gamma(P, x0, v0, kep, jm, drift_first);
+  compute_jacobian_gamma(P, x0, v0, kep, jm, DF);
   // jac_ij's mass columns 6 and 13 (the k == 6, 13 cases of jij_coef),
   // formed from registers: reading them back from the slot after the
   // stores below would cost an LDS round trip each
@@ -213,6 +238,11 @@ static __device__ __attribute__((noinline)) void pair_jacobian(PairSlot* sl, boo
   for (int q = 0; q < 48; ++q) sl->kep[q] = kep[q];
   for (int q = 0; q < 6; ++q) sl->jm[q] = jm[q];
   for (int q = 0; q < 24; ++q) sl->mc[q] = mc[q];
+}
+
+__device__ __forceinline__ void pair_jacobian_dir(PairSlot* sl, bool drift_first) {
+  if (drift_first) pair_jacobian<true>(lds_slot(sl));
+  else pair_jacobian<false>(lds_slot(sl));
 }
 
 // ---------------------------------------------------------------------------
@@ -921,7 +951,8 @@ __device__ __attribute__((always_inline)) inline void pair_level_lane(Smem<NB, G
   const double m_i = S.m[i], m_j = S.m[j];
   const double gm = NBG_GNEWT * (m_i + m_j);
   if (gm != 0.0) {
-    pair_drift(&sl, gm, hh, drift_first);
+    if (drift_first) pair_drift<true>(lds_slot(&sl), gm, hh);
+    else pair_drift<false>(lds_slot(&sl), gm, hh);
     const double mijinv = 1.0 / (m_i + m_j);
     const double mi = m_i * mijinv;
     const double mj = m_j * mijinv;
@@ -1045,7 +1076,7 @@ __device__ __attribute__((always_inline)) inline void sweep(Smem<NB, G>& S, Swor
     c0 += cnt;
     if (!(needJ || needQ)) continue;
     // ---- B: analytic Kepler-drift Jacobians, one lane per pair
-    if (lane < cnt && W.slot[lane].valid) pair_jacobian(&W.slot[lane], drift_first);
+    if (lane < cnt && W.slot[lane].valid) pair_jacobian_dir(&W.slot[lane], drift_first);
     wsync();
     // ---- C: jac_ij, Jacobian rows and dq/dt, in sweep order
     sweep_rows<NB, G, WAVE, FACT>(S, W.slot, cnt, needJ, needQ, lane);
@@ -1092,7 +1123,7 @@ __device__ __attribute__((always_inline)) inline void sweep2(Smem<NB, G>& S0, Sm
     if (lane < 2 * cnt) {
       const int sys = lane >= cnt ? 1 : 0;
       PairSlot* sl = slots + sys * ch + (lane - sys * cnt);
-      if ((sys ? pj1 : pj0) && sl->valid) pair_jacobian(sl, drift_first);
+      if ((sys ? pj1 : pj0) && sl->valid) pair_jacobian_dir(sl, drift_first);
     }
     wsync();
     if constexpr (HALF) {  // both systems' rows at once, one per half of the wave

@@ -462,6 +462,283 @@ NBG_HD KParams jac_delxv_gamma(const double* x0, const double* v0, double* delxv
 }
 
 // --------------------------------------------------------------------------
+// The common case of the functions above, as one straight line.  An orbit
+// step is usually a small part of a period (|gamma| < 1/2), its elementary
+// functions lie on their polynomial paths and nothing is near a range limit.
+// A wave issues one instruction at a time, so what a solve costs is the
+// number of instructions on its path: here the range checks, reductions,
+// scaled divisions and special cases of the general functions are replaced by
+// one vote, and a wave with a lane that does not qualify runs the general
+// functions instead (same inputs, from the start).  Every lane's result has
+// the bits the general functions give it.
+// --------------------------------------------------------------------------
+// 1 / c for the series' whole divisors
+template <int C> struct Recip {
+  static constexpr double c = (double)C, rc = 1.0 / (double)C;
+};
+
+// One term of a joint series: the running sum s (previous sums s1, s2) takes
+// v unless its own stopping test has fired before.
+struct SerSum {
+  double s, s1, s2;
+  bool done;
+  NBG_HD void take(double v) {
+    const bool stop = v == s || v == s1;
+    s2 = s1;
+    s1 = s;
+    s = done ? s : v;
+    done = done || stop;
+  }
+};
+
+// series_set's sums for |gamma| < 1/2 (each converges within SER_MAX terms):
+// the divisors are constants, so every quotient is a product with the
+// divisor's reciprocal and one correction (cdiv), and the term of a series
+// that has stopped may run on -- only its sum is kept.
+constexpr int SER_MAX = 12;
+struct SerState {
+  double tg, t1, t2, t3, t5, t6;
+  SerSum g, h1, h2, h3, h5, h6;
+};
+template <int MASK, int N> NBG_HD bool series_terms(double x2, SerState& S) {
+  if constexpr (N <= SER_MAX) {
+    constexpr double f = (double)(1ll << (2 * N + 2));  // 4^(N+1)
+    if constexpr ((MASK & SER_G3) != 0) {
+      using R = Recip<(2 * N + 3) * (2 * N + 2)>;
+      S.tg = S.tg * cdiv(x2, R::c, R::rc);
+      S.g.take(S.g.s + S.tg);
+    }
+    if constexpr ((MASK & SER_H1) != 0) {
+      using R = Recip<(2 * N + 4) * (2 * N + 3) * N>;
+      S.t1 = cdiv(S.t1 * (x2 * (double)(N + 1)), R::c, R::rc);
+      S.h1.take(S.h1.s + S.t1);
+    }
+    if constexpr ((MASK & SER_H2) != 0) {
+      using R = Recip<(4 * N + 6) * N>;
+      S.t2 = cdiv(S.t2 * x2, R::c, R::rc);
+      S.h2.take(S.h2.s + S.t2);
+    }
+    if constexpr ((MASK & SER_H3) != 0) {
+      using R = Recip<(2 * N + 4) * (2 * N + 5)>;
+      S.t3 = cdiv(S.t3 * x2, R::c, R::rc);
+      S.h3.take(S.h3.s + S.t3 * (f - 1.0));
+    }
+    if constexpr ((MASK & SER_H5) != 0) {
+      using R = Recip<(2 * N + 5) * (2 * N + 4) * N>;
+      S.t5 = cdiv(S.t5 * (x2 * (double)(N + 1)), R::c, R::rc);
+      S.h5.take(S.h5.s + S.t5);
+    }
+    if constexpr ((MASK & SER_H6) != 0) {
+      using R = Recip<(2 * N + 5) * (2 * N + 6)>;
+      S.t6 = cdiv(S.t6 * x2, R::c, R::rc);
+      S.h6.take(S.h6.s + S.t6 * ((4.0 * f - (double)(3 * N)) - 7.0));
+    }
+    if constexpr (N >= 4) {  // none converges earlier for a step worth integrating
+      const bool done = S.g.done && S.h1.done && S.h2.done && S.h3.done && S.h5.done && S.h6.done;
+      if (NBG_ALL(done)) return true;
+    }
+    return series_terms<MASK, N + 1>(x2, S);
+  }
+  return false;
+}
+// gfuncs for lanes that all have 2^-60 <= |gamma| < 1/2 and |beta|, sqb in
+// range; false when a series of some lane has not converged.
+template <int MASK> NBG_HD bool series_fast(double gamma, double beta, double sqb, SeriesOut& o) {
+  const double x2 = (-nbg::sign(beta)) * (gamma * gamma);
+  SerState S;
+  auto start = [](double v, int bit) { return SerSum{v, 2.0 * v, 2.0 * v, (MASK & bit) == 0}; };
+  S.tg = 1.0; S.g = start(1.0, SER_G3);
+  S.t1 = 1.0; S.h1 = start(1.0, SER_H1);
+  S.t2 = 1.0; S.h2 = start(1.0, SER_H2);
+  S.t3 = 1.0 / 30.0; S.h3 = start(1.0 / 10.0, SER_H3);
+  S.t5 = 1.0 / 60.0; S.h5 = start(1.0 / 60.0, SER_H5);
+  S.t6 = 1.0 / 360.0; S.h6 = start(1.0 / 40.0, SER_H6);
+  if (!series_terms<MASK, 1>(x2, S)) return false;
+  const double bs = beta * sqb, b2 = beta * beta, x4 = x2 * x2;
+  if constexpr ((MASK & SER_G3) != 0) o.g3 = S.g.s * fdiv((-x2) * gamma, (6.0 * beta) * sqb);
+  if constexpr ((MASK & SER_H1) != 0) o.h1 = S.h1.s * fdiv(x4, 12.0 * b2);
+  if constexpr ((MASK & SER_H2) != 0) o.h2 = S.h2.s * fdiv((-x2) * gamma, (3.0 * beta) * sqb);
+  if constexpr ((MASK & (SER_H3 | SER_H5)) != 0) {
+    const double q = fdiv((-x4) * gamma, bs);
+    if constexpr ((MASK & SER_H3) != 0) o.h3 = S.h3.s * q;
+    if constexpr ((MASK & SER_H5) != 0) o.h5 = S.h5.s * q;
+  }
+  if constexpr ((MASK & SER_H6) != 0) o.h6 = S.h6.s * fdiv(-(x2 * x2 * x2), b2);
+  return true;
+}
+
+// sc_pair on its polynomial paths, with one odd polynomial for sin and sinh:
+// Horner's sums of ksin are those of sinh_poly in -y^2 up to sign (the sign
+// alternates from one multiply-add to the next and rounding is symmetric), so
+// w = -y^2 on elliptic lanes and y^2 on the others serves both.  ANYE / ANYH:
+// some lane of the wave is elliptic / hyperbolic.
+NBG_HD void sc_fast(bool ell, bool anyE, bool anyH, double y, double* sx, double* cx) {
+  const double z = y * y;
+  const double w = ell ? -z : z;
+  double q = fmac(w, F21, F19);
+  q = fmac(q, w, F17);
+  q = fmac(q, w, F15);
+  q = fmac(q, w, F13);
+  q = fmac(q, w, F11);
+  q = fmac(q, w, F9);
+  q = fmac(q, w, F7);
+  q = fmac(q, w, F5);
+  q = fmac(q, w, F3);
+  const double u = y * z;
+  double s = y - u * q, c = 0.0;
+  if (anyE) {
+    double p = fmac(z, F18, -F16);
+    p = fmac(z, p, F14);
+    p = fmac(z, p, -F12);
+    p = fmac(z, p, F10);
+    p = fmac(z, p, -F8);
+    p = fmac(z, p, F6);
+    p = fmac(z, p, -F4);
+    const double hz = 0.5 * z;
+    const double t = 1.0 - hz;
+    c = t + (((1.0 - t) - hz) - (z * z) * p);
+  }
+  if (anyH) {
+    const double s2 = fmad(u, q, y);
+    const double c2 = exp_poly(-y) + s2;
+    s = ell ? s : s2;
+    c = ell ? c : c2;
+  }
+  *sx = s;
+  *cx = c;
+}
+
+NBG_HD bool in_range(double lo, double hi, double x) {
+  return nbg::fabsd(x) >= lo && nbg::fabsd(x) <= hi;
+}
+
+// cubic1 for the start of the Kepler solve; *ok is cleared where a formula
+// would leave the plain range.
+NBG_HD double cubic1_fast(double a, double b, double c, bool* ok) {
+  const double a3 = a * NBG_THIRD;
+  const double Q = a3 * a3 - b * NBG_THIRD;
+  const double R = a3 * a3 * a3 + 0.5 * ((-a3) * b + c);
+  const double R2 = R * R;
+  const double Q3 = Q * Q * Q;
+  const bool three = R2 < Q3;
+  double A = b;
+  if (NBG_ANY(!three)) {
+    const double rad = three ? 1.0 : R2 - Q3;
+    *ok = *ok && in_range(0x1p-400, 0x1p400, rad) && in_range(0x1p-200, 0x1p200, three ? 1.0 : R);
+    const double w = three ? 1.0 : nbg::fabsd(R) + fsqrt(rad);
+    const double k = (-nbg::sign(R)) * nbg::cbrt_core(w);
+    A = three ? b : k;
+  }
+  const double d = fdiv(three ? -c : Q, A);
+  return three ? d : (A + d) - a3;
+}
+
+template <bool DF>
+NBG_HD bool jac_delxv_gamma_fast(const double* x0, const double* v0, double* delxv, double k, double h, KParams& P) {
+  double y0[3];
+  for (int j = 0; j < 3; ++j) y0[j] = DF ? x0[j] - h * v0[j] : x0[j];
+  const double rr = dot3(y0), vv = dot3(v0);
+  const double r0 = fsqrt(rr);
+  const double r0inv = fdiv(1.0, r0);
+  const double beta0 = (2.0 * k) * r0inv - vv;
+  const double signb = nbg::sign(beta0);
+  const double ab = signb * beta0;
+  const double beta0inv = fdiv(1.0, beta0);
+  const double sqb = fsqrt(ab);
+  const double zeta = k - r0 * beta0;
+  const double eta = dot3(y0, v0);
+  bool ok = in_range(0x1p-60, 0x1p60, r0) && in_range(0x1p-60, 0x1p60, beta0) && in_range(0x1p-60, 0x1p60, zeta) &&
+            in_range(0x1p-100, 0x1p60, k) && in_range(0x1p-60, 0x1p60, h) && nbg::fabsd(eta) <= 0x1p60;
+  const double zinv = fdiv(6.0, zeta);
+  double gamma = cubic1_fast(((0.5 * eta) * sqb) * zinv, ((r0 * signb) * beta0) * zinv,
+                             ((((-h) * signb) * beta0) * sqb) * zinv, &ok);
+  if (!NBG_ALL(ok)) return false;
+  double gamma1 = 2.0 * gamma, gamma2 = 3.0 * gamma;
+  int iter = 0;
+  const double c2 = (-2.0) * zeta;
+  const double c3 = ((2.0 * eta) * signb) * sqb;
+  const double c4 = ((-sqb) * h) * beta0;
+  const double c6 = (2.0 * signb) * zeta;
+  const double c7 = r0 * beta0;
+  const bool ell = beta0 > 0.0;
+  const bool anyE = NBG_ANY(ell), anyH = NBG_ANY(!ell);
+  // |gamma / 2| up to which sc_pair's polynomials apply without reduction
+  // (|y| 2/pi < 1/2, |y| log2 e < 1/2); the series below want |gamma| < 1/2
+  const double ymax = ell ? 0.75 : 0.34;
+  double sx = 0.0, cx = 0.0, used = gamma;
+  bool run = true;
+  do {
+    const double xx = 0.5 * gamma;
+    ok = ok && in_range(0x1p-27, ymax, xx);
+    if (!NBG_ALL(ok)) return false;
+    used = gamma;
+    sc_fast(ell, anyE, anyH, xx, &sx, &cx);
+    const double ss = sx * sx;
+    const double num = ((k * gamma + (c2 * sx) * cx) + c3 * ss) + c4;
+    const double den = (c6 * ss + (c3 * sx) * cx) + c7;
+    ok = in_range(0x1p-200, 0x1p200, den);
+    const double gn = gamma - fdiv(num, den);
+    if (run) {
+      gamma2 = gamma1;
+      gamma1 = gamma;
+      gamma = gn;
+      iter += 1;
+      run = !(gamma == gamma2 || gamma == gamma1) && iter < 20;
+    }
+  } while (NBG_ANY(run));
+  ok = ok && in_range(0x1p-27, 0x1.fffffep-2, gamma) && nbg::fabsd(gamma) <= 2.0 * ymax;
+  if (!NBG_ALL(ok)) return false;
+  // the last evaluation stands when every lane's gamma has repeated it
+  if (!NBG_ALL(gamma == used)) sc_fast(ell, anyE, anyH, 0.5 * gamma, &sx, &cx);
+  const double g1bs = fdiv((2.0 * sx) * cx, sqb);
+  const double g2bs = ((2.0 * signb) * (sx * sx)) * beta0inv;
+  const double g0bs = 1.0 - beta0 * g2bs;
+  const double r = (r0 * g0bs + eta * g1bs) + k * g2bs;
+  ok = in_range(0x1p-100, 0x1p100, r);
+  const double rinv = fdiv(1.0, r);
+  SeriesOut so = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  if (!series_fast<DF ? SER_G3 : (SER_G3 | SER_H1 | SER_H2)>(gamma, beta0, sqb, so)) return false;
+  if (!NBG_ALL(ok)) return false;
+  const double g3bs = so.g3, h1 = so.h1, h2 = so.h2;
+  const double dfdt = (((-k) * g1bs) * rinv) * r0inv;
+  double fm1, gmh, dgdtm1;
+  if (DF) {
+    fm1 = ((-k) * r0inv) * g2bs;
+    gmh = (k * r0inv) * (h * g2bs - r0 * g3bs);
+    dgdtm1 = ((k * r0inv) * rinv) * (h * g1bs - r0 * g2bs);
+  } else {
+    fm1 = (k * rinv) * (g2bs - (k * r0inv) * h1);
+    gmh = (k * rinv) * (r0 * h2 + eta * h1);
+    dgdtm1 = ((-k) * rinv) * g2bs;
+  }
+  for (int j = 0; j < 3; ++j) delxv[j] = fm1 * x0[j] + gmh * v0[j];
+  for (int j = 0; j < 3; ++j) delxv[3 + j] = dfdt * x0[j] + dgdtm1 * v0[j];
+  P.gamma = gamma; P.g0 = g0bs; P.g1 = g1bs; P.g2 = g2bs; P.g3 = g3bs; P.h1 = h1; P.h2 = h2;
+  P.dfdt = dfdt; P.fm1 = fm1; P.gmh = gmh; P.dgdtm1 = dgdtm1; P.r0 = r0; P.r = r;
+  P.r0inv = r0inv; P.rinv = rinv; P.k = k; P.h = h; P.beta = beta0; P.betainv = beta0inv;
+  P.eta = eta; P.sqb = sqb; P.zeta = zeta; P.iters = iter;
+  return true;
+}
+
+// jac_delxv_gamma! by the common case where the wave allows it
+template <bool DF> NBG_HD KParams kepler_drift(const double* x0, const double* v0, double* delxv, double k, double h) {
+  KParams P;
+  if (!jac_delxv_gamma_fast<DF>(x0, v0, delxv, k, h, P)) P = jac_delxv_gamma(x0, v0, delxv, k, h, DF);
+  return P;
+}
+
+// gfuncs by the common case where the wave allows it
+template <int MASK> NBG_HD_COLD SeriesOut gfuncs_general(double gamma, double beta, double sqb) {
+  return gfuncs<MASK>(gamma, beta, sqb);
+}
+template <int MASK> NBG_HD SeriesOut gfuncs_fast(double gamma, double beta, double sqb) {
+  SeriesOut o = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  const bool ok = in_range(0x1p-60, 0x1.fffffep-2, gamma) && in_range(0x1p-60, 0x1p60, beta);
+  if (NBG_ALL(ok) && series_fast<MASK>(gamma, beta, sqb, o)) return o;
+  return gfuncs_general<MASK>(gamma, beta, sqb);
+}
+
+// --------------------------------------------------------------------------
 // compute_jacobian_gamma!: ahl21.jl:896-1139 (debug = false).  Pinned by the
 // f128 central finite differences of test_kepler_driftij_gamma.jl:4-282
 // (both drift_first, elliptic and hyperbolic).
@@ -491,7 +768,7 @@ void compute_jacobian_gamma(const KParams& P, const double* x0, const double* v0
     double c9 = (((double)(2) * g2) * h) - (((double)(3) * g3) * r0);
     double c10 = (k * (r0inv2 * r0inv2)) * ((((-g2) * r0) * h + ((k * c9) * betainv)) - ((c3 * c13) * rinv));
     double c24 = r0inv3 * ((r0 * (((double)(2) * k) * r0inv - beta)) * betainv - ((g1 * c3) * rinv) / g2);
-    const SeriesOut so = gfuncs<SER_H1 | SER_H2 | SER_H3 | SER_H5 | SER_H6>(gamma, beta, sqb);
+    const SeriesOut so = gfuncs_fast<SER_H1 | SER_H2 | SER_H3 | SER_H5 | SER_H6>(gamma, beta, sqb);
     double h6 = so.h6;
     double dfm1dxx = fm1 * c24;
     double dfm1dxv = (-fm1) * (g1 * rinv + h * c24);
@@ -620,7 +897,7 @@ void compute_jacobian_gamma(const KParams& P, const double* x0, const double* v0
     double c18 = eta * g1 + ((double)(2) * g2) * k;
     double c19 = ((double)(4) * eta) * h1 + ((double)(3) * h2) * r0;
     double c23 = h2 * k - r0 * g1;
-    const SeriesOut so = gfuncs<SER_H3 | SER_H5 | SER_H6>(gamma, beta, sqb);
+    const SeriesOut so = gfuncs_fast<SER_H3 | SER_H5 | SER_H6>(gamma, beta, sqb);
     double h6 = so.h6;
     double h3 = so.h3;
     double h5 = so.h5;
