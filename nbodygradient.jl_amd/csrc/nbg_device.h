@@ -72,7 +72,7 @@ template <int NB, bool G = (NB >= JGLOBAL_MIN)> struct Smem {
   int seq;  // the system has such a pair: sweeps keep the sequential order
   int rowupd;  // SysDesc::rowupd: the form of the Jacobian row update (pair_cols)
   double dqij[14];       // dqdt_ij
-  double x[N3], v[N3], xe[N3], ve[N3], m[NB];
+  double x[N3], v[N3], xe[N3], ve[N3], m[NB];  // in this order (drift_levels)
   double px[N3], pv[N3], pxe[N3], pve[N3];  // s_prior
   double a[N3];
   double dqdt[N7], pdqdt[N7], dqdt_phi[N7], dqdt_kick[N7];
@@ -195,19 +195,123 @@ static __device__ __attribute__((noinline)) void pair_drift_general(uint32_t slo
   for (int k = 0; k < 6; ++k) sl->delxv[k] = delxv[k];
 }
 
-template <bool DF> static __device__ __attribute__((noinline)) void pair_drift(uint32_t slot, double gm, double hh) {
-  PairSlot* sl = slot_at(slot);
-  double x0[3], v0[3], delxv[6];
-  for (int k = 0; k < 3; ++k) {
-    x0[k] = sl->x0[k];
-    v0[k] = sl->v0[k];
-  }
-  KParams P;
-  if (jac_delxv_gamma_fast<DF>(x0, v0, delxv, gm, hh, P)) {
-    sl->P = P;
-    for (int k = 0; k < 6; ++k) sl->delxv[k] = delxv[k];
-  } else {
-    pair_drift_general(slot, gm, hh, DF);
+// Phase A of a sweep: the Kepler drifts and Kahan state updates
+// (kepler_driftij_gamma!, ahl21.jl:706-733) of the levels [lev, end), one
+// lane per pair of a level: of one system, or of two of equal schedule (lanes
+// [0, w) the first's pairs, [w, 2w) the second's).  One out-of-line copy of
+// each direction serves every body count, and a call a run of levels: what a
+// call saves and restores, and the constants it sets up, are paid once per
+// run, and waves of different body counts share the code in the instruction
+// cache.  Records and slots are named by LDS offsets.
+struct LevelRun {
+  uint32_t x0, x1;        // the records' x (then v, xerror, verror, m)
+  uint32_t slot0, slot1;  // the run's first slots
+  uint32_t pl, lw;        // the schedule: the run's first pair, the first level's width
+  int n3;                 // 3 n
+  int levels;
+  int two;                // a second system
+  int store;              // the pair Jacobians follow: keep their inputs in the slots
+  double hh0, hh1;
+};
+template <class T> __device__ __forceinline__ T* lds_at(uint32_t off) {
+  return (T*)(__attribute__((address_space(3))) T*)(uintptr_t)off;
+}
+template <class T> __device__ __forceinline__ uint32_t lds_off(const T* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const T*)p;
+}
+template <bool DF> static __device__ __attribute__((noinline)) void drift_levels(LevelRun R) {
+  const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  const int levels = __builtin_amdgcn_readfirstlane(R.levels), n3 = __builtin_amdgcn_readfirstlane(R.n3);
+  const bool two = __builtin_amdgcn_readfirstlane(R.two) != 0, store = __builtin_amdgcn_readfirstlane(R.store) != 0;
+  const uint8_t* lw = lds_at<uint8_t>(__builtin_amdgcn_readfirstlane(R.lw));
+  const uint8_t* pl = lds_at<uint8_t>(__builtin_amdgcn_readfirstlane(R.pl));
+  // the next level's width and pairs are read while this one is solved
+  auto pair_of = [&](int q0, int w) { return lane - (lane >= w ? w : 0) + q0; };
+  int q0 = 0, w = __builtin_amdgcn_readfirstlane((int)lw[0]);
+  int q = pair_of(0, w);
+  uint32_t ij = 0;
+  if (lane < (two ? 2 * w : w)) ij = pl[2 * q] | ((uint32_t)pl[2 * q + 1] << 8);
+#pragma unroll 1
+  for (int L = 0; L < levels; ++L) {
+    const int w1 = L + 1 < levels ? (int)lw[L + 1] : 0;
+    if (lane < (two ? 2 * w : w)) {
+      const bool second = lane >= w;
+      double* x = lds_at<double>(second ? R.x1 : R.x0);
+      double* v = x + n3;
+      PairSlot* sl = slot_at((second ? R.slot1 : R.slot0) + (uint32_t)(q * sizeof(PairSlot)));
+      const double hh = second ? R.hh1 : R.hh0;
+      const int i = ij & 0xff, j = ij >> 8;
+      // every LDS operand is read into registers before anything is written
+      // back: the compiler cannot tell the slot from the state arrays, so
+      // interleaved reads and writes would each wait for the previous write
+      double xi[3], xj[3], vi[3], vj[3], exi[3], exj[3], evi[3], evj[3], x0[3], v0[3], d[6];
+      for (int k = 0; k < 3; ++k) {
+        xi[k] = x[3 * i + k];
+        xj[k] = x[3 * j + k];
+        vi[k] = v[3 * i + k];
+        vj[k] = v[3 * j + k];
+      }
+      const double m_i = x[4 * n3 + i], m_j = x[4 * n3 + j];
+      for (int k = 0; k < 3; ++k) {
+        exi[k] = x[2 * n3 + 3 * i + k];
+        exj[k] = x[2 * n3 + 3 * j + k];
+        evi[k] = x[3 * n3 + 3 * i + k];
+        evj[k] = x[3 * n3 + 3 * j + k];
+      }
+      for (int k = 0; k < 3; ++k) {
+        x0[k] = xi[k] - xj[k];
+        v0[k] = vi[k] - vj[k];
+      }
+      const double gm = NBG_GNEWT * (m_i + m_j);
+      if (gm != 0.0) {
+        KParams P;
+        double mijinv;
+        if (jac_delxv_gamma_fast<DF>(x0, v0, d, gm, hh, P)) {
+          mijinv = fdiv(1.0, m_i + m_j);  // gm is in the plain range
+          if (store) {
+            sl->P = P;
+            for (int k = 0; k < 3; ++k) {
+              sl->x0[k] = x0[k];
+              sl->v0[k] = v0[k];
+            }
+            for (int k = 0; k < 6; ++k) sl->delxv[k] = d[k];
+          }
+        } else {
+          for (int k = 0; k < 3; ++k) {
+            sl->x0[k] = x0[k];
+            sl->v0[k] = v0[k];
+          }
+          pair_drift_general(lds_slot(sl), gm, hh, DF);
+          for (int k = 0; k < 6; ++k) d[k] = sl->delxv[k];
+          mijinv = 1.0 / (m_i + m_j);
+        }
+        const double mi = m_i * mijinv;
+        const double mj = m_j * mijinv;
+        for (int k = 0; k < 3; ++k) {
+          kahan(xi[k], exi[k], mj * d[k]);
+          kahan(xj[k], exj[k], (-mi) * d[k]);
+          kahan(vi[k], evi[k], mj * d[3 + k]);
+          kahan(vj[k], evj[k], (-mi) * d[3 + k]);
+        }
+        for (int k = 0; k < 3; ++k) {
+          x[3 * i + k] = xi[k];
+          x[3 * j + k] = xj[k];
+          v[3 * i + k] = vi[k];
+          v[3 * j + k] = vj[k];
+          x[2 * n3 + 3 * i + k] = exi[k];
+          x[2 * n3 + 3 * j + k] = exj[k];
+          x[3 * n3 + 3 * i + k] = evi[k];
+          x[3 * n3 + 3 * j + k] = evj[k];
+        }
+        if (store) { sl->mi = mi; sl->mj = mj; sl->mijinv = mijinv; sl->m_i = m_i; sl->m_j = m_j; }
+      }
+      if (store) { sl->valid = (gm != 0.0); sl->i = i; sl->j = j; }
+    }
+    q0 += w;
+    w = __builtin_amdgcn_readfirstlane(w1);
+    q = pair_of(q0, w);
+    if (lane < (two ? 2 * w : w)) ij = pl[2 * q] | ((uint32_t)pl[2 * q + 1] << 8);
+    wsync();
   }
 }
 
@@ -926,69 +1030,26 @@ __device__ inline void pair_cols(Smem<NB, G>& S, const PairSlot& sl, int i, int 
 // state, so running all state updates of a chunk before its Jacobian updates
 // gives the reference's results exactly.
 // ---------------------------------------------------------------------------
-// Phase A for one lane: the Kepler drift of pair (i, j) of system S into
-// slot sl and the Kahan update of the two bodies' state.
+// Phase A of the levels [lev, end) of a sweep (pairs from c0 on) of one
+// system, or of two at once.
 template <int NB, bool G>
-__device__ __attribute__((always_inline)) inline void pair_level_lane(Smem<NB, G>& S, PairSlot& sl, int i, int j,
-                                                                      double hh, bool drift_first) {
-  // every LDS operand is read into registers before anything is written
-  // back: the compiler cannot tell the slot from the state arrays, so
-  // interleaved reads and writes would each wait for the previous write (a
-  // dozen LDS round trips in a row per level)
-  {
-    double xi[3], xj[3], vi[3], vj[3];
-    for (int k = 0; k < 3; ++k) {
-      xi[k] = S.x[3 * i + k];
-      xj[k] = S.x[3 * j + k];
-      vi[k] = S.v[3 * i + k];
-      vj[k] = S.v[3 * j + k];
-    }
-    for (int k = 0; k < 3; ++k) {
-      sl.x0[k] = xi[k] - xj[k];
-      sl.v0[k] = vi[k] - vj[k];
-    }
-  }
-  const double m_i = S.m[i], m_j = S.m[j];
-  const double gm = NBG_GNEWT * (m_i + m_j);
-  if (gm != 0.0) {
-    if (drift_first) pair_drift<true>(lds_slot(&sl), gm, hh);
-    else pair_drift<false>(lds_slot(&sl), gm, hh);
-    const double mijinv = 1.0 / (m_i + m_j);
-    const double mi = m_i * mijinv;
-    const double mj = m_j * mijinv;
-    double d[6], xi[3], xj[3], vi[3], vj[3], exi[3], exj[3], evi[3], evj[3];
-    for (int k = 0; k < 6; ++k) d[k] = sl.delxv[k];
-    for (int k = 0; k < 3; ++k) {
-      xi[k] = S.x[3 * i + k];
-      exi[k] = S.xe[3 * i + k];
-      xj[k] = S.x[3 * j + k];
-      exj[k] = S.xe[3 * j + k];
-      vi[k] = S.v[3 * i + k];
-      evi[k] = S.ve[3 * i + k];
-      vj[k] = S.v[3 * j + k];
-      evj[k] = S.ve[3 * j + k];
-    }
-    for (int k = 0; k < 3; ++k) {
-      kahan(xi[k], exi[k], mj * d[k]);
-      kahan(xj[k], exj[k], (-mi) * d[k]);
-    }
-    for (int k = 0; k < 3; ++k) {
-      kahan(vi[k], evi[k], mj * d[3 + k]);
-      kahan(vj[k], evj[k], (-mi) * d[3 + k]);
-    }
-    for (int k = 0; k < 3; ++k) {
-      S.x[3 * i + k] = xi[k];
-      S.xe[3 * i + k] = exi[k];
-      S.x[3 * j + k] = xj[k];
-      S.xe[3 * j + k] = exj[k];
-      S.v[3 * i + k] = vi[k];
-      S.ve[3 * i + k] = evi[k];
-      S.v[3 * j + k] = vj[k];
-      S.ve[3 * j + k] = evj[k];
-    }
-    sl.mi = mi; sl.mj = mj; sl.mijinv = mijinv; sl.m_i = m_i; sl.m_j = m_j;
-  }
-  sl.valid = (gm != 0.0); sl.i = i; sl.j = j;
+__device__ __forceinline__ LevelRun level_run(Smem<NB, G>& S, PairSlot* slots, int dir, int lev, int end, int c0,
+                                              double hh, bool store) {
+  LevelRun R;
+  R.x0 = R.x1 = lds_off(S.x);
+  R.slot0 = R.slot1 = lds_off(slots);
+  R.pl = lds_off(S.plist[dir] + 2 * c0);
+  R.lw = lds_off(S.lvw[dir] + lev);
+  R.n3 = 3 * NB;
+  R.levels = end - lev;
+  R.two = 0;
+  R.store = store;
+  R.hh0 = R.hh1 = hh;
+  return R;
+}
+__device__ __forceinline__ void run_levels(const LevelRun& R, bool drift_first) {
+  if (drift_first) drift_levels<true>(R);
+  else drift_levels<false>(R);
 }
 
 // Phase C of one chunk of `cnt` pairs (slots[0..cnt)) of system S, with the
@@ -1052,26 +1113,14 @@ __device__ __attribute__((always_inline)) inline void sweep(Smem<NB, G>& S, Swor
   constexpr int CH = Swork<NB>::CH;
   const bool drift_first = (dir == 0);
   const int nlev = S.nlv[dir];
-  const uint8_t* pl = S.plist[dir];
   const uint8_t* lw = S.lvw[dir];
   int lev = 0, c0 = 0;
   while (lev < nlev) {
     // a chunk is a run of whole levels holding at most CH pairs
     int cnt = 0, lev_end = lev;
     while (lev_end < nlev && cnt + lw[lev_end] <= CH) cnt += lw[lev_end++];
-    // ---- A: Kepler drifts and state updates, one level at a time: the
-    // pairs of a level share no body, so lane l solves pair l of the level
-    int q0 = 0;
-#pragma unroll 1
-    for (int L = lev; L < lev_end; ++L) {
-      const int w = lw[L];
-      if (lane < w) {
-        const int q = q0 + lane;
-        pair_level_lane<NB>(S, W.slot[q], pl[2 * (c0 + q)], pl[2 * (c0 + q) + 1], hh, drift_first);
-      }
-      q0 += w;
-      wsync();
-    }
+    // ---- A: Kepler drifts and state updates, one level at a time
+    run_levels(level_run<NB>(S, W.slot, dir, lev, lev_end, c0, hh, needJ || needQ), drift_first);
     lev = lev_end;
     c0 += cnt;
     if (!(needJ || needQ)) continue;
@@ -1096,27 +1145,18 @@ __device__ __attribute__((always_inline)) inline void sweep2(Smem<NB, G>& S0, Sm
                                                              bool nJ1, bool nQ1, int lane) {
   const bool drift_first = (dir == 0);
   const int nlev = S0.nlv[dir];
-  const uint8_t* pl = S0.plist[dir];
   const uint8_t* lw = S0.lvw[dir];
   const bool pj0 = nJ0 || nQ0, pj1 = nJ1 || nQ1;
   int lev = 0, c0 = 0;
   while (lev < nlev) {
     int cnt = 0, lev_end = lev;
     while (lev_end < nlev && cnt + lw[lev_end] <= ch) cnt += lw[lev_end++];
-    int q0 = 0;
-#pragma unroll 1
-    for (int L = lev; L < lev_end; ++L) {
-      const int w = lw[L];
-      if (lane < 2 * w) {
-        const int sys = lane >= w ? 1 : 0;
-        const int q = q0 + lane - sys * w;
-        Smem<NB, G>& S = sys ? S1 : S0;
-        pair_level_lane<NB>(S, slots[sys * ch + q], pl[2 * (c0 + q)], pl[2 * (c0 + q) + 1], sys ? hh1 : hh0,
-                            drift_first);
-      }
-      q0 += w;
-      wsync();
-    }
+    LevelRun R = level_run<NB>(S0, slots, dir, lev, lev_end, c0, hh0, pj0 || pj1);
+    R.two = 1;
+    R.x1 = lds_off(S1.x);
+    R.slot1 = lds_off(slots + ch);
+    R.hh1 = hh1;
+    run_levels(R, drift_first);
     lev = lev_end;
     c0 += cnt;
     if (!(pj0 || pj1)) continue;

@@ -25,6 +25,8 @@
 // the full double range.
 #pragma once
 
+#include <stdint.h>
+
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
 #define NBG_HD __host__ __device__ inline
@@ -39,8 +41,8 @@
 // qualifies, so the branch is scalar and each lane's result is exactly what
 // the general path would give it.
 #if defined(__HIP_DEVICE_COMPILE__)
-#define NBG_ALL(p) (__all((int)(p)) != 0)
-#define NBG_ANY(p) (__any((int)(p)) != 0)
+#define NBG_ALL(p) (__builtin_amdgcn_ballot_w64(!(p)) == 0)
+#define NBG_ANY(p) (__builtin_amdgcn_ballot_w64((p)) != 0)
 #else
 #define NBG_ALL(p) (p)
 #define NBG_ANY(p) (p)
@@ -135,6 +137,34 @@ NBG_HD double fsqrt(double x) {
   return __builtin_sqrt(x);
 #endif
 }
+// a / b given r, 1 / b to about an ulp (the same correction).
+NBG_HD double fdiv_by(double a, double b, double r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double q = a * r;
+  return __builtin_fma(__builtin_fma(-b, q, a), r, q);
+#else
+  (void)r;
+  return a / b;
+#endif
+}
+// sqrt(x), and its reciprocal to about an ulp for fdiv_by: the iteration has it.
+NBG_HD double fsqrt_recip(double x, double* r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double e = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, e, g);
+  h = __builtin_fma(h, e, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  const double q = h + h;
+  *r = __builtin_fma(__builtin_fma(-g, q, 1.0), q, q);
+  return g;
+#else
+  *r = 0.0;
+  return __builtin_sqrt(x);
+#endif
+}
 // a / c for a small positive whole number c, given rc = the double nearest to
 // 1 / c: a * rc is within 1.5 ulp of the quotient, its remainder is exact, and
 // the corrected quotient is within 2^-51 ulp of a / c before its one rounding,
@@ -150,6 +180,8 @@ NBG_HD double fabsd(double x) { return __builtin_fabs(x); }
 NBG_HD double copysignd(double a, double b) { return __builtin_copysign(a, b); }
 NBG_HD double ldexpd(double x, int e) { return __builtin_ldexp(x, e); }
 NBG_HD double frexpd(double x, int* e) { return __builtin_frexp(x, e); }
+// the upper 32 bits of |x|: orders like |x| itself
+NBG_HD int32_t hi_word(double x) { return (int32_t)((__builtin_bit_cast(uint64_t, x) >> 32) & 0x7fffffff); }
 NBG_HD double infd() { return __builtin_inf(); }
 
 // sin(hi + lo) on |hi| <= ~pi/4 (lo: tail of the reduced argument):
@@ -435,6 +467,25 @@ NBG_HD double cbrt_core(double x) {
   const double res = fmad(p, y, -m) + pe * y;
   y = y - fdiv(res, 3.0 * p);
   return copysignd(ldexpd(y, e / 3), x);
+}
+
+// cbrt_core for x in [2^-100, 2^100]: the device starts from the hardware's
+// single-precision logarithm and exponential (within 3e-6, so one Halley step
+// reaches 2e-17), 20 instructions against 60.  The polish's result is the
+// cube root to about 2^-105 before its one rounding, so where it started from
+// does not show.
+NBG_HD double cbrt_mid(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)x) * 0.33333334f);
+  const double t = y * y * y;
+  y = fdiv(y * (t + 2.0 * x), 2.0 * t + x);
+  const double p = y * y;
+  const double pe = fmad(y, y, -p);
+  const double res = fmad(p, y, -x) + pe * y;
+  return y - fdiv(res, 3.0 * p);
+#else
+  return cbrt_core(x);
+#endif
 }
 
 NBG_HD double cbrt(double x) {

@@ -477,135 +477,129 @@ template <int C> struct Recip {
   static constexpr double c = (double)C, rc = 1.0 / (double)C;
 };
 
-// One term of a joint series: the running sum s (previous sums s1, s2) takes
-// v unless its own stopping test has fired before.
-struct SerSum {
-  double s, s1, s2;
-  bool done;
-  NBG_HD void take(double v) {
-    const bool stop = v == s || v == s1;
-    s2 = s1;
-    s1 = s;
-    s = done ? s : v;
-    done = done || stop;
-  }
-};
-
-// series_set's sums for |gamma| < 1/2 (each converges within SER_MAX terms):
-// the divisors are constants, so every quotient is a product with the
-// divisor's reciprocal and one correction (cdiv), and the term of a series
-// that has stopped may run on -- only its sum is kept.
-constexpr int SER_MAX = 12;
-struct SerState {
-  double tg, t1, t2, t3, t5, t6;
-  SerSum g, h1, h2, h3, h5, h6;
-};
-template <int MASK, int N> NBG_HD bool series_terms(double x2, SerState& S) {
-  if constexpr (N <= SER_MAX) {
-    constexpr double f = (double)(1ll << (2 * N + 2));  // 4^(N+1)
-    if constexpr ((MASK & SER_G3) != 0) {
+// series_set for lanes that all have 2^-60 <= |gamma| < 1/2 and |beta|, sqb in
+// range, its sums with a fixed number of terms.  Every series' terms fall by
+// more than a factor 60 from one to the next, so the first one too small to
+// change its sum is where its loop stops (the sum repeats; no earlier term can
+// undo a change), and every later one leaves the sum as it is: with all terms
+// of at least 2^-54 of the sum at gamma^2 = 1/4 -- six, seven for H3 and H6 --
+// the sum is the loop's.  The divisors are constants, so a quotient is a
+// product with the divisor's reciprocal and one correction (cdiv).
+constexpr int SER_TERMS = 6, SER_TERMS_36 = 7;
+template <int N> struct SerTerm {
+  static constexpr double f = (double)(1ll << (2 * N + 2));  // 4^(N+1)
+  template <int MASK> NBG_HD static void add(double x2, SeriesOut& t, SeriesOut& s) {
+    if constexpr ((MASK & SER_G3) != 0 && N <= SER_TERMS) {
       using R = Recip<(2 * N + 3) * (2 * N + 2)>;
-      S.tg = S.tg * cdiv(x2, R::c, R::rc);
-      S.g.take(S.g.s + S.tg);
+      t.g3 = t.g3 * cdiv(x2, R::c, R::rc);
+      s.g3 = s.g3 + t.g3;
     }
-    if constexpr ((MASK & SER_H1) != 0) {
+    if constexpr ((MASK & SER_H1) != 0 && N <= SER_TERMS) {
       using R = Recip<(2 * N + 4) * (2 * N + 3) * N>;
-      S.t1 = cdiv(S.t1 * (x2 * (double)(N + 1)), R::c, R::rc);
-      S.h1.take(S.h1.s + S.t1);
+      t.h1 = cdiv(t.h1 * (x2 * (double)(N + 1)), R::c, R::rc);
+      s.h1 = s.h1 + t.h1;
     }
-    if constexpr ((MASK & SER_H2) != 0) {
+    if constexpr ((MASK & SER_H2) != 0 && N <= SER_TERMS) {
       using R = Recip<(4 * N + 6) * N>;
-      S.t2 = cdiv(S.t2 * x2, R::c, R::rc);
-      S.h2.take(S.h2.s + S.t2);
+      t.h2 = cdiv(t.h2 * x2, R::c, R::rc);
+      s.h2 = s.h2 + t.h2;
     }
     if constexpr ((MASK & SER_H3) != 0) {
       using R = Recip<(2 * N + 4) * (2 * N + 5)>;
-      S.t3 = cdiv(S.t3 * x2, R::c, R::rc);
-      S.h3.take(S.h3.s + S.t3 * (f - 1.0));
+      t.h3 = cdiv(t.h3 * x2, R::c, R::rc);
+      s.h3 = s.h3 + t.h3 * (f - 1.0);
     }
-    if constexpr ((MASK & SER_H5) != 0) {
+    if constexpr ((MASK & SER_H5) != 0 && N <= SER_TERMS) {
       using R = Recip<(2 * N + 5) * (2 * N + 4) * N>;
-      S.t5 = cdiv(S.t5 * (x2 * (double)(N + 1)), R::c, R::rc);
-      S.h5.take(S.h5.s + S.t5);
+      t.h5 = cdiv(t.h5 * (x2 * (double)(N + 1)), R::c, R::rc);
+      s.h5 = s.h5 + t.h5;
     }
     if constexpr ((MASK & SER_H6) != 0) {
       using R = Recip<(2 * N + 5) * (2 * N + 6)>;
-      S.t6 = cdiv(S.t6 * x2, R::c, R::rc);
-      S.h6.take(S.h6.s + S.t6 * ((4.0 * f - (double)(3 * N)) - 7.0));
+      t.h6 = cdiv(t.h6 * x2, R::c, R::rc);
+      s.h6 = s.h6 + t.h6 * ((4.0 * f - (double)(3 * N)) - 7.0);
     }
-    if constexpr (N >= 4) {  // none converges earlier for a step worth integrating
-      const bool done = S.g.done && S.h1.done && S.h2.done && S.h3.done && S.h5.done && S.h6.done;
-      if (NBG_ALL(done)) return true;
-    }
-    return series_terms<MASK, N + 1>(x2, S);
+    if constexpr (N < SER_TERMS_36) SerTerm<N + 1>::template add<MASK>(x2, t, s);
   }
-  return false;
-}
-// gfuncs for lanes that all have 2^-60 <= |gamma| < 1/2 and |beta|, sqb in
-// range; false when a series of some lane has not converged.
-template <int MASK> NBG_HD bool series_fast(double gamma, double beta, double sqb, SeriesOut& o) {
+};
+template <int MASK> NBG_HD SeriesOut series_fast(double gamma, double beta, double sqb) {
   const double x2 = (-nbg::sign(beta)) * (gamma * gamma);
-  SerState S;
-  auto start = [](double v, int bit) { return SerSum{v, 2.0 * v, 2.0 * v, (MASK & bit) == 0}; };
-  S.tg = 1.0; S.g = start(1.0, SER_G3);
-  S.t1 = 1.0; S.h1 = start(1.0, SER_H1);
-  S.t2 = 1.0; S.h2 = start(1.0, SER_H2);
-  S.t3 = 1.0 / 30.0; S.h3 = start(1.0 / 10.0, SER_H3);
-  S.t5 = 1.0 / 60.0; S.h5 = start(1.0 / 60.0, SER_H5);
-  S.t6 = 1.0 / 360.0; S.h6 = start(1.0 / 40.0, SER_H6);
-  if (!series_terms<MASK, 1>(x2, S)) return false;
-  const double bs = beta * sqb, b2 = beta * beta, x4 = x2 * x2;
-  if constexpr ((MASK & SER_G3) != 0) o.g3 = S.g.s * fdiv((-x2) * gamma, (6.0 * beta) * sqb);
-  if constexpr ((MASK & SER_H1) != 0) o.h1 = S.h1.s * fdiv(x4, 12.0 * b2);
-  if constexpr ((MASK & SER_H2) != 0) o.h2 = S.h2.s * fdiv((-x2) * gamma, (3.0 * beta) * sqb);
+  SeriesOut t = {1.0, 1.0, 1.0, 1.0 / 30.0, 1.0 / 60.0, 1.0 / 360.0};
+  SeriesOut s = {1.0, 1.0, 1.0, 1.0 / 10.0, 1.0 / 60.0, 1.0 / 40.0};
+  SerTerm<1>::template add<MASK>(x2, t, s);
+  SeriesOut o = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  const double b2 = beta * beta, x4 = x2 * x2;
+  if constexpr ((MASK & SER_G3) != 0) o.g3 = s.g3 * fdiv((-x2) * gamma, (6.0 * beta) * sqb);
+  if constexpr ((MASK & SER_H1) != 0) o.h1 = s.h1 * fdiv(x4, 12.0 * b2);
+  if constexpr ((MASK & SER_H2) != 0) o.h2 = s.h2 * fdiv((-x2) * gamma, (3.0 * beta) * sqb);
   if constexpr ((MASK & (SER_H3 | SER_H5)) != 0) {
-    const double q = fdiv((-x4) * gamma, bs);
-    if constexpr ((MASK & SER_H3) != 0) o.h3 = S.h3.s * q;
-    if constexpr ((MASK & SER_H5) != 0) o.h5 = S.h5.s * q;
+    const double q = fdiv((-x4) * gamma, beta * sqb);
+    o.h3 = s.h3 * q;
+    o.h5 = s.h5 * q;
   }
-  if constexpr ((MASK & SER_H6) != 0) o.h6 = S.h6.s * fdiv(-(x2 * x2 * x2), b2);
-  return true;
+  if constexpr ((MASK & SER_H6) != 0) o.h6 = s.h6 * fdiv(-(x2 * x2 * x2), b2);
+  return o;
 }
 
 // sc_pair on its polynomial paths, with one odd polynomial for sin and sinh:
 // Horner's sums of ksin are those of sinh_poly in -y^2 up to sign (the sign
 // alternates from one multiply-add to the next and rounding is symmetric), so
-// w = -y^2 on elliptic lanes and y^2 on the others serves both.  ANYE / ANYH:
-// some lane of the wave is elliptic / hyperbolic.
-NBG_HD void sc_fast(bool ell, bool anyE, bool anyH, double y, double* sx, double* cx) {
+// w = -y^2 on elliptic lanes and y^2 on the others serves both.  E / H: some
+// lane of the wave is elliptic / hyperbolic; each mix is one straight block,
+// so that its polynomial chains overlap.
+template <bool E, bool H> NBG_HD void sc_block(bool ell, double y, double* sx, double* cx) {
   const double z = y * y;
-  const double w = ell ? -z : z;
-  double q = fmac(w, F21, F19);
-  q = fmac(q, w, F17);
-  q = fmac(q, w, F15);
-  q = fmac(q, w, F13);
-  q = fmac(q, w, F11);
-  q = fmac(q, w, F9);
-  q = fmac(q, w, F7);
-  q = fmac(q, w, F5);
-  q = fmac(q, w, F3);
+  const double w = !H ? -z : (!E ? z : (ell ? -z : z));
   const double u = y * z;
-  double s = y - u * q, c = 0.0;
-  if (anyE) {
-    double p = fmac(z, F18, -F16);
-    p = fmac(z, p, F14);
-    p = fmac(z, p, -F12);
-    p = fmac(z, p, F10);
-    p = fmac(z, p, -F8);
-    p = fmac(z, p, F6);
-    p = fmac(z, p, -F4);
+  double q = fmac(w, F21, F19), p = 0.0, r = 0.0;
+  if (E) p = fmac(z, F18, -F16);
+  if (H) r = fmac(-y, F13, F12);
+  q = fmac(q, w, F17);
+  if (E) p = fmac(z, p, F14);
+  if (H) r = fmac(r, -y, F11);
+  q = fmac(q, w, F15);
+  if (E) p = fmac(z, p, -F12);
+  if (H) r = fmac(r, -y, F10);
+  q = fmac(q, w, F13);
+  if (E) p = fmac(z, p, F10);
+  if (H) r = fmac(r, -y, F9);
+  q = fmac(q, w, F11);
+  if (E) p = fmac(z, p, -F8);
+  if (H) r = fmac(r, -y, F8);
+  q = fmac(q, w, F9);
+  if (E) p = fmac(z, p, F6);
+  if (H) r = fmac(r, -y, F7);
+  q = fmac(q, w, F7);
+  if (E) p = fmac(z, p, -F4);
+  if (H) r = fmac(r, -y, F6);
+  q = fmac(q, w, F5);
+  if (H) r = fmac(r, -y, F5);
+  q = fmac(q, w, F3);
+  double s = 0.0, c = 0.0;
+  if (E) {
     const double hz = 0.5 * z;
     const double t = 1.0 - hz;
+    s = y - u * q;
     c = t + (((1.0 - t) - hz) - (z * z) * p);
   }
-  if (anyH) {
+  if (H) {
+    r = fmac(r, -y, F4);
+    r = fmac(r, -y, F3);
+    r = fmac(r, -y, F2);
+    r = fmad(r, -y, 1.0);
+    r = fmad(r, -y, 1.0);
     const double s2 = fmad(u, q, y);
-    const double c2 = exp_poly(-y) + s2;
-    s = ell ? s : s2;
-    c = ell ? c : c2;
+    const double c2 = r + s2;
+    s = E && ell ? s : s2;
+    c = E && ell ? c : c2;
   }
   *sx = s;
   *cx = c;
+}
+NBG_HD void sc_fast(bool ell, bool anyE, bool anyH, double y, double* sx, double* cx) {
+  if (anyE && anyH) sc_block<true, true>(ell, y, sx, cx);
+  else if (anyE) sc_block<true, false>(ell, y, sx, cx);
+  else sc_block<false, true>(ell, y, sx, cx);
 }
 
 NBG_HD bool in_range(double lo, double hi, double x) {
@@ -624,36 +618,44 @@ NBG_HD double cubic1_fast(double a, double b, double c, bool* ok) {
   double A = b;
   if (NBG_ANY(!three)) {
     const double rad = three ? 1.0 : R2 - Q3;
-    *ok = *ok && in_range(0x1p-400, 0x1p400, rad) && in_range(0x1p-200, 0x1p200, three ? 1.0 : R);
-    const double w = three ? 1.0 : nbg::fabsd(R) + fsqrt(rad);
-    const double k = (-nbg::sign(R)) * nbg::cbrt_core(w);
+    const double w = (three ? 0.0 : nbg::fabsd(R)) + fsqrt(rad);
+    *ok = in_range(0x1p-180, 0x1p180, rad) && in_range(0x1p-100, 0x1p90, w) && R != 0.0;
+    const double k = (-nbg::sign(R)) * nbg::cbrt_mid(w);
     A = three ? b : k;
   }
   const double d = fdiv(three ? -c : Q, A);
   return three ? d : (A + d) - a3;
 }
 
+// Range checks are gathered and voted on once at the end: a lane outside them
+// computes harmless nonsense until then (its Newton loop ends after 20
+// iterations at the latest; a NaN fails the last check).
 template <bool DF>
 NBG_HD bool jac_delxv_gamma_fast(const double* x0, const double* v0, double* delxv, double k, double h, KParams& P) {
   double y0[3];
   for (int j = 0; j < 3; ++j) y0[j] = DF ? x0[j] - h * v0[j] : x0[j];
-  const double rr = dot3(y0), vv = dot3(v0);
-  const double r0 = fsqrt(rr);
-  const double r0inv = fdiv(1.0, r0);
-  const double beta0 = (2.0 * k) * r0inv - vv;
+  double r0r, sqr;
+  const double r0 = fsqrt_recip(dot3(y0), &r0r);
+  const double r0inv = fdiv_by(1.0, r0, r0r);
+  const double beta0 = (2.0 * k) * r0inv - dot3(v0);
   const double signb = nbg::sign(beta0);
   const double ab = signb * beta0;
   const double beta0inv = fdiv(1.0, beta0);
-  const double sqb = fsqrt(ab);
+  const double sqb = fsqrt_recip(ab, &sqr);
   const double zeta = k - r0 * beta0;
   const double eta = dot3(y0, v0);
-  bool ok = in_range(0x1p-60, 0x1p60, r0) && in_range(0x1p-60, 0x1p60, beta0) && in_range(0x1p-60, 0x1p60, zeta) &&
-            in_range(0x1p-100, 0x1p60, k) && in_range(0x1p-60, 0x1p60, h) && nbg::fabsd(eta) <= 0x1p60;
   const double zinv = fdiv(6.0, zeta);
+  bool ok = true;
   double gamma = cubic1_fast(((0.5 * eta) * sqb) * zinv, ((r0 * signb) * beta0) * zinv,
                              ((((-h) * signb) * beta0) * sqb) * zinv, &ok);
-  if (!NBG_ALL(ok)) return false;
-  double gamma1 = 2.0 * gamma, gamma2 = 3.0 * gamma;
+  {  // r0, |beta|, |zeta|, |h| in [2^-60, 2^60), k in [2^-100, 2^60): as above, on the upper words
+    const int32_t lo = (1023 - 60) << 20, hi = (1023 + 60) << 20;
+    const int32_t a = hi_word(r0), b = hi_word(ab), c = hi_word(zeta), d = hi_word(h), e = hi_word(k);
+    ok = ok && k > 0.0 &&
+         ((a - lo) | (hi - a) | (b - lo) | (hi - b) | (c - lo) | (hi - c) | (d - lo) | (hi - d) |
+          (e - (lo - (40 << 20))) | (hi - e)) >= 0;
+  }
+  double gamma1 = 2.0 * gamma, gamma2;
   int iter = 0;
   const double c2 = (-2.0) * zeta;
   const double c3 = ((2.0 * eta) * signb) * sqb;
@@ -663,42 +665,46 @@ NBG_HD bool jac_delxv_gamma_fast(const double* x0, const double* v0, double* del
   const bool ell = beta0 > 0.0;
   const bool anyE = NBG_ANY(ell), anyH = NBG_ANY(!ell);
   // |gamma / 2| up to which sc_pair's polynomials apply without reduction
-  // (|y| 2/pi < 1/2, |y| log2 e < 1/2); the series below want |gamma| < 1/2
-  const double ymax = ell ? 0.75 : 0.34;
-  double sx = 0.0, cx = 0.0, used = gamma;
+  // (|y| 2/pi < 1/2, |y| log2 e < 1/2) and gamma stays below the series' 1/2;
+  // checked on the upper words, whose differences' signs gather in `off`.
+  // The quotient needs no check: its divisor is a sum of terms that the
+  // checks here and above keep within [2^-180, 2^190], and it ends the loop
+  // as a NaN where those cancel to zero.
+  const int32_t ylo = 0x3e400000;                        // 2^-27
+  const int32_t yhi = ell ? 0x3fe80000 : 0x3fd5c28f;     // 0.75, 0.34
+  int32_t off = 0;
+  double sx, cx, used;
   bool run = true;
+  gamma2 = 3.0 * gamma;
   do {
     const double xx = 0.5 * gamma;
-    ok = ok && in_range(0x1p-27, ymax, xx);
-    if (!NBG_ALL(ok)) return false;
-    used = gamma;
+    const int32_t hx = hi_word(xx);
+    off |= (hx - ylo) | (yhi - hx);
     sc_fast(ell, anyE, anyH, xx, &sx, &cx);
     const double ss = sx * sx;
     const double num = ((k * gamma + (c2 * sx) * cx) + c3 * ss) + c4;
     const double den = (c6 * ss + (c3 * sx) * cx) + c7;
-    ok = in_range(0x1p-200, 0x1p200, den);
     const double gn = gamma - fdiv(num, den);
-    if (run) {
-      gamma2 = gamma1;
-      gamma1 = gamma;
-      gamma = gn;
-      iter += 1;
-      run = !(gamma == gamma2 || gamma == gamma1) && iter < 20;
-    }
-  } while (NBG_ANY(run));
-  ok = ok && in_range(0x1p-27, 0x1.fffffep-2, gamma) && nbg::fabsd(gamma) <= 2.0 * ymax;
+    used = gamma;
+    // a lane that has stopped keeps its gamma (what it compares it with no
+    // longer matters)
+    gamma2 = gamma1;
+    gamma1 = gamma;
+    gamma = run ? gn : gamma;
+    iter += 1;
+    run = run && !(gamma == gamma2 || gamma == gamma1);
+  } while (NBG_ANY(run) && iter < 20);
+  ok = ok && off >= 0 && in_range(0x1p-26, 0x1.fffffep-2, gamma);
   if (!NBG_ALL(ok)) return false;
   // the last evaluation stands when every lane's gamma has repeated it
   if (!NBG_ALL(gamma == used)) sc_fast(ell, anyE, anyH, 0.5 * gamma, &sx, &cx);
-  const double g1bs = fdiv((2.0 * sx) * cx, sqb);
+  const double g1bs = fdiv_by((2.0 * sx) * cx, sqb, sqr);
   const double g2bs = ((2.0 * signb) * (sx * sx)) * beta0inv;
   const double g0bs = 1.0 - beta0 * g2bs;
   const double r = (r0 * g0bs + eta * g1bs) + k * g2bs;
-  ok = in_range(0x1p-100, 0x1p100, r);
   const double rinv = fdiv(1.0, r);
-  SeriesOut so = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  if (!series_fast<DF ? SER_G3 : (SER_G3 | SER_H1 | SER_H2)>(gamma, beta0, sqb, so)) return false;
-  if (!NBG_ALL(ok)) return false;
+  if (!NBG_ALL(in_range(0x1p-100, 0x1p100, r))) return false;
+  const SeriesOut so = series_fast<DF ? SER_G3 : (SER_G3 | SER_H1 | SER_H2)>(gamma, beta0, sqb);
   const double g3bs = so.g3, h1 = so.h1, h2 = so.h2;
   const double dfdt = (((-k) * g1bs) * rinv) * r0inv;
   double fm1, gmh, dgdtm1;
@@ -732,9 +738,8 @@ template <int MASK> NBG_HD_COLD SeriesOut gfuncs_general(double gamma, double be
   return gfuncs<MASK>(gamma, beta, sqb);
 }
 template <int MASK> NBG_HD SeriesOut gfuncs_fast(double gamma, double beta, double sqb) {
-  SeriesOut o = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   const bool ok = in_range(0x1p-60, 0x1.fffffep-2, gamma) && in_range(0x1p-60, 0x1p60, beta);
-  if (NBG_ALL(ok) && series_fast<MASK>(gamma, beta, sqb, o)) return o;
+  if (NBG_ALL(ok)) return series_fast<MASK>(gamma, beta, sqb);
   return gfuncs_general<MASK>(gamma, beta, sqb);
 }
 
