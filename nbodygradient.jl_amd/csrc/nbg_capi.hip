@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -49,6 +50,14 @@ extern "C" int nbg_coop_max_bodies();
 extern "C" hipError_t nbg_launch_group_duo(int cls, nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int grid,
                                            unsigned long long* units, hipStream_t stream);
 extern "C" int nbg_duo_pairs(int cls, int n);
+// two waves a workgroup, the state on one and the Jacobian on the other: one
+// system per workgroup, two, or few systems on the whole GPU
+extern "C" hipError_t nbg_launch_split(int cls, nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int64_t bound_job,
+                                       int grid, unsigned long long* units, unsigned long long* err, hipStream_t stream);
+extern "C" hipError_t nbg_launch_split_duo(nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int64_t bound_job, int grid,
+                                           unsigned long long* units, unsigned long long* err, hipStream_t stream);
+extern "C" hipError_t nbg_launch_split_wide(nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int64_t bound_job, int grid,
+                                            unsigned long long* units, unsigned long long* err, hipStream_t stream);
 
 namespace {
 
@@ -238,6 +247,17 @@ void group_layout(Layout& L) {
   }
 }
 
+// Whether a system may run on the two-wave launches: transit and plain runs
+// whose pairs are all Kepler pairs, none of them massless (such a pair reuses
+// the one before it, which keeps the sequential order).
+int split_ok(const nbg::SysDesc& d, const double* m) {
+  if ((d.mode != nbg::MODE_TRANSITS && d.mode != nbg::MODE_STEPS) || d.any_kick) return 0;
+  for (int i = 0; i < d.n - 1; ++i)
+    for (int j = i + 1; j < d.n; ++j)
+      if (nbg::NBG_GNEWT * (m[i] + m[j]) == 0.0) return 0;
+  return 1;
+}
+
 bool mass_rows_ok(int n, const double* J, const double* JE) {
   const int s = 7 * n;
   for (int b = 0; b < n; ++b) {
@@ -359,6 +379,26 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
   NBG_HIP(hipMemset(S.units.p, 0, sizeof(unsigned long long) * (13 * G + 14)));
   const nbg::SysBufs B = bufs ? *bufs : bufs_of(S);
   const int ns = (int)ctx->streams.size();
+  // Launch classes whose systems all qualify run on two waves a system, or a
+  // pair of systems (nbg_split.h).  A batch that leaves a compute unit to each
+  // system takes the wide launch, which serves every class.
+  std::vector<char> split(G, 1), paired(G, 0);
+  bool wide = (int)L.desc.size() <= ctx->cu_count;
+  for (size_t g = 0; g < G; ++g) {
+    for (int k = 0; k < L.gcnt[g]; ++k)
+      if (!L.desc[L.order[L.goff[g] + k]].split) split[g] = 0;
+    if (L.pairs) {
+      const int* us = L.ustart.data() + L.uoff[g];
+      for (int u = 0; us[u] < L.gcnt[g]; ++u)
+        if (us[u + 1] - us[u] == 2) paired[g] = 1;
+    }
+    if (paired[g] && L.gn[g] != 9) split[g] = 0;  // pairs of up to 9 bodies only
+    if (!split[g] || paired[g]) wide = false;
+  }
+  bool any_split = false;
+  const int64_t split_bound = ctx->coop_polls > 0 ? ctx->coop_polls : (int64_t)1 << 24;
+  const int64_t split_job = ctx->coop_polls > 0 ? ctx->coop_polls : (int64_t)1 << 40;
+  unsigned long long* const wait_err = S.units.p + 13 * G + 13;
   NBG_HIP(hipEventRecord(ctx->ev0, 0));
   for (int s = 0; s < ns; ++s) NBG_HIP(hipStreamWaitEvent(ctx->streams[s], ctx->ev0, 0));
   // One launch per launch class (groups are in decreasing class order).  A
@@ -413,6 +453,7 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
     const int cap = std::min(ctx->coop_max, ctx->cu_count / 2);
     for (size_t g = 0; g < G; ++g) {
       if (L.gn[g] > nbg_coop_max_bodies()) continue;
+      if (ctx->coop_mode == 1 && split[g]) continue;  // every system has its second wave
       while (K < cap && kg[g] < L.gcnt[g]) {
         const int i = L.order[L.goff[g] + kg[g]];
         if (L.desc[i].mode != nbg::MODE_TRANSITS) break;
@@ -468,10 +509,13 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
   std::iota(gord.begin(), gord.end(), 0);
   std::vector<double> load(ns, 0.0);
   for (size_t g : gord) {
+    if (wide && g > 0) break;  // the first launch takes every class
     if (g == 1 && chunk == 0) std::this_thread::sleep_for(std::chrono::microseconds(2000));
     nbg::GroupList gl{};
     gl.rowupd = ctx->row_update;
-    for (size_t h = g; h < G; ++h) {  // own class, then the smaller ones
+    // own class, then the smaller ones whose launch takes systems the same way
+    for (size_t h = g; h < G; ++h) {
+      if (h > g && !wide && (split[h] != split[g] || (split[g] && (paired[h] || paired[g])))) continue;
       const int skip = kg[h];  // the cooperative systems
       gl.nsys[gl.ng] = L.gcnt[h] - skip;
       gl.descs[gl.ng] = S.desc.p + L.goff[h] + skip;
@@ -487,7 +531,9 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
       }
       gl.ng += 1;
     }
-    const int grid = grids[g];
+    const int grid = wide ? std::max(1, std::min({(int)L.desc.size(), ctx->cu_count, ctx->grid_cap > 0 ? ctx->grid_cap : INT_MAX}))
+                          : grids[g];
+    if (wide && group_grid) (*group_grid)[g] = grid;
     if (K > 0) load[0] += 1e30;  // the cooperative launch holds stream 0
     const int si = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     load[si] += L.gcost[g] / grid;
@@ -496,7 +542,13 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
     int64_t work = 0;  // systems this launch can take (none left when all went to cooperative workgroups)
     for (int e = 0; e < gl.ng; ++e) work += gl.nsys[e];
     if (timed) NBG_HIP(hipEventRecord(ctx->gev[2 * g], st));
-    if (work > 0)
+    if (work > 0 && split[g]) {
+      any_split = true;
+      unsigned long long* un = S.units.p + 13 * g;
+      NBG_HIP(wide ? nbg_launch_split_wide(gl, B, chunk, split_bound, split_job, grid, un, wait_err, st)
+              : paired[g] ? nbg_launch_split_duo(gl, B, chunk, split_bound, split_job, grid, un, wait_err, st)
+                          : nbg_launch_split(L.gn[g], gl, B, chunk, split_bound, split_job, grid, un, wait_err, st));
+    } else if (work > 0)
       NBG_HIP(L.pairs ? nbg_launch_group_duo(L.gn[g], gl, B, chunk, grid, S.units.p + 13 * g, st)
                       : nbg_launch_group(L.gn[g], gl, B, chunk, grid, S.units.p + 13 * g, st));
     if (timed) NBG_HIP(hipEventRecord(ctx->gev[2 * g + 1], st));
@@ -518,13 +570,14 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
   }
   if (group_ms) {
     group_ms->assign(G, 0.0f);
-    for (size_t g = 0; g < G; ++g) NBG_HIP(hipEventElapsedTime(&(*group_ms)[g], ctx->gev[2 * g], ctx->gev[2 * g + 1]));
+    for (size_t g = 0; g < (wide ? 1 : G); ++g)
+      NBG_HIP(hipEventElapsedTime(&(*group_ms)[g], ctx->gev[2 * g], ctx->gev[2 * g + 1]));
   }
-  if (K > 0) {
+  if (K > 0 || any_split) {
     unsigned long long werr = 0;
-    NBG_HIP(hipMemcpy(&werr, S.units.p + 13 * G + 13, sizeof(werr), hipMemcpyDeviceToHost));
+    NBG_HIP(hipMemcpy(&werr, wait_err, sizeof(werr), hipMemcpyDeviceToHost));
     if (werr) {
-      ctx->err = "cooperative workgroup: a wait between its two waves timed out";
+      ctx->err = "two-wave workgroup: a wait between its two waves timed out";
       return -2;
     }
   }
@@ -601,6 +654,7 @@ int run_single(nbg_ctx* ctx, nbg::SysDesc d, double* x, double* v, double* xe, d
                const uint8_t* pair, double* J, double* JE, double* dqdt, const double* jinit, double* t,
                double* tt, double* dtdq0, double* dtdel, int64_t* count, const TrajOut* traj = nullptr) {
   Layout L;
+  d.split = split_ok(d, m);
   L.desc.push_back(d);
   finalize_layout(L);
   const nbg::SysDesc& D = L.desc[0];
@@ -1127,6 +1181,7 @@ static int batch_build(nbg_ctx* ctx, int32_t nsys, const int32_t* n, const doubl
     d.any_kick = pair ? any_kick(n[s], pair + op[s]) : 0;
     d.nsteps = std::llabs(jround(tmax[s] / h[s]));
     d.ntt = ntt[s]; d.h = h[s] * check_step(t0[s], tmax[s] + t0[s]); d.hstep = h[s]; d.hlast = 0.0; d.t0 = t0[s];
+    d.split = split_ok(d, m + ob[s]);
     b->steps_main += d.nsteps;
   }
   finalize_layout(b->L);
@@ -1936,6 +1991,7 @@ int nbg_server_submit(nbg_server* sv, int32_t n, double h, double tmax, double t
   d.any_kick = pair ? any_kick(n, pair) : 0;
   d.nsteps = std::llabs(jround(tmax / h));
   d.ntt = ntt; d.h = h * check_step(t0, tmax + t0); d.hstep = h; d.hlast = 0.0; d.t0 = t0;
+  d.split = split_ok(d, m);
   r->lay = req_layout(n, ntbv, ntt);
   pack_system(d, x, v, nullptr, nullptr, m, pair, nullptr, nullptr, nullptr, jac_init, t0, nullptr, nullptr, r->init);
   if (Arena::round(r->lay.bytes) > sv->arena.cap) {

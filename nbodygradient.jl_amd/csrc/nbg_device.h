@@ -122,13 +122,9 @@ __device__ __forceinline__ gdouble* uniform_global(const double* p) {
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
   return (gdouble*)((((uint64_t)hi) << 32) | lo);
 }
-template <int NB, bool G> __device__ __forceinline__ auto jj(Smem<NB, G>& S) {
-  if constexpr (G) return uniform_global(S.jg);
-  else return static_cast<double*>(S.JJ);
-}
-template <int NB, bool G> __device__ __forceinline__ auto jj(const Smem<NB, G>& S) {
-  if constexpr (G) return (const gdouble*)uniform_global(S.jg);
-  else return static_cast<const double*>(S.JJ);
+template <int NB, class R> __device__ __forceinline__ auto jj(R& S) {
+  if constexpr (R::JG) return uniform_global(S.jg);
+  else return &S.JJ[0];
 }
 
 // Synchronisation of the lanes of one wave (a system's lanes are one wave):
@@ -182,17 +178,80 @@ __device__ __forceinline__ PairSlot* slot_at(uint32_t off) { return (PairSlot*)(
 
 // The drift by the general formulas: waves with a lane outside the common
 // case of nbg_pair.h (a long step, a nearly parabolic or radial orbit).
-static __device__ __attribute__((noinline)) void pair_drift_general(uint32_t slot, double gm, double hh, bool drift_first) {
+struct DriftOut {
+  KParams P;
+  double d[6];
+};
+static __device__ __attribute__((noinline)) void pair_drift_general(double x, double y, double z, double vx, double vy,
+                                                                    double vz, double gm, double hh, bool drift_first,
+                                                                    DriftOut* out) {
   drift_first = __builtin_amdgcn_readfirstlane((int)drift_first) != 0;  // the same for the whole sweep
-  PairSlot* sl = slot_at(slot);
-  double x0[3], v0[3], delxv[6];
+  const double x0[3] = {x, y, z}, v0[3] = {vx, vy, vz};
+  double d[6];
+  out->P = jac_delxv_gamma(x0, v0, d, gm, hh, drift_first);
+  for (int k = 0; k < 6; ++k) out->d[k] = d[k];
+}
+
+// kepler_driftij_gamma! (ahl21.jl:706-733) of pair (i, j) by one lane: the
+// Kepler drift and the Kahan update of the two bodies' state in the record
+// whose x is given (then v, xerror, verror and m).  x0, v0, P, d and mijinv
+// are what the pair's Jacobian needs; false for a massless pair.
+template <bool DF>
+__device__ __forceinline__ bool pair_state(double* x, int n3, int i, int j, double hh, double (&x0)[3], double (&v0)[3],
+                                           KParams& P, double (&d)[6], double& m_i, double& m_j, double& mijinv) {
+  double* v = x + n3;
+  double xi[3], xj[3], vi[3], vj[3], exi[3], exj[3], evi[3], evj[3];
+  // every LDS operand is read into registers before anything is written
+  // back: the compiler cannot tell the arrays apart, so interleaved reads and
+  // writes would each wait for the previous write
   for (int k = 0; k < 3; ++k) {
-    x0[k] = sl->x0[k];
-    v0[k] = sl->v0[k];
+    xi[k] = x[3 * i + k];
+    xj[k] = x[3 * j + k];
+    vi[k] = v[3 * i + k];
+    vj[k] = v[3 * j + k];
   }
-  const KParams P = jac_delxv_gamma(x0, v0, delxv, gm, hh, drift_first);
-  sl->P = P;
-  for (int k = 0; k < 6; ++k) sl->delxv[k] = delxv[k];
+  m_i = x[4 * n3 + i];
+  m_j = x[4 * n3 + j];
+  for (int k = 0; k < 3; ++k) {
+    exi[k] = x[2 * n3 + 3 * i + k];
+    exj[k] = x[2 * n3 + 3 * j + k];
+    evi[k] = x[3 * n3 + 3 * i + k];
+    evj[k] = x[3 * n3 + 3 * j + k];
+  }
+  for (int k = 0; k < 3; ++k) {
+    x0[k] = xi[k] - xj[k];
+    v0[k] = vi[k] - vj[k];
+  }
+  const double gm = NBG_GNEWT * (m_i + m_j);
+  if (gm == 0.0) return false;
+  if (jac_delxv_gamma_fast<DF>(x0, v0, d, gm, hh, P)) {
+    mijinv = fdiv(1.0, m_i + m_j);  // gm is in the plain range
+  } else {
+    DriftOut o;
+    pair_drift_general(x0[0], x0[1], x0[2], v0[0], v0[1], v0[2], gm, hh, DF, &o);
+    P = o.P;
+    for (int k = 0; k < 6; ++k) d[k] = o.d[k];
+    mijinv = 1.0 / (m_i + m_j);
+  }
+  const double mi = m_i * mijinv;
+  const double mj = m_j * mijinv;
+  for (int k = 0; k < 3; ++k) {
+    kahan(xi[k], exi[k], mj * d[k]);
+    kahan(xj[k], exj[k], (-mi) * d[k]);
+    kahan(vi[k], evi[k], mj * d[3 + k]);
+    kahan(vj[k], evj[k], (-mi) * d[3 + k]);
+  }
+  for (int k = 0; k < 3; ++k) {
+    x[3 * i + k] = xi[k];
+    x[3 * j + k] = xj[k];
+    v[3 * i + k] = vi[k];
+    v[3 * j + k] = vj[k];
+    x[2 * n3 + 3 * i + k] = exi[k];
+    x[2 * n3 + 3 * j + k] = exj[k];
+    x[3 * n3 + 3 * i + k] = evi[k];
+    x[3 * n3 + 3 * j + k] = evj[k];
+  }
+  return true;
 }
 
 // Phase A of a sweep: the Kepler drifts and Kahan state updates
@@ -236,76 +295,24 @@ template <bool DF> static __device__ __attribute__((noinline)) void drift_levels
     const int w1 = L + 1 < levels ? (int)lw[L + 1] : 0;
     if (lane < (two ? 2 * w : w)) {
       const bool second = lane >= w;
-      double* x = lds_at<double>(second ? R.x1 : R.x0);
-      double* v = x + n3;
       PairSlot* sl = slot_at((second ? R.slot1 : R.slot0) + (uint32_t)(q * sizeof(PairSlot)));
-      const double hh = second ? R.hh1 : R.hh0;
       const int i = ij & 0xff, j = ij >> 8;
-      // every LDS operand is read into registers before anything is written
-      // back: the compiler cannot tell the slot from the state arrays, so
-      // interleaved reads and writes would each wait for the previous write
-      double xi[3], xj[3], vi[3], vj[3], exi[3], exj[3], evi[3], evj[3], x0[3], v0[3], d[6];
-      for (int k = 0; k < 3; ++k) {
-        xi[k] = x[3 * i + k];
-        xj[k] = x[3 * j + k];
-        vi[k] = v[3 * i + k];
-        vj[k] = v[3 * j + k];
-      }
-      const double m_i = x[4 * n3 + i], m_j = x[4 * n3 + j];
-      for (int k = 0; k < 3; ++k) {
-        exi[k] = x[2 * n3 + 3 * i + k];
-        exj[k] = x[2 * n3 + 3 * j + k];
-        evi[k] = x[3 * n3 + 3 * i + k];
-        evj[k] = x[3 * n3 + 3 * j + k];
-      }
-      for (int k = 0; k < 3; ++k) {
-        x0[k] = xi[k] - xj[k];
-        v0[k] = vi[k] - vj[k];
-      }
-      const double gm = NBG_GNEWT * (m_i + m_j);
-      if (gm != 0.0) {
-        KParams P;
-        double mijinv;
-        if (jac_delxv_gamma_fast<DF>(x0, v0, d, gm, hh, P)) {
-          mijinv = fdiv(1.0, m_i + m_j);  // gm is in the plain range
-          if (store) {
-            sl->P = P;
-            for (int k = 0; k < 3; ++k) {
-              sl->x0[k] = x0[k];
-              sl->v0[k] = v0[k];
-            }
-            for (int k = 0; k < 6; ++k) sl->delxv[k] = d[k];
-          }
-        } else {
+      double x0[3], v0[3], d[6], m_i, m_j, mijinv;
+      KParams P;
+      const bool valid = pair_state<DF>(lds_at<double>(second ? R.x1 : R.x0), n3, i, j, second ? R.hh1 : R.hh0, x0, v0, P,
+                                        d, m_i, m_j, mijinv);
+      if (store) {
+        if (valid) {
+          sl->P = P;
           for (int k = 0; k < 3; ++k) {
             sl->x0[k] = x0[k];
             sl->v0[k] = v0[k];
           }
-          pair_drift_general(lds_slot(sl), gm, hh, DF);
-          for (int k = 0; k < 6; ++k) d[k] = sl->delxv[k];
-          mijinv = 1.0 / (m_i + m_j);
+          for (int k = 0; k < 6; ++k) sl->delxv[k] = d[k];
+          sl->mi = m_i * mijinv; sl->mj = m_j * mijinv; sl->mijinv = mijinv; sl->m_i = m_i; sl->m_j = m_j;
         }
-        const double mi = m_i * mijinv;
-        const double mj = m_j * mijinv;
-        for (int k = 0; k < 3; ++k) {
-          kahan(xi[k], exi[k], mj * d[k]);
-          kahan(xj[k], exj[k], (-mi) * d[k]);
-          kahan(vi[k], evi[k], mj * d[3 + k]);
-          kahan(vj[k], evj[k], (-mi) * d[3 + k]);
-        }
-        for (int k = 0; k < 3; ++k) {
-          x[3 * i + k] = xi[k];
-          x[3 * j + k] = xj[k];
-          v[3 * i + k] = vi[k];
-          v[3 * j + k] = vj[k];
-          x[2 * n3 + 3 * i + k] = exi[k];
-          x[2 * n3 + 3 * j + k] = exj[k];
-          x[3 * n3 + 3 * i + k] = evi[k];
-          x[3 * n3 + 3 * j + k] = evj[k];
-        }
-        if (store) { sl->mi = mi; sl->mj = mj; sl->mijinv = mijinv; sl->m_i = m_i; sl->m_j = m_j; }
+        sl->valid = valid; sl->i = i; sl->j = j;
       }
-      if (store) { sl->valid = (gm != 0.0); sl->i = i; sl->j = j; }
     }
     q0 += w;
     w = __builtin_amdgcn_readfirstlane(w1);
@@ -424,10 +431,15 @@ template <int NB, bool G> __device__ void kick_build(Smem<NB, G>& S, Swork<NB>& 
 // col = lane) or two on its halves (STEP = 32, phi_build2).  The lane of
 // body d's coordinate p writes the acceleration a[p, d]; col 0 writes the
 // other uniform values (v, dqdt_phi).  FACT: jac_phi in the factored form.
-template <int NB, bool G, int STEP, bool FACT = false>
-__device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>& S, Swork<NB>& W, double h, bool anyKick,
-                                                                     bool needQ, int col) {
+// STATE: the velocities are updated too (a record that carries them).
+template <int NB, bool G, int STEP, bool FACT = false, bool STATE = true, class R, class WK>
+__device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W, double h, bool anyKick, bool needQ,
+                                                                     int col) {
   constexpr int N3 = 3 * NB, N4 = 4 * NB;
+  auto kicked = [](const R& rec, bool any, int i, int j) {
+    if constexpr (STATE) return any && rec.pair[i + NB * j];
+    else return false;
+  };
   const bool own = col < N4;
   int myd = -1, myp = -1;
   if (own) col_dp<NB>(col, myd, myp);
@@ -445,7 +457,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
   // order; looping over the partner c in increasing order therefore repeats
   // every accumulation in the reference's order.  a and dadq start at zero
   // (ahl21.jl:559-563); jac_phi keeps phic!'s terms.
-  constexpr int NP = Swork<NB>::NP, PQ = Swork<NB>::PQ;
+  constexpr int NP = WK::NP, PQ = WK::PQ;
   double* pq = W.f.pq;
   auto pidx = [](int i, int j) { return i * (2 * NB - i - 1) / 2 + (j - i - 1); };
   const double coeff = (((2.0 * (h * h * h)) / 96.0) * 2.0) * NBG_GNEWT;
@@ -488,7 +500,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
       const int i = b < myd ? b : myd, j = b < myd ? myd : b;
       const bool bi = (b == i);
       double t[3] = {0.0, 0.0, 0.0};
-      if (!(anyKick && S.pair[i + NB * j])) {
+      if (!kicked(S, anyKick, i, j)) {
         const double* o = pq + pidx(i, j) * PQ;
         const double m = S.m[myd];  // b's partner's mass
         const double f2m = o[0] * m;
@@ -510,7 +522,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
     for (int c = 0; c < NB; ++c) {
       if (c == myd) continue;
       const int i = c < myd ? c : myd, j = c < myd ? myd : c;
-      if (anyKick && S.pair[i + NB * j]) continue;
+      if (kicked(S, anyKick, i, j)) continue;
       const double* o = pq + pidx(i, j) * PQ;
       const bool bi = (myd == i);
       const double m = S.m[c];  // the partner's mass
@@ -583,8 +595,11 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
     for (int i = 0; i < NB - 1; ++i) {
       double vi[3], vie[3], qi[3], pi[3], xi[3], Di[3];
       for (int k = 0; k < 3; ++k) {
-        vi[k] = S.v[3 * i + k];
-        vie[k] = S.ve[3 * i + k];
+        vi[k] = vie[k] = 0.0;
+        if constexpr (STATE) {
+          vi[k] = S.v[3 * i + k];
+          vie[k] = S.ve[3 * i + k];
+        }
         qi[k] = needQ ? S.dqdt_phi[7 * i + 3 + k] : 0.0;
         pi[k] = own ? PHI[(3 * i + k) * N4 + col] : 0.0;
         xi[k] = S.x[3 * i + k];
@@ -594,15 +609,18 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
       const bool di = myd == i;
 #pragma unroll 1
       for (int j = i + 1; j < NB; ++j, ++p) {
-        if (anyKick && S.pair[i + NB * j]) continue;
+        if (kicked(S, anyKick, i, j)) continue;
         const double* o = pq + p * PQ;
         const double mj = S.m[j];
         double rij[3], Dj[3], vj[3], vje[3], qj[3], pj[3];
         for (int k = 0; k < 3; ++k) {
           rij[k] = xi[k] - S.x[3 * j + k];
           Dj[k] = own ? D[(3 * j + k) * N4 + col] : 0.0;
-          vj[k] = S.v[3 * j + k];
-          vje[k] = S.ve[3 * j + k];
+          vj[k] = vje[k] = 0.0;
+          if constexpr (STATE) {
+            vj[k] = S.v[3 * j + k];
+            vje[k] = S.ve[3 * j + k];
+          }
           qj[k] = needQ ? S.dqdt_phi[7 * j + 3 + k] : 0.0;
           pj[k] = own ? PHI[(3 * j + k) * N4 + col] : 0.0;
         }
@@ -615,8 +633,10 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
           const double fac = o[k];
-          kahan(vi[k], vie[k], mj * fac);
-          kahan(vj[k], vje[k], -(mi * fac));
+          if constexpr (STATE) {
+            kahan(vi[k], vie[k], mj * fac);
+            kahan(vj[k], vje[k], -(mi * fac));
+          }
           if (needQ) {
             qi[k] += (q3h * mj) * fac;
             qj[k] += -((q3h * mi) * fac);
@@ -631,8 +651,10 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
         for (int k = 0; k < 3; ++k) {
           if (own) PHI[(3 * j + k) * N4 + col] = pj[k];
           if (col == 0) {
-            S.v[3 * j + k] = vj[k];
-            S.ve[3 * j + k] = vje[k];
+            if constexpr (STATE) {
+              S.v[3 * j + k] = vj[k];
+              S.ve[3 * j + k] = vje[k];
+            }
             if (needQ) S.dqdt_phi[7 * j + 3 + k] = qj[k];
           }
         }
@@ -640,8 +662,10 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
       for (int k = 0; k < 3; ++k) {
         if (own) PHI[(3 * i + k) * N4 + col] = pi[k];
         if (col == 0) {
-          S.v[3 * i + k] = vi[k];
-          S.ve[3 * i + k] = vie[k];
+          if constexpr (STATE) {
+            S.v[3 * i + k] = vi[k];
+            S.ve[3 * i + k] = vie[k];
+          }
           if (needQ) S.dqdt_phi[7 * i + 3 + k] = qi[k];
         }
       }
@@ -651,8 +675,11 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
   for (int b = 0; b < NB; ++b) {
     double vb[3], veb[3], qb[3], pb[3];
     for (int k = 0; k < 3; ++k) {
-      vb[k] = S.v[3 * b + k];
-      veb[k] = S.ve[3 * b + k];
+      vb[k] = veb[k] = 0.0;
+      if constexpr (STATE) {
+        vb[k] = S.v[3 * b + k];
+        veb[k] = S.ve[3 * b + k];
+      }
       qb[k] = needQ ? S.dqdt_phi[7 * b + 3 + k] : 0.0;
       pb[k] = (anyKick && own) ? PHI[(3 * b + k) * N4 + col] : 0.0;
     }
@@ -660,7 +687,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
     for (int c = 0; c < NB; ++c) {
       if (c == b) continue;
       const int i = c < b ? c : b, j = c < b ? b : c;
-      if (anyKick && S.pair[i + NB * j]) continue;
+      if (kicked(S, anyKick, i, j)) continue;
       const double* o = pq + pidx(i, j) * PQ;
       double rij[3], Di[3], Dj[3];
       for (int k = 0; k < 3; ++k) {
@@ -682,7 +709,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
       for (int k = 0; k < 3; ++k) {
         const double fac = o[k], f5 = fac * o[3], fm = o[4 + k], fr = o[7 + k], ff = o[10] * rij[k];
         const double mf = m * fac;
-        kahan(vb[k], veb[k], bi ? mf : -mf);
+        if constexpr (STATE) kahan(vb[k], veb[k], bi ? mf : -mf);
         if (needQ) {
           const double qm = (q3h * m) * fac;
           qb[k] += bi ? qm : -qm;
@@ -706,8 +733,10 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>
       for (int k = 0; k < 3; ++k) PHI[(3 * b + k) * N4 + col] = pb[k];
     if (col == 0)
       for (int k = 0; k < 3; ++k) {
-        S.v[3 * b + k] = vb[k];
-        S.ve[3 * b + k] = veb[k];
+        if constexpr (STATE) {
+          S.v[3 * b + k] = vb[k];
+          S.ve[3 * b + k] = veb[k];
+        }
         if (needQ) S.dqdt_phi[7 * b + 3 + k] = qb[k];
       }
   }
@@ -871,7 +900,7 @@ __device__ void phi_build(Smem<NB, G>& S, Swork<NB>& W, double h, bool anyKick, 
 // Jacobian column kernels (lane owns column c).
 // ---------------------------------------------------------------------------
 // Position rows of column c (pre-update), the operand of K*J and Phi*J.
-template <int NB, bool G> __device__ inline void load_pos(const Smem<NB, G>& S, int c, double* P) {
+template <int NB, class R> __device__ inline void load_pos(const R& S, int c, double* P) {
   const auto J_ = jj<NB>(S);
   constexpr int N7 = 7 * NB;
 #pragma unroll
@@ -883,7 +912,7 @@ template <int NB, bool G> __device__ inline void load_pos(const Smem<NB, G>& S, 
 // J[velocity rows, c] += (B * J)[velocity rows, c] with Kahan compensation,
 // B = K or Phi (3n x 4n block); then the zero-addend Kahan pass over the
 // position rows that comp_sum_matrix! applies to the rest of the matrix.
-template <int NB, bool G> __device__ inline void vel_product_add(Smem<NB, G>& S, const double* B, int c, const double* P) {
+template <int NB, class R> __device__ inline void vel_product_add(R& S, const double* B, int c, const double* P) {
   const auto J_ = jj<NB>(S);
   constexpr int N3 = 3 * NB, N4 = 4 * NB, N7 = 7 * NB;
 #pragma unroll 1
@@ -903,7 +932,7 @@ template <int NB, bool G> __device__ inline void vel_product_add(Smem<NB, G>& S,
   }
 }
 
-template <int NB, bool G> __device__ inline void zero_add_rows(Smem<NB, G>& S, int c, bool pos, bool vel) {
+template <int NB, class R> __device__ inline void zero_add_rows(R& S, int c, bool pos, bool vel) {
   const auto J_ = jj<NB>(S);
   constexpr int N7 = 7 * NB;
 #pragma unroll 1
@@ -921,7 +950,7 @@ template <int NB, bool G> __device__ inline void zero_add_rows(Smem<NB, G>& S, i
 }
 
 // drift_grad! Jacobian part (ahl21.jl:326-328)
-template <int NB, bool G> __device__ inline void drift_cols(Smem<NB, G>& S, int c, double hh) {
+template <int NB, class R> __device__ inline void drift_cols(R& S, int c, double hh) {
   const auto J_ = jj<NB>(S);
   constexpr int N7 = 7 * NB;
 #pragma unroll 1
@@ -940,8 +969,8 @@ template <int NB, bool G> __device__ inline void drift_cols(Smem<NB, G>& S, int 
 // running sum starts at +0 and can never become -0, so the sign of a zero
 // coefficient cannot change it), and the mass columns 6 and 13 take their
 // coefficients from the slot, where pair_jacobian stored them.
-template <int NB, bool G, bool FACT = false>
-__device__ inline void pair_cols(Smem<NB, G>& S, const PairSlot& sl, int i, int j, int c) {
+template <int NB, bool G, bool FACT = false, class R, class SL>
+__device__ inline void pair_cols(R& S, const SL& sl, int i, int j, int c) {
   const auto J_ = jj<NB>(S);
   constexpr int N7 = 7 * NB;
   const int ri = 6 * i, rj = 6 * j;
@@ -1183,22 +1212,34 @@ __device__ __attribute__((always_inline)) inline void sweep2(Smem<NB, G>& S0, Sm
 // every flag combination (so grad and no-grad runs agree bit for bit, as the
 // reference's no-grad map ahl21_no_grad.jl:6-18 does).
 // ---------------------------------------------------------------------------
+// The state's drift over h2: entries are independent.
+template <int NB, int STEP, class R> __device__ inline void drift_state(R& S, double h2, int col) {
+  for (int q = col; q < 3 * NB; q += STEP) {
+    double xq = S.x[q], eq = S.xe[q];
+    kahan(xq, eq, h2 * S.v[q]);
+    S.x[q] = xq;
+    S.xe[q] = eq;
+  }
+}
+
 // The stages of one step between the pair sweeps: before the forward sweep
 // (kickfast! and the first drift), between the sweeps (phic!/phisalpha!),
 // after the backward sweep (the second drift and kickfast!).  The
 // zero-addend compensated passes of comp_sum_matrix! over the rows an
 // operation leaves unchanged (zero_add_rows) re-normalise pairs that their
 // last update already normalised; the factored form (FACT) leaves them out.
-template <int NB, bool G, int STEP = WAVE, bool FACT = false>
-__device__ __attribute__((always_inline)) inline void step_pre(Smem<NB, G>& S, Swork<NB>& W, double h, bool needJ, bool needQ, bool anyKick, int col) {
+template <int NB, bool G, int STEP = WAVE, bool FACT = false, bool STATE = true, class R, class WK>
+__device__ __attribute__((always_inline)) inline void step_pre(R& S, WK& W, double h, bool needJ, bool needQ, bool anyKick, int col) {
   constexpr int N3 = 3 * NB, N4 = 4 * NB, N7 = 7 * NB;
   const double h2 = 0.5 * h;
   const double h6 = h / 6.0;
   // zero_out!(d); fill!(s.dqdt, 0)
   if (col < 14) S.dqij[col] = 0.0;
-  if (S.seq)  // jac_ij = 0 at the start of the step (zero_out!, ahl21.jl:8)
-    for (int w = col; w < (int)(sizeof(PairSlot) / sizeof(double)); w += STEP)
-      reinterpret_cast<double*>(&S.jlast)[w] = 0.0;
+  if constexpr (STATE) {
+    if (S.seq)  // jac_ij = 0 at the start of the step (zero_out!, ahl21.jl:8)
+      for (int w = col; w < (int)(sizeof(PairSlot) / sizeof(double)); w += STEP)
+        reinterpret_cast<double*>(&S.jlast)[w] = 0.0;
+  }
   if (needQ)
     for (int r = col; r < N7; r += STEP) {
       S.dqdt[r] = 0.0;
@@ -1207,7 +1248,7 @@ __device__ __attribute__((always_inline)) inline void step_pre(Smem<NB, G>& S, S
     }
   wsync();
   // ---- kickfast!(s, d, h/6)
-  if constexpr (STEP == WAVE) {  // kicked pairs: whole-wave form only
+  if constexpr (STEP == WAVE && STATE) {  // kicked pairs: whole-wave form only
     if (anyKick) kick_build<NB>(S, W, h6, needQ, col);
   }
   wsync();
@@ -1241,12 +1282,7 @@ __device__ __attribute__((always_inline)) inline void step_pre(Smem<NB, G>& S, S
       if (anyKick) vel_product_add<NB>(S, W.f.dadq, c, P);
     }
   // ---- drift of the state (drift_grad! / drift!): entries are independent
-  for (int q = col; q < N3; q += STEP) {
-    double xq = S.x[q], eq = S.xe[q];
-    kahan(xq, eq, h2 * S.v[q]);
-    S.x[q] = xq;
-    S.xe[q] = eq;
-  }
+  if constexpr (STATE) drift_state<NB, STEP>(S, h2, col);
   wsync();
   if (needQ) {
     for (int q = col; q < N3; q += STEP) {
@@ -1257,8 +1293,8 @@ __device__ __attribute__((always_inline)) inline void step_pre(Smem<NB, G>& S, S
   wsync();
 }
 
-template <int NB, bool G, int STEP = WAVE, bool FACT = false>
-__device__ __attribute__((always_inline)) inline void step_mid_rest(Smem<NB, G>& S, Swork<NB>& W, bool needJ, bool needQ,
+template <int NB, bool G, int STEP = WAVE, bool FACT = false, class R, class WK>
+__device__ __attribute__((always_inline)) inline void step_mid_rest(R& S, WK& W, bool needJ, bool needQ,
                                                                     int col);
 
 template <int NB, bool G, bool FACT = false>
@@ -1271,8 +1307,8 @@ __device__ __attribute__((always_inline)) inline void step_mid(Smem<NB, G>& S, S
 
 // The rest of the stage between the sweeps, once jac_phi is built:
 // J_vel += jac_phi * J_pos, and dq/dt.
-template <int NB, bool G, int STEP, bool FACT>
-__device__ __attribute__((always_inline)) inline void step_mid_rest(Smem<NB, G>& S, Swork<NB>& W, bool needJ, bool needQ,
+template <int NB, bool G, int STEP, bool FACT, class R, class WK>
+__device__ __attribute__((always_inline)) inline void step_mid_rest(R& S, WK& W, bool needJ, bool needQ,
                                                                     int col) {
   constexpr int N3 = 3 * NB, N4 = 4 * NB, N7 = 7 * NB;
   if (needJ)
@@ -1307,20 +1343,15 @@ __device__ __attribute__((always_inline)) inline void step_mid_rest(Smem<NB, G>&
   wsync();
 }
 
-template <int NB, bool G, int STEP = WAVE, bool FACT = false>
-__device__ __attribute__((always_inline)) inline void step_post(Smem<NB, G>& S, Swork<NB>& W, double h, bool needJ, bool needQ, bool anyKick, int col) {
+template <int NB, bool G, int STEP = WAVE, bool FACT = false, bool STATE = true, class R, class WK>
+__device__ __attribute__((always_inline)) inline void step_post(R& S, WK& W, double h, bool needJ, bool needQ, bool anyKick, int col) {
   constexpr int N3 = 3 * NB, N4 = 4 * NB, N7 = 7 * NB;
   const double h2 = 0.5 * h;
   const double h6 = h / 6.0;
   // ---- drift
   if (needJ)
     for (int c = col; c < N7; c += STEP) drift_cols<NB>(S, c, h2);
-  for (int q = col; q < N3; q += STEP) {
-    double xq = S.x[q], eq = S.xe[q];
-    kahan(xq, eq, h2 * S.v[q]);
-    S.x[q] = xq;
-    S.xe[q] = eq;
-  }
+  if constexpr (STATE) drift_state<NB, STEP>(S, h2, col);
   wsync();
   if (needQ) {
     for (int q = col; q < N3; q += STEP) {
@@ -1331,7 +1362,7 @@ __device__ __attribute__((always_inline)) inline void step_post(Smem<NB, G>& S, 
   }
   wsync();
   // ---- kickfast!(s, d, h/6)
-  if constexpr (STEP == WAVE) {  // kicked pairs: whole-wave form only
+  if constexpr (STEP == WAVE && STATE) {  // kicked pairs: whole-wave form only
     if (anyKick) kick_build<NB>(S, W, h6, needQ, col);
   }
   wsync();
@@ -1465,11 +1496,11 @@ __device__ void ahl21_step2h(Smem<NB, false>& S0, Smem<NB, false>& S1, Swork<NB>
 // ---------------------------------------------------------------------------
 // Transit search (timing.jl:3-110) and element gradients (timing.jl:112-138)
 // ---------------------------------------------------------------------------
-template <int NB, bool G> __device__ inline double gsky(const Smem<NB, G>& S, int i, int j) {
+template <int NB, class R> __device__ inline double gsky(const R& S, int i, int j) {
   return (S.x[3 * j] - S.x[3 * i]) * (S.v[3 * j] - S.v[3 * i]) +
          (S.x[3 * j + 1] - S.x[3 * i + 1]) * (S.v[3 * j + 1] - S.v[3 * i + 1]);
 }
-template <int NB, bool G> __device__ inline double gdot(const Smem<NB, G>& S, int i, int j) {
+template <int NB, class R> __device__ inline double gdot(const R& S, int i, int j) {
   return (((S.x[3 * j] - S.x[3 * i]) * (S.dqdt[7 * j + 3] - S.dqdt[7 * i + 3]) +
            (S.x[3 * j + 1] - S.x[3 * i + 1]) * (S.dqdt[7 * j + 4] - S.dqdt[7 * i + 4])) +
           (S.v[3 * j] - S.v[3 * i]) * (S.dqdt[7 * j + 0] - S.dqdt[7 * i + 0])) +
@@ -1649,6 +1680,56 @@ template <int NB, bool G> __device__ void dtdelements(Smem<NB, G>& S, const SysD
 // ---------------------------------------------------------------------------
 // Load / store of a system between its HBM record and LDS.
 // ---------------------------------------------------------------------------
+// The level schedule of both sweeps from a record's masses and pair mask
+// (one lane).
+template <int NB, class R> __device__ inline void build_schedule(R& S) {
+  constexpr int NPS = Smem<NB>::NP > 0 ? Smem<NB>::NP : 1;
+  // a massless pair (gm == 0) leaves jac_ij from the pair before it in
+  // place (ahl21.jl:712-713), so systems with one keep the sequential order
+  bool seq = false;
+  for (int i = 0; i < NB - 1; ++i)
+    for (int j = i + 1; j < NB; ++j)
+      if (!S.pair[i + NB * j] && NBG_GNEWT * (S.m[i] + S.m[j]) == 0.0) seq = true;
+  S.seq = seq ? 1 : 0;
+  for (int dir = 0; dir < 2; ++dir) {
+    uint8_t pi_[NPS], pj_[NPS], lv[NPS];
+    int np = 0;
+    if (dir == 0) {
+      for (int i = 0; i < NB - 1; ++i)
+        for (int j = i + 1; j < NB; ++j)
+          if (!S.pair[i + NB * j]) { pi_[np] = (uint8_t)i; pj_[np] = (uint8_t)j; ++np; }
+    } else {
+      for (int i = NB - 2; i >= 0; --i)
+        for (int j = NB - 1; j >= i + 1; --j)
+          if (!S.pair[i + NB * j]) { pi_[np] = (uint8_t)i; pj_[np] = (uint8_t)j; ++np; }
+    }
+    int last[NB];
+    for (int b = 0; b < NB; ++b) last[b] = 0;
+    int nl = 0;
+    for (int p = 0; p < np; ++p) {
+      const int a = last[pi_[p]], b = last[pj_[p]];
+      const int l = seq ? p + 1 : (a > b ? a : b) + 1;
+      lv[p] = (uint8_t)l;
+      last[pi_[p]] = l;
+      last[pj_[p]] = l;
+      nl = l > nl ? l : nl;
+    }
+    int w = 0;
+    for (int l = 1; l <= nl; ++l) {
+      int cntl = 0;
+      for (int p = 0; p < np; ++p)
+        if (lv[p] == l) {
+          S.plist[dir][2 * w] = pi_[p];
+          S.plist[dir][2 * w + 1] = pj_[p];
+          ++w;
+          ++cntl;
+        }
+      S.lvw[dir][l - 1] = (uint8_t)cntl;
+    }
+    S.nlv[dir] = nl;
+  }
+}
+
 template <int NB, bool G> __device__ void load_system(Smem<NB, G>& S, const SysDesc& D, const SysBufs& B, int lane,
                                               bool loadJ = true) {
   double* J_ = S.JJ;
@@ -1676,53 +1757,7 @@ template <int NB, bool G> __device__ void load_system(Smem<NB, G>& S, const SysD
     S.rowupd = D.rowupd;
   }
   wsync();
-  if (lane == 0) {
-    constexpr int NPS = Smem<NB>::NP > 0 ? Smem<NB>::NP : 1;
-    // a massless pair (gm == 0) leaves jac_ij from the pair before it in
-    // place (ahl21.jl:712-713), so systems with one keep the sequential order
-    bool seq = false;
-    for (int i = 0; i < NB - 1; ++i)
-      for (int j = i + 1; j < NB; ++j)
-        if (!S.pair[i + NB * j] && NBG_GNEWT * (S.m[i] + S.m[j]) == 0.0) seq = true;
-    S.seq = seq ? 1 : 0;
-    for (int dir = 0; dir < 2; ++dir) {
-      uint8_t pi_[NPS], pj_[NPS], lv[NPS];
-      int np = 0;
-      if (dir == 0) {
-        for (int i = 0; i < NB - 1; ++i)
-          for (int j = i + 1; j < NB; ++j)
-            if (!S.pair[i + NB * j]) { pi_[np] = (uint8_t)i; pj_[np] = (uint8_t)j; ++np; }
-      } else {
-        for (int i = NB - 2; i >= 0; --i)
-          for (int j = NB - 1; j >= i + 1; --j)
-            if (!S.pair[i + NB * j]) { pi_[np] = (uint8_t)i; pj_[np] = (uint8_t)j; ++np; }
-      }
-      int last[NB];
-      for (int b = 0; b < NB; ++b) last[b] = 0;
-      int nl = 0;
-      for (int p = 0; p < np; ++p) {
-        const int a = last[pi_[p]], b = last[pj_[p]];
-        const int l = seq ? p + 1 : (a > b ? a : b) + 1;
-        lv[p] = (uint8_t)l;
-        last[pi_[p]] = l;
-        last[pj_[p]] = l;
-        nl = l > nl ? l : nl;
-      }
-      int w = 0;
-      for (int l = 1; l <= nl; ++l) {
-        int cntl = 0;
-        for (int p = 0; p < np; ++p)
-          if (lv[p] == l) {
-            S.plist[dir][2 * w] = pi_[p];
-            S.plist[dir][2 * w + 1] = pj_[p];
-            ++w;
-            ++cntl;
-          }
-        S.lvw[dir][l - 1] = (uint8_t)cntl;
-      }
-      S.nlv[dir] = nl;
-    }
-  }
+  if (lane == 0) build_schedule<NB>(S);
   if (D.grad && loadJ) {
     const double* J = B.jac + D.off_jac;
     const double* JE = J + (int64_t)N7 * N7;

@@ -47,7 +47,7 @@ struct SysDesc {
   int32_t tag;       // reported in SysBufs.done_list when the system finishes
   int32_t traj;      // MODE_CARTESIAN: TRAJ_* flags of the optional records
   int32_t rowupd;    // Jacobian row update of the pair sweeps: 0 the reference's order, 1 factored (set per launch)
-  int32_t pad_;
+  int32_t split;     // may run on the two-wave launches (nbg_split.h): Kepler pairs only, none of them massless
   int64_t nsteps;    // full steps in the run
   int64_t chunk;     // > 0: at most this many steps per visit (overrides the launch's chunk)
   int64_t ntt;
