@@ -62,6 +62,7 @@ extern "C" hipError_t nbg_launch_split_wide(nbg::GroupList gl, nbg::SysBufs bufs
 namespace {
 
 constexpr int NB_MIN = 2, NB_MAX = 12;
+constexpr int SPLIT_PAIR_MAX = 7;  // bodies of the largest systems paired on the two-wave launches
 
 template <class T> struct DevVec {
   T* p = nullptr;
@@ -204,6 +205,12 @@ void group_layout(Layout& L) {
   std::vector<int> partner(ns, -1);  // by system index
   for (size_t g = 0; g < L.gn.size() && budget > 0; ++g) {
     const int off = L.goff[g], cnt = L.gcnt[g], cls = L.gn[g];
+    // On the two-wave launches pairs pay up to SPLIT_PAIR_MAX bodies: from 8 on
+    // the Jacobians of twice as many systems overflow the L2 cache (rounds of
+    // 100 steps over 2048 systems of n bodies, one against two a workgroup: 3:
+    // 8.9, 6.1 ms; 5: 17.0, 13.9; 7: 31.6, 26.9; 8: 44.1, 42.3; 9: 52.1, 74.4).
+    bool two_wave = cls == 9;
+    for (int k = 0; k < cnt; ++k) two_wave = two_wave && L.desc[L.order[off + k]].split;
     std::vector<std::vector<int>> pos(NB_MAX + 1);  // systems by body count, longest first
     for (int k = 0; k < cnt; ++k) pos[L.desc[L.order[off + k]].n].push_back(L.order[off + k]);
     // the shortest systems first, across body counts
@@ -213,7 +220,7 @@ void group_layout(Layout& L) {
       int bn = -1;
       double bc = 0.0;
       for (int n = NB_MIN; n <= NB_MAX; ++n) {
-        if (at[n] < 1 || !nbg_duo_pairs(cls, n)) continue;
+        if (at[n] < 1 || !nbg_duo_pairs(cls, n) || (two_wave && n > SPLIT_PAIR_MAX)) continue;
         const double c = cost(pos[n][at[n] - 1]);
         if (bn < 0 || c < bc) { bn = n; bc = c; }
       }

@@ -28,6 +28,8 @@
 // one-wave step's, so results are the same bits.
 #pragma once
 
+#include <type_traits>
+
 #include "nbg_device.h"
 
 namespace nbg {
@@ -78,12 +80,81 @@ struct RingSlot {
   double mijinv;
   int i, j;
 };
-// A pair's Jacobian as the row updates read it.
+// A pair's Jacobian as the row updates read it: their coefficients in the
+// order of use -- in the reference's order mj * kep (36), mi * kep (36) and the
+// mass columns mc (24); factored kep (36) and mc (24) -- and kep's h column.
+// The kep block is column-major, rk + 6 k.
 struct JacSlot {
-  double kep[48];
-  double mc[24];
+  double c[96];
+  double kh[6];
   double mi, mj;
   int i, j;
+};
+
+// acc[r] = fma(+-coefficient I + r, x, acc[r]), r = 0..5, the coefficients held
+// one per lane: lane l of every row of 16 lanes has coefficients l, 16 + l, ...
+// in cf, and each multiply-add broadcasts its own along the row (DPP
+// row_newbcast).  Read from LDS instead, a coefficient costs every lane its
+// bytes -- 16 cycles of the compute unit's LDS per pair of coefficients -- and a wait:
+// an update of 9 bodies' rows took 2,850 cycles of which its arithmetic
+// issues 1,000.  Every lane of the row must be active.  The leading wait keeps
+// a coefficient that was just copied between registers readable by DPP.
+template <int I, bool NEG = false> __device__ __forceinline__ void fmac6(double* acc, const double* cf, double x) {
+#define NBG_FMAC6(SIGN)                                                                              \
+  asm("s_nop 1\n\t"                                                                                  \
+      "v_fmac_f64_dpp %0, %6, " SIGN "%12 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"           \
+      "v_fmac_f64_dpp %1, %7, " SIGN "%12 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"           \
+      "v_fmac_f64_dpp %2, %8, " SIGN "%12 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"           \
+      "v_fmac_f64_dpp %3, %9, " SIGN "%12 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"           \
+      "v_fmac_f64_dpp %4, %10, " SIGN "%12 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"          \
+      "v_fmac_f64_dpp %5, %11, " SIGN "%12 row_newbcast:%18 row_mask:0xf bank_mask:0xf"              \
+      : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5])           \
+      : "v"(cf[I / 16]), "v"(cf[(I + 1) / 16]), "v"(cf[(I + 2) / 16]), "v"(cf[(I + 3) / 16]),        \
+        "v"(cf[(I + 4) / 16]), "v"(cf[(I + 5) / 16]), "v"(x), "n"(I % 16), "n"((I + 1) % 16),        \
+        "n"((I + 2) % 16), "n"((I + 3) % 16), "n"((I + 4) % 16), "n"((I + 5) % 16))
+  if constexpr (NEG) NBG_FMAC6("-");
+  else NBG_FMAC6("");
+#undef NBG_FMAC6
+}
+// s = fma(coefficient I + r, x[r], s) for r = 0..2, then coefficient M with u.
+template <int I, int M> __device__ __forceinline__ double fmac_body(double s, const double* cf, const double* x, double u) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %1, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %2, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %3, %7 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %4, %8 row_newbcast:%12 row_mask:0xf bank_mask:0xf"
+      : "+v"(s)
+      : "v"(cf[I / 16]), "v"(cf[(I + 1) / 16]), "v"(cf[(I + 2) / 16]), "v"(cf[M / 16]), "v"(x[0]), "v"(x[1]), "v"(x[2]),
+        "v"(u), "n"(I % 16), "n"((I + 1) % 16), "n"((I + 2) % 16), "n"(M % 16));
+  return s;
+}
+
+template <int NB, int D> __device__ __forceinline__ double split_row_product(double s, const double* cf, const double* P, const double* u) {
+  if constexpr (D < NB) {
+    s = fmac_body<3 * D, 3 * NB + D>(s, cf, P + 3 * D, u[D]);
+    return split_row_product<NB, D + 1>(s, cf, P, u);
+  }
+  return s;
+}
+
+// A column of J and its error: rows at whole distances from one 32-bit
+// offset, so that an access is a base, an offset register and an immediate
+// (global: the scalar base of the record's store).
+template <int NB, class R> struct Column {
+  static constexpr int N7 = 7 * NB;
+  static constexpr uint32_t ERR = 8u * R::JOFF;
+  typename std::conditional<R::JG, __attribute__((address_space(1))) char*, char*>::type base;
+  uint32_t off;
+  __device__ __forceinline__ Column(R& S, int row, int c) : off(8u * (uint32_t)(row * N7 + c)) {
+    if constexpr (R::JG) base = (__attribute__((address_space(1))) char*)uniform_global(S.jg);
+    else base = (char*)S.JJ;
+  }
+  __device__ __forceinline__ auto& j(int k) const { return at(off + 8u * (uint32_t)(k * N7)); }
+  __device__ __forceinline__ auto& e(int k) const { return at(off + ERR + 8u * (uint32_t)(k * N7)); }
+  __device__ __forceinline__ auto& at(uint32_t o) const {
+    if constexpr (R::JG) return *(gdouble*)(base + o);
+    else return *(double*)(base + o);
+  }
 };
 
 // The state wave's record of a system.
@@ -112,8 +183,10 @@ template <int NB, bool G> struct JacRec {
   double mv[N3], mx[N3], qx[N3], qv[N3];
 };
 
-// The Jacobian wave's work area: the force-gradient stage, or pair Jacobians.
-template <int NB> struct JacWork {
+// The Jacobian wave's work area: the force-gradient stage, or pair Jacobians
+// -- as many as fit beside it, and at least CHMIN (a call that forms pair
+// Jacobians takes the same time for one pair as for a wave of them).
+template <int NB, int CHMIN> struct JacWork {
   static constexpr int N3 = 3 * NB, N4 = 4 * NB, NP = NB * (NB - 1) / 2, PQ = 13;
   struct F {
     double phi[N3 * N4];
@@ -121,7 +194,8 @@ template <int NB> struct JacWork {
     double pq[NP * PQ];
   };
   static constexpr int FIT = (int)(sizeof(F) / sizeof(JacSlot));
-  static constexpr int CH = FIT < 1 ? 1 : (FIT < NP ? FIT : NP);
+  static constexpr int CH1 = FIT < CHMIN ? CHMIN : FIT;
+  static constexpr int CH = CH1 < NP ? CH1 : NP;
   union {
     F f;
     JacSlot slot[CH];
@@ -148,16 +222,17 @@ template <int NB, bool G, bool TWO, int LIMIT> struct SplitLds {
                                   sizeof(Schedule<NB>) + 64;
   static constexpr int NP = NB * (NB - 1) / 2;
   static constexpr int RMIN = NB / 2 < 1 ? 1 : NB / 2;
+  using Work = JacWork<NB, (LIMIT > 100000 ? 20 : NB <= 4 ? 6 : 1)>;
   // two work areas where they fit: both systems' force gradients at once
   static constexpr bool PHI2 = TWO && 4 * NB <= 32 && NP <= 32 &&
-                               FIXED + 2 * sizeof(JacWork<NB>) + 2 * RMIN * sizeof(RingSlot) <= (size_t)LIMIT;
+                               FIXED + 2 * sizeof(Work) + 2 * RMIN * sizeof(RingSlot) <= (size_t)LIMIT;
   static constexpr int NW = PHI2 ? 2 : 1;
-  static constexpr long LEFT = (long)LIMIT - (long)(FIXED + NW * sizeof(JacWork<NB>));
+  static constexpr long LEFT = (long)LIMIT - (long)(FIXED + NW * sizeof(Work));
   static constexpr int RFIT = LEFT > 0 ? (int)(LEFT / (long)(NS * sizeof(RingSlot))) : 0;
   static constexpr int R = RFIT < NP ? RFIT : NP;  // ring slots per system
   static constexpr bool fits = RFIT >= RMIN;
   // pairs per chunk of the Jacobian wave (a chunk is a run of whole levels)
-  static constexpr int CHW = TWO && !PHI2 ? JacWork<NB>::CH / 2 : JacWork<NB>::CH;
+  static constexpr int CHW = TWO && !PHI2 ? Work::CH / 2 : Work::CH;
   static constexpr int CHL = TWO ? 32 : 64;
   static constexpr int CH0 = CHW < CHL ? CHW : CHL;
   static constexpr int RR = R < 1 ? 1 : R;
@@ -165,7 +240,7 @@ template <int NB, bool G, bool TWO, int LIMIT> struct SplitLds {
   static constexpr bool ok = fits && CH >= RMIN;
   StateRec<NB> t[NS];
   JacRec<NB, G> j[NS];
-  JacWork<NB> w[NW];
+  Work w[NW];
   RingSlot ring[NS][RR];
   SplitCtl ctl;
   Schedule<NB> sched;
@@ -662,7 +737,8 @@ __device__ void split_state(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0, c
 // One pair's Jacobian (pair_jacobian) from its ring slot: the drift's other
 // quantities by the formulas of jac_delxv_gamma!.
 template <bool DF>
-static __device__ __attribute__((noinline)) void split_pair_jacobian(uint32_t ring, uint32_t slot, double m_i, double m_j, double h) {
+static __device__ __attribute__((noinline)) void split_pair_jacobian(uint32_t ring, uint32_t slot, double m_i, double m_j, double h, int factored) {
+  const bool fact = __builtin_amdgcn_readfirstlane(factored) != 0;
   const RingSlot* a = lds_at<RingSlot>(ring);
   JacSlot* o = lds_at<JacSlot>(slot);
   KParams P;
@@ -698,24 +774,143 @@ static __device__ __attribute__((noinline)) void split_pair_jacobian(uint32_t ri
   for (int q = 0; q < 48; ++q) kep[q] = 0.0;
   for (int q = 0; q < 6; ++q) jm[q] = 0.0;
   compute_jacobian_gamma(P, x0, v0, kep, jm, DF);
+  double* mc = fact ? o->c + 36 : o->c + 72;
   for (int rk = 0; rk < 6; ++rk) {
-    o->mc[rk] = jm[rk] * m_j;
-    o->mc[6 + rk] = (((-mj) * dl[rk]) * mijinv) - ((NBG_GNEWT * mi) * kep[rk + 36]);
-    o->mc[12 + rk] = ((mi * dl[rk]) * mijinv) + ((NBG_GNEWT * mj) * kep[rk + 36]);
-    o->mc[18 + rk] = (-jm[rk]) * m_i;
+    mc[rk] = jm[rk] * m_j;
+    mc[6 + rk] = (((-mj) * dl[rk]) * mijinv) - ((NBG_GNEWT * mi) * kep[rk + 36]);
+    mc[12 + rk] = ((mi * dl[rk]) * mijinv) + ((NBG_GNEWT * mj) * kep[rk + 36]);
+    mc[18 + rk] = (-jm[rk]) * m_i;
   }
-  for (int q = 0; q < 48; ++q) o->kep[q] = kep[q];
+  if (fact) {
+    for (int q = 0; q < 36; ++q) o->c[q] = kep[q];
+  } else {
+    for (int q = 0; q < 36; ++q) {
+      o->c[q] = mj * kep[q];
+      o->c[36 + q] = mi * kep[q];
+    }
+  }
+  for (int q = 0; q < 6; ++q) o->kh[q] = kep[42 + q];
   o->mi = mi; o->mj = mj;
   o->i = a->i; o->j = a->j;
 }
 
-// jij_coef from a JacSlot (the mass columns as pair_cols takes them).
-__device__ inline double split_coef(const JacSlot& sl, bool rowi, int rk, int k) {
-  if (k == 6) return sl.mc[(rowi ? 0 : 6) + rk];
-  if (k == 13) return sl.mc[(rowi ? 12 : 18) + rk];
-  const double kv = sl.kep[rk + 6 * (k < 7 ? k : k - 7)];
-  if (rowi == (k < 7)) return 0.0 + (rowi ? sl.mj : sl.mi) * kv;
-  return 0.0 - (rowi ? sl.mj : sl.mi) * kv;
+// jij_coef from a JacSlot, without its sign for k of the Kepler block.
+template <bool FACT> __device__ __forceinline__ double split_coef(const JacSlot& sl, bool rowi, int rk, int k) {
+  constexpr int MC = FACT ? 36 : 72;
+  if (k == 6) return sl.c[MC + (rowi ? 0 : 6) + rk];
+  if (k == 13) return sl.c[MC + (rowi ? 12 : 18) + rk];
+  const int at = rk + 6 * (k < 7 ? k : k - 7);
+  const double v = FACT ? (rowi ? sl.mj : sl.mi) * sl.c[at] : sl.c[(rowi ? 0 : 36) + at];
+  return rowi == (k < 7) ? v : -v;
+}
+
+// pair_cols from a JacSlot (same operations), STEP lanes a system, every one
+// of them taking part: those past the last column compute it again and store
+// nothing.
+template <int NB, bool G, int STEP, bool FACT, class R>
+__device__ __attribute__((always_inline)) inline void split_pair_cols(R& S, const JacSlot& sl, int i, int j, int col) {
+  constexpr int N7 = 7 * NB, NC = FACT ? 4 : 6;
+  double cf[NC];
+#pragma unroll
+  for (int r = 0; r < NC; ++r) cf[r] = sl.c[16 * r + (col & 15)];
+  const double mi = sl.mi, mj = sl.mj;
+#pragma unroll 1
+  for (int c0 = 0; c0 < N7; c0 += STEP) {
+    const bool on = c0 + col < N7;
+    const int c = on ? c0 + col : N7 - 1;
+    double a[12], e[12], o[12];
+    const Column<NB, R> Ci(S, 6 * i, c), Cj(S, 6 * j, c);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      a[k] = Ci.j(k);
+      a[6 + k] = Cj.j(k);
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      e[k] = Ci.e(k);
+      e[6 + k] = Cj.e(k);
+    }
+    // all 24 rows are in flight before the arithmetic starts (left alone, the
+    // scheduler moves the error rows' loads down to their uses, each with a
+    // wait of its own)
+    __builtin_amdgcn_sched_barrier(0);
+    const double a6 = (c == 7 * i + 6) ? 1.0 : 0.0;
+    const double a13 = (c == 7 * j + 6) ? 1.0 : 0.0;
+    if constexpr (FACT) {
+      double d[6], sk[6];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        d[k] = a[k] - a[6 + k];
+        sk[k] = 0.0;
+      }
+      fmac6<0>(sk, cf, d[0]);
+      fmac6<6>(sk, cf, d[1]);
+      fmac6<12>(sk, cf, d[2]);
+      fmac6<18>(sk, cf, d[3]);
+      fmac6<24>(sk, cf, d[4]);
+      fmac6<30>(sk, cf, d[5]);
+#pragma unroll
+      for (int rk = 0; rk < 6; ++rk) {
+        o[rk] = mj * sk[rk];
+        o[6 + rk] = (-mi) * sk[rk];
+      }
+      fmac6<36>(o, cf, a6);
+      fmac6<42>(o + 6, cf, a6);
+      fmac6<48>(o, cf, a13);
+      fmac6<54>(o + 6, cf, a13);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 12; ++q) o[q] = 0.0;
+      // k = 0..5: rows of i get +mj*kep * a_i[k], rows of j -mi*kep * a_i[k]
+      fmac6<0>(o, cf, a[0]);
+      fmac6<36, true>(o + 6, cf, a[0]);
+      fmac6<6>(o, cf, a[1]);
+      fmac6<42, true>(o + 6, cf, a[1]);
+      fmac6<12>(o, cf, a[2]);
+      fmac6<48, true>(o + 6, cf, a[2]);
+      fmac6<18>(o, cf, a[3]);
+      fmac6<54, true>(o + 6, cf, a[3]);
+      fmac6<24>(o, cf, a[4]);
+      fmac6<60, true>(o + 6, cf, a[4]);
+      fmac6<30>(o, cf, a[5]);
+      fmac6<66, true>(o + 6, cf, a[5]);
+      fmac6<72>(o, cf, a6);
+      fmac6<78>(o + 6, cf, a6);
+      // k = 7..12: rows of i get -mj*kep * a_j[k], rows of j +mi*kep * a_j[k]
+      fmac6<0, true>(o, cf, a[6]);
+      fmac6<36>(o + 6, cf, a[6]);
+      fmac6<6, true>(o, cf, a[7]);
+      fmac6<42>(o + 6, cf, a[7]);
+      fmac6<12, true>(o, cf, a[8]);
+      fmac6<48>(o + 6, cf, a[8]);
+      fmac6<18, true>(o, cf, a[9]);
+      fmac6<54>(o + 6, cf, a[9]);
+      fmac6<24, true>(o, cf, a[10]);
+      fmac6<60>(o + 6, cf, a[10]);
+      fmac6<30, true>(o, cf, a[11]);
+      fmac6<66>(o + 6, cf, a[11]);
+      fmac6<84>(o, cf, a13);
+      fmac6<90>(o + 6, cf, a13);
+    }
+#pragma unroll
+    for (int q = 0; q < 12; ++q) {
+      double sv = a[q], se = e[q];
+      se += o[q];
+      const double t = sv + se;
+      se += sv - t;
+      a[q] = t;
+      e[q] = se;
+    }
+    if (on) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        Ci.j(k) = a[k];
+        Cj.j(k) = a[6 + k];
+        Ci.e(k) = e[k];
+        Cj.e(k) = e[6 + k];
+      }
+    }
+  }
 }
 
 // Phase C of a chunk (sweep_rows).
@@ -725,8 +920,7 @@ __device__ __attribute__((always_inline)) inline void split_rows(R& S, const Jac
   for (int q = 0; q < cnt; ++q) {
     const JacSlot& sl = slots[q];
     const int i = sl.i, j = sl.j;
-    if (needJ)
-      for (int c = col; c < 7 * NB; c += STEP) pair_cols<NB, G, FACT>(S, sl, i, j, c);
+    if (needJ) split_pair_cols<NB, G, STEP, FACT>(S, sl, i, j, col);
     if (needQ) {
       // dqdt_ij (ahl21.jl:743-748) and dq/dt's rows
       if (col < 14) {
@@ -740,8 +934,8 @@ __device__ __attribute__((always_inline)) inline void split_rows(R& S, const Jac
         double s2 = 0.0, dq = S.dqij[col];
         const double mine = S.dqdt[rowi ? 7 * i + rk : 7 * j + rk];
         if (rk < 6) {
-          dq = (rowi ? sl.mj : -sl.mi) * sl.kep[rk + 42];
-          for (int k = 0; k < 14; ++k) s2 = fmad(split_coef(sl, rowi, rk, k), q1[k], s2);
+          dq = (rowi ? sl.mj : -sl.mi) * sl.kh[rk];
+          for (int k = 0; k < 14; ++k) s2 = fmad(split_coef<FACT>(sl, rowi, rk, k), q1[k], s2);
         } else {
           for (int k = 0; k < 14; ++k) s2 = fmad(0.0, q1[k], s2);
         }
@@ -787,8 +981,8 @@ __device__ __attribute__((always_inline)) inline bool split_sweep(SplitLds<NB, G
         const double* m = second ? P.j[K].m : P.j[0].m;
         JacSlot* o = (second ? s1 : s0) + q;
         const double hh = second ? hh1 : hh0;
-        if (dir == 0) split_pair_jacobian<true>(lds_off(a), lds_off(o), m[a->i], m[a->j], hh);
-        else split_pair_jacobian<false>(lds_off(a), lds_off(o), m[a->i], m[a->j], hh);
+        if (dir == 0) split_pair_jacobian<true>(lds_off(a), lds_off(o), m[a->i], m[a->j], hh, FACT);
+        else split_pair_jacobian<false>(lds_off(a), lds_off(o), m[a->i], m[a->j], hh, FACT);
       }
     }
     wsync();
@@ -808,6 +1002,310 @@ __device__ __attribute__((always_inline)) inline bool split_sweep(SplitLds<NB, G
     }
   }
   return true;
+}
+
+// phisalpha! with Jacobian (phisalpha_cols' operations and order) for Kepler
+// pairs only, STEP lanes a system, a lane a column of dadq and jac_phi (column
+// (d, p): coordinate p of body d, p = 3 its mass).  The terms that depend on a
+// column's role in a pair enter as products with 0, 1 or -1 -- exact, and a
+// zero added instead of left out changes at most a zero's sign -- where selects
+// of 64-bit values took three quarters of the loop's 315 instructions.
+template <int NB, int STEP, bool FACT, class R, class WK>
+__device__ __attribute__((always_inline)) inline void split_phi(R& S, WK& W, double h, bool needQ, int col) {
+  constexpr int N3 = 3 * NB, N4 = 4 * NB, NP = WK::NP, PQ = WK::PQ, PP = (NP + STEP - 1) / STEP;
+  double* PHI = W.f.phi;
+  double* D = W.f.dadq;
+  double* pq = W.f.pq;
+  const double coeff = (((2.0 * (h * h * h)) / 96.0) * 2.0) * NBG_GNEWT;
+  // loop 1 factors (ahl21.jl:569-575)
+#pragma unroll
+  for (int u = 0; u < PP; ++u) {
+    const int p = col + u * STEP;
+    if (p < NP) {
+      int i, j;
+      pair_at<NB>(p, i, j);
+      double rij[3];
+      for (int k = 0; k < 3; ++k) rij[k] = S.x[3 * i + k] - S.x[3 * j + k];
+      const double r2 = dot3(rij);
+      const double fac2 = NBG_GNEWT / (r2 * __builtin_sqrt(r2));
+      const double q = 3.0 / r2;
+      double* o = pq + p * PQ;
+      o[0] = fac2;
+      for (int k = 0; k < 3; ++k) {
+        o[1 + k] = fac2 * rij[k];
+        o[4 + k] = (fac2 * rij[k]) * q;
+      }
+    }
+  }
+  wsync();
+  // the lane's column; columns past the last work on it again for nothing
+  const bool own = col < N4;
+  const int cc = own ? col : N4 - 1;
+  const int myd = cc < N3 ? cc / 3 : cc - N3, myp = cc < N3 ? cc - 3 * (cc / 3) : 3;
+  const double pos = myp < 3 ? 1.0 : 0.0, mass = 1.0 - pos;
+  const int ry = myp < 3 ? myp : 0;
+  double pk[3];
+  for (int k = 0; k < 3; ++k) pk[k] = myp == k ? 1.0 : 0.0;
+  // loop 1 (ahl21.jl:567-602), the lane's column: row block b != myd from the
+  // pair (b, myd), row block myd over the partners in increasing order
+  {
+    const double md = S.m[myd], xd = S.x[3 * myd + ry];
+    double db[3] = {0.0, 0.0, 0.0}, ab = 0.0;
+#pragma unroll 2
+    for (int q = 0; q < NB - 1; ++q) {
+      const bool after = q >= myd;  // the other body comes after myd
+      const int b = after ? q + 1 : q;
+      const double* o = pq + (after ? pair_index<NB>(myd, b) : pair_index<NB>(b, myd)) * PQ;
+      const double sg = after ? 1.0 : -1.0;  // +1: myd is i
+      const double rmy = (sg * pos) * (xd - S.x[3 * b + ry]);
+      const double mb = S.m[b], f2 = o[0], mm = sg * mass;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double fac = o[1 + k], f3 = o[4 + k];
+        // row block b: myd is its partner
+        const double t1 = fmad(mm, fac, -((f3 * md) * rmy));
+        const double t = (0.0 + t1) + pk[k] * (f2 * md);
+        if (own) D[(3 * b + k) * N4 + cc] = t;
+        // row block myd
+        db[k] = (db[k] + (f3 * mb) * rmy) - pk[k] * (f2 * mb);
+      }
+      const double mf = mb * o[1 + ry];
+      ab -= sg * mf;
+    }
+    if (own)
+      for (int k = 0; k < 3; ++k) D[(3 * myd + k) * N4 + cc] = db[k];
+    if (own && myp < 3) S.a[3 * myd + myp] = ab;
+  }
+  wsync();
+  // loop 2 factors (ahl21.jl:609-640)
+#pragma unroll
+  for (int u = 0; u < PP; ++u) {
+    const int p = col + u * STEP;
+    if (p < NP) {
+      int i, j;
+      pair_at<NB>(p, i, j);
+      double rij[3], aij[3];
+      for (int k = 0; k < 3; ++k) {
+        aij[k] = S.a[3 * i + k] - S.a[3 * j + k];
+        rij[k] = S.x[3 * i + k] - S.x[3 * j + k];
+      }
+      const double r2 = dot3(rij);
+      const double r1 = __builtin_sqrt(r2);
+      const double ardot = dot3(aij, rij);
+      const double fac1 = coeff / ((r2 * r2) * r1);
+      const double mi = S.m[i], mj = S.m[j];
+      const double fac2 = ((2.0 * NBG_GNEWT) * (mi + mj)) / r1 + 3.0 * ardot;
+      double* o = pq + p * PQ;
+      for (int k = 0; k < 3; ++k) {
+        o[k] = fac1 * (rij[k] * fac2 - r2 * aij[k]);                                             // fac
+        o[4 + k] = (((2.0 * NBG_GNEWT) * fac1) * rij[k]) / r1;                                   // fm
+        o[7 + k] = ((-2.0) * fac1) * ((((rij[k] * NBG_GNEWT) * (mi + mj)) / (r2 * r1)) + aij[k]);  // fr
+      }
+      o[3] = 5.0 / r2;
+      o[10] = fac1 * 3.0;
+      o[11] = fac1 * fac2;   // fd
+      o[12] = (-fac1) * r2;  // fa
+    }
+  }
+  wsync();
+  if (needQ) {
+    // dqdt_phi, a lane an entry: the pairs of a body in increasing order of
+    // its partner, as in the reference's loop
+    const double q3h = 3.0 / h;
+    for (int e = col; e < N3; e += STEP) {
+      const int b = e / 3, k = e - 3 * b;
+      double qb = S.dqdt_phi[7 * b + 3 + k];
+      for (int q = 0; q < NB - 1; ++q) {
+        const bool bi = q >= b;
+        const int c = bi ? q + 1 : q;
+        const double qm = (q3h * S.m[c]) * pq[(bi ? pair_index<NB>(b, c) : pair_index<NB>(c, b)) * PQ + k];
+        qb += bi ? qm : -qm;
+      }
+      S.dqdt_phi[7 * b + 3 + k] = qb;
+    }
+  }
+  // loop 2 (ahl21.jl:607-698)
+  if constexpr (FACT) {
+    // pair by pair: the rows of body i receive mj * X, those of body j
+    // -mi * X of the same column term X (phisalpha_cols' factored form)
+    if (own)
+      for (int r = 0; r < N3; ++r) PHI[r * N4 + cc] = 0.0;
+    int p = 0;
+#pragma unroll 1
+    for (int i = 0; i < NB - 1; ++i) {
+      double pi[3], xi[3], Di[3];
+      for (int k = 0; k < 3; ++k) {
+        pi[k] = PHI[(3 * i + k) * N4 + cc];
+        xi[k] = S.x[3 * i + k];
+        Di[k] = D[(3 * i + k) * N4 + cc];
+      }
+      const double mi = S.m[i], ai = S.a[3 * i + ry], xr = S.x[3 * i + ry];
+      const double si = myd == i ? 1.0 : 0.0;
+#pragma unroll 1
+      for (int j = i + 1; j < NB; ++j, ++p) {
+        const double* o = pq + p * PQ;
+        const double mj = S.m[j], sj = myd == j ? 1.0 : 0.0;
+        const double sg = pos * (si - sj), mm = mass * (si + sj), ci = mass * si, cj = mass * sj;
+        double r[3], dD[3], pj[3];
+        for (int k = 0; k < 3; ++k) {
+          r[k] = xi[k] - S.x[3 * j + k];
+          dD[k] = Di[k] - D[(3 * j + k) * N4 + cc];
+          pj[k] = PHI[(3 * j + k) * N4 + cc];
+        }
+        const double rmy = xr - S.x[3 * j + ry], amy = ai - S.a[3 * j + ry];
+        double dot = 0.0;
+        for (int k = 0; k < 3; ++k) dot += r[k] * dD[k];
+        const double fd = o[11], fa = o[12];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const double fac = o[k], ff = o[10] * r[k];
+          const double base = (pk[k] * fd - (fac * o[3]) * rmy) + (o[7 + k] * rmy + ff * amy);
+          const double role = fmad(mm, o[4 + k], sg * base);
+          const double X = (role + fa * dD[k]) + ff * dot;
+          pi[k] += fmad(cj, fac, mj * X);
+          pj[k] += fmad(-ci, fac, (-mi) * X);
+        }
+        if (own)
+          for (int k = 0; k < 3; ++k) PHI[(3 * j + k) * N4 + cc] = pj[k];
+      }
+      if (own)
+        for (int k = 0; k < 3; ++k) PHI[(3 * i + k) * N4 + cc] = pi[k];
+    }
+  } else {
+    // one row block at a time over its partners c in increasing order; with
+    // r, dD and the like taken from b to c, the signs of the pair's order
+    // cancel except in the terms that carry sb
+#pragma unroll 1
+    for (int b = 0; b < NB; ++b) {
+      double pb[3], xb[3], Db[3];
+      for (int k = 0; k < 3; ++k) {
+        pb[k] = 0.0;
+        xb[k] = S.x[3 * b + k];
+        Db[k] = D[(3 * b + k) * N4 + cc];
+      }
+      const double ar = S.a[3 * b + ry], xr = S.x[3 * b + ry], self = myd == b ? 1.0 : 0.0;
+#pragma unroll 1
+      for (int q = 0; q < NB - 1; ++q) {
+        const bool bi = q >= b;
+        const int c = bi ? q + 1 : q;
+        const double* o = pq + (bi ? pair_index<NB>(b, c) : pair_index<NB>(c, b)) * PQ;
+        const double sb = bi ? 1.0 : -1.0, m = S.m[c], other = myd == c ? 1.0 : 0.0;
+        const double sg = pos * (self - other);
+        const double rs = (sg * sb) * (xr - S.x[3 * c + ry]), as = (sg * sb) * (ar - S.a[3 * c + ry]);
+        const double ms = (mass * self) * sb, mo = (mass * other) * sb;
+        double r[3], dD[3];
+        for (int k = 0; k < 3; ++k) {
+          r[k] = xb[k] - S.x[3 * c + k];
+          dD[k] = Db[k] - D[(3 * c + k) * N4 + cc];
+        }
+        double dot = 0.0;
+        for (int k = 0; k < 3; ++k) dot += r[k] * dD[k];
+        const double fdm = o[11] * m, fam = o[12] * m;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const double fac = o[k], ff = o[10] * (sb * r[k]), y = o[4 + k] * m;
+          const double t1 = fmad(ms, y, fmad(mo, fac, -(((fac * o[3]) * m) * rs)));
+          const double t2 = fmad(mo, y, fdm * (sg * pk[k]));
+          const double t3 = m * (o[7 + k] * rs + ff * as);
+          pb[k] = (((((pb[k] + t1) + t2) + t3) + fam * dD[k]) + (ff * m) * (sb * dot));
+        }
+      }
+      if (own)
+        for (int k = 0; k < 3; ++k) PHI[(3 * b + k) * N4 + cc] = pb[k];
+    }
+  }
+}
+
+// The drift of J's position rows (drift_grad!) and, in the reference's order,
+// the zero-addend compensated pass over every row that follows it; a body's
+// rows at a time, all in flight together.
+template <int NB, bool G, int STEP, bool FACT, class R>
+__device__ __attribute__((always_inline)) inline void split_drift(R& S, double hh, int col) {
+  constexpr int N7 = 7 * NB;
+  for (int c = col; c < N7; c += STEP) {
+#pragma unroll 1
+    for (int b = 0; b < NB; ++b) {
+      const Column<NB, R> C(S, 6 * b, c);
+      double a[6], e[6];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        a[k] = C.j(k);
+        if (!FACT || k < 3) e[k] = C.e(k);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) kahan(a[k], e[k], hh * a[3 + k]);
+      if constexpr (!FACT) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+          e[k] += 0.0;
+          const double t = a[k] + e[k];
+          e[k] += a[k] - t;
+          a[k] = t;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < (FACT ? 3 : 6); ++k) {
+        C.j(k) = a[k];
+        C.e(k) = e[k];
+      }
+    }
+  }
+}
+
+// J_vel += Phi * J_pos (step_mid_rest): Phi's rows broadcast along the lanes,
+// the columns' position rows in registers.
+template <int NB, bool G, int STEP, bool FACT, class R>
+__device__ __attribute__((always_inline)) inline void split_vel_product(R& S, const double* B, int col) {
+  constexpr int N3 = 3 * NB, N4 = 4 * NB, N7 = 7 * NB, NC = (N4 + 15) / 16;
+#pragma unroll 1
+  for (int c0 = 0; c0 < N7; c0 += STEP) {
+    const bool on = c0 + col < N7;
+    const int c = on ? c0 + col : N7 - 1;
+    const Column<NB, R> C(S, 0, c);
+    double P[N3], u[NB];
+#pragma unroll
+    for (int d = 0; d < NB; ++d) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) P[3 * d + p] = C.j(6 * d + p);
+      u[d] = (c == 7 * d + 6) ? 1.0 : 0.0;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+    for (int b = 0; b < NB; ++b) {
+      const Column<NB, R> V(S, 6 * b + 3, c);
+      double s[3], a[3], e[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        a[k] = V.j(k);
+        e[k] = V.e(k);
+      }
+      double cf[3][NC];
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int r = 0; r < NC; ++r) {
+          const int at = 16 * r + (col & 15);
+          cf[k][r] = B[(3 * b + k) * N4 + (at < N4 ? at : N4 - 1)];
+        }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        s[k] = split_row_product<NB, 0>(0.0, cf[k], P, u);
+        kahan(a[k], e[k], s[k]);
+      }
+      if (on) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          V.j(k) = a[k];
+          V.e(k) = e[k];
+        }
+      }
+    }
+    if constexpr (!FACT) {
+      if (on) zero_add_rows<NB>(S, c, true, false);
+    }
+  }
 }
 
 // The Jacobian kept for (or back from) a transit's gradient step.
@@ -902,8 +1400,8 @@ __device__ void split_jacobian(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0
   SplitFollow<NB, G, TWO, LIMIT> F{0, 0, bound, err};
   JacRec<NB, G>& J0 = P.j[0];
   JacRec<NB, G>& J1 = P.j[K];
-  JacWork<NB>& W0 = P.w[0];
-  JacWork<NB>& W1 = P.w[L::NW - 1];
+  typename L::Work& W0 = P.w[0];
+  typename L::Work& W1 = P.w[L::NW - 1];
   const bool sys = L::HALF && lane >= 32;
   const int col = L::HALF ? lane & 31 : lane;
   int seen = 0, answered = 0;
@@ -926,11 +1424,17 @@ __device__ void split_jacobian(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0
     if (n0 & SPLIT_SAVE) split_keep_jac<NB>(J0, B.ws + D0.off_ws, false, lane);
     if (n1 & SPLIT_SAVE) split_keep_jac<NB>(J1, B.ws + D1.off_ws, false, lane);
     if constexpr (L::HALF) {
-      step_pre<NB, G, 32, FACT, false>(sys ? J1 : J0, W0, sys ? h1 : h0, sys ? j1 : j0, sys ? q1 : q0, false, col);
+      step_pre<NB, G, 32, FACT, false>(sys ? J1 : J0, W0, sys ? h1 : h0, false, sys ? q1 : q0, false, col);
+      if (sys ? j1 : j0) split_drift<NB, G, 32, FACT>(sys ? J1 : J0, 0.5 * (sys ? h1 : h0), col);
     } else {
-      step_pre<NB, G, STEP, FACT, false>(J0, W0, h0, j0, q0, false, lane);
-      if constexpr (TWO) step_pre<NB, G, STEP, FACT, false>(J1, W0, h1, j1, q1, false, lane);
+      step_pre<NB, G, STEP, FACT, false>(J0, W0, h0, false, q0, false, lane);
+      if (j0) split_drift<NB, G, WAVE, FACT>(J0, 0.5 * h0, lane);
+      if constexpr (TWO) {
+        step_pre<NB, G, STEP, FACT, false>(J1, W0, h1, false, q1, false, lane);
+        if (j1) split_drift<NB, G, WAVE, FACT>(J1, 0.5 * h1, lane);
+      }
     }
+    wsync();
     if (!split_sweep<NB, G, TWO, LIMIT, FACT>(P, F, 0, 0.5 * h0, 0.5 * h1, n0, n1, lane)) return;
     if (!wait_for(&ctl->sent, seen + 1, ctl, bound, err, lane)) return;
     for (int q = lane; q < N3; q += WAVE) {
@@ -943,25 +1447,30 @@ __device__ void split_jacobian(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0
       {
         const bool hi = lane >= 32;
         if (hi ? (j1 || q1) : (j0 || q0))
-          phisalpha_cols<NB, G, 32, FACT, false>(hi ? J1 : J0, hi ? W1 : W0, hi ? h1 : h0, false, hi ? q1 : q0, lane & 31);
+          split_phi<NB, 32, FACT>(hi ? J1 : J0, hi ? W1 : W0, hi ? h1 : h0, hi ? q1 : q0, lane & 31);
       }
       wsync();
       if constexpr (L::HALF) {
-        step_mid_rest<NB, G, 32, FACT>(sys ? J1 : J0, sys ? W1 : W0, sys ? j1 : j0, sys ? q1 : q0, col);
+        if (sys ? j1 : j0) split_vel_product<NB, G, 32, FACT>(sys ? J1 : J0, (sys ? W1 : W0).f.phi, col);
+        step_mid_rest<NB, G, 32, FACT>(sys ? J1 : J0, sys ? W1 : W0, false, sys ? q1 : q0, col);
       } else {
-        step_mid_rest<NB, G, WAVE, FACT>(J0, W0, j0, q0, lane);
-        step_mid_rest<NB, G, WAVE, FACT>(J1, W1, j1, q1, lane);
+        if (j0) split_vel_product<NB, G, WAVE, FACT>(J0, W0.f.phi, lane);
+        step_mid_rest<NB, G, WAVE, FACT>(J0, W0, false, q0, lane);
+        if (j1) split_vel_product<NB, G, WAVE, FACT>(J1, W1.f.phi, lane);
+        step_mid_rest<NB, G, WAVE, FACT>(J1, W1, false, q1, lane);
       }
     } else {
       if (j0 || q0) {
-        phisalpha_cols<NB, G, WAVE, FACT, false>(J0, W0, h0, false, q0, lane);
+        split_phi<NB, WAVE, FACT>(J0, W0, h0, q0, lane);
         wsync();
-        step_mid_rest<NB, G, WAVE, FACT>(J0, W0, j0, q0, lane);
+        if (j0) split_vel_product<NB, G, WAVE, FACT>(J0, W0.f.phi, lane);
+        step_mid_rest<NB, G, WAVE, FACT>(J0, W0, false, q0, lane);
       }
       if (TWO && (j1 || q1)) {
-        phisalpha_cols<NB, G, WAVE, FACT, false>(J1, W0, h1, false, q1, lane);
+        split_phi<NB, WAVE, FACT>(J1, W0, h1, q1, lane);
         wsync();
-        step_mid_rest<NB, G, WAVE, FACT>(J1, W0, j1, q1, lane);
+        if (j1) split_vel_product<NB, G, WAVE, FACT>(J1, W0.f.phi, lane);
+        step_mid_rest<NB, G, WAVE, FACT>(J1, W0, false, q1, lane);
       }
     }
     if (!split_sweep<NB, G, TWO, LIMIT, FACT>(P, F, 1, 0.5 * h0, 0.5 * h1, n0, n1, lane)) return;
@@ -973,11 +1482,17 @@ __device__ void split_jacobian(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0
     wsync();
     publish(&ctl->seen, ++seen, lane);
     if constexpr (L::HALF) {
-      step_post<NB, G, 32, FACT, false>(sys ? J1 : J0, W0, sys ? h1 : h0, sys ? j1 : j0, sys ? q1 : q0, false, col);
+      step_post<NB, G, 32, FACT, false>(sys ? J1 : J0, W0, sys ? h1 : h0, false, sys ? q1 : q0, false, col);
+      if (sys ? j1 : j0) split_drift<NB, G, 32, FACT>(sys ? J1 : J0, 0.5 * (sys ? h1 : h0), col);
     } else {
-      step_post<NB, G, STEP, FACT, false>(J0, W0, h0, j0, q0, false, lane);
-      if constexpr (TWO) step_post<NB, G, STEP, FACT, false>(J1, W0, h1, j1, q1, false, lane);
+      step_post<NB, G, STEP, FACT, false>(J0, W0, h0, false, q0, false, lane);
+      if (j0) split_drift<NB, G, WAVE, FACT>(J0, 0.5 * h0, lane);
+      if constexpr (TWO) {
+        step_post<NB, G, STEP, FACT, false>(J1, W0, h1, false, q1, false, lane);
+        if (j1) split_drift<NB, G, WAVE, FACT>(J1, 0.5 * h1, lane);
+      }
     }
+    wsync();
     publish(&ctl->answered, ++answered, lane);
     auto end = [&](JacRec<NB, G>& S, const SysDesc& D, int need, int body, int64_t index) {
       if (need & SPLIT_SAVE) {
