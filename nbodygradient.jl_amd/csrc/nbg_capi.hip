@@ -254,11 +254,11 @@ void group_layout(Layout& L) {
   }
 }
 
-// Whether a system may run on the two-wave launches: transit and plain runs
-// whose pairs are all Kepler pairs, none of them massless (such a pair reuses
+// Whether a system may run on the two-wave launches: transit, plain and
+// trajectory runs whose pairs are all Kepler pairs, none of them massless (such a pair reuses
 // the one before it, which keeps the sequential order).
 int split_ok(const nbg::SysDesc& d, const double* m) {
-  if ((d.mode != nbg::MODE_TRANSITS && d.mode != nbg::MODE_STEPS) || d.any_kick) return 0;
+  if (d.mode == nbg::MODE_SNAPSHOT || d.any_kick) return 0;
   for (int i = 0; i < d.n - 1; ++i)
     for (int j = i + 1; j < d.n; ++j)
       if (nbg::NBG_GNEWT * (m[i] + m[j]) == 0.0) return 0;

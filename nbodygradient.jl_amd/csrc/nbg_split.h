@@ -211,7 +211,7 @@ struct SplitCtl {
   int quit;           // the state wave is done, or a wait ran out
   int act[2];         // PRE: what the step is
   int body[2];        // PRE: a gradient step's body ...
-  int64_t index[2];   // ... and transit
+  int64_t index[2];   // ... and transit (else the step's number)
   double h[2];
 };
 
@@ -222,7 +222,7 @@ template <int NB, bool G, bool TWO, int LIMIT> struct SplitLds {
                                   sizeof(Schedule<NB>) + 64;
   static constexpr int NP = NB * (NB - 1) / 2;
   static constexpr int RMIN = NB / 2 < 1 ? 1 : NB / 2;
-  using Work = JacWork<NB, (LIMIT > 100000 ? 20 : NB <= 4 ? 6 : 1)>;
+  using Work = JacWork<NB, (NB <= 4 ? 6 : 1)>;
   // two work areas where they fit: both systems' force gradients at once
   static constexpr bool PHI2 = TWO && 4 * NB <= 32 && NP <= 32 &&
                                FIXED + 2 * sizeof(Work) + 2 * RMIN * sizeof(RingSlot) <= (size_t)LIMIT;
@@ -526,6 +526,41 @@ template <int NB> __device__ void split_record(StateRec<NB>& S, const SysDesc& D
   }
 }
 
+// The state before step k of a MODE_CARTESIAN run (write_snapshot's part
+// without the Jacobian).
+template <int NB> __device__ void split_write_state(const StateRec<NB>& S, const SysDesc& D, const SysBufs& B, int64_t k, int lane) {
+  constexpr int N3 = 3 * NB;
+  const int64_t ns = D.nsteps;
+  double* base = B.traj + D.off_traj;
+  if (lane == 0) base[k] = (k == 0) ? D.t0 : D.t0 + (D.h * (double)k);  // s.t[1] = t0 + (h * i)
+  for (int q = lane; q < N3; q += WAVE) {
+    base[traj_off_x(NB, ns) + N3 * k + q] = S.x[q];
+    base[traj_off_v(NB, ns) + N3 * k + q] = S.v[q];
+    if (D.traj & TRAJ_ERR) {
+      base[traj_off_xe(NB, ns) + N3 * k + q] = S.xe[q];
+      base[traj_off_ve(NB, ns) + N3 * k + q] = S.ve[q];
+    }
+  }
+}
+// ... and the Jacobian's part: column-major matrices, an element a lane; the
+// mass rows are unit rows of jac_step and zero rows of jac_error.
+template <int NB, class R> __device__ void split_write_jac(R& S, const SysDesc& D, const SysBufs& B, int64_t k, int lane) {
+  constexpr int N7 = 7 * NB, NN = N7 * N7;
+  const auto J_ = jj<NB>(S);
+  double* base = B.traj + D.off_traj;
+  for (int w = 0; w < 2; ++w) {
+    if (!(D.traj & (w ? TRAJ_JACERR : TRAJ_JAC))) continue;
+    double* o = base + (w ? traj_off_jacerr(NB, D.nsteps, D.traj) : traj_off_jac(NB, D.nsteps, D.traj)) + (int64_t)NN * k;
+#pragma unroll 4
+    for (int e = lane; e < NN; e += WAVE) {
+      const int c = e / N7, r = e - N7 * c, b = r / 7, kk = r - 7 * b;
+      double v = w == 0 && c == r ? 1.0 : 0.0;
+      if (kk < 6) v = J_[(unsigned)((w ? R::JOFF : 0) + (6 * b + kk) * N7 + c)];
+      o[e] = v;
+    }
+  }
+}
+
 // After the cursor's step (cursor_finish).  J: the Jacobian wave's record,
 // whose dq/dt is complete for a Newton step.
 template <int NB, class R>
@@ -622,10 +657,9 @@ __device__ inline Visit visit_of(const SysDesc& D, const SysBufs& B, int64_t chu
   return v;
 }
 
-template <int NB, bool G, bool TWO, int LIMIT>
-__device__ void split_state(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0, const SysDesc& D1, const SysBufs& B,
+template <int NB, bool TWO, class L>
+__device__ void split_state(L& P, const SysDesc& D0, const SysDesc& D1, const SysBufs& B,
                             const Visit& v0, const Visit& v1, int lane, int64_t bound, unsigned long long* err) {
-  using L = SplitLds<NB, G, TWO, LIMIT>;
   constexpr int N3 = 3 * NB, NP = L::NP, K = TWO ? 1 : 0;
   constexpr int STEP = TWO && N3 <= 32 ? 32 : WAVE;
   SplitCtl* ctl = &P.ctl;
@@ -652,6 +686,8 @@ __device__ void split_state(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0, c
     int n0 = ACT_DONE, n1 = ACT_DONE;
     if (a0) split_prepare<NB>(P.t[0], D0, c[0], h0, n0, lane);
     if (a1) split_prepare<NB>(P.t[K], D1, c[1], h1, n1, lane);
+    if (D0.mode == MODE_CARTESIAN && a0) split_write_state<NB>(P.t[0], D0, B, c[0].is, lane);
+    if (TWO && D1.mode == MODE_CARTESIAN && a1) split_write_state<NB>(P.t[K], D1, B, c[1].is, lane);
     const bool keep = ((n0 | n1) & (SPLIT_J | SPLIT_Q)) != 0;
     if (keep) {
       // PRE; its buffers are free once the message three before it is copied
@@ -661,8 +697,8 @@ __device__ void split_state(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0, c
         if (n1 & SPLIT_Q) P.j[K].mv[q] = P.t[K].v[q];
       }
       if (lane == 0) {
-        ctl->act[0] = n0; ctl->h[0] = h0; ctl->body[0] = c[0].jb; ctl->index[0] = n0 & SPLIT_SAVE ? P.t[0].count[c[0].jb] - 1 : 0;
-        ctl->act[1] = n1; ctl->h[1] = h1; ctl->body[1] = c[1].jb; ctl->index[1] = n1 & SPLIT_SAVE ? P.t[K].count[c[1].jb] - 1 : 0;
+        ctl->act[0] = n0; ctl->h[0] = h0; ctl->body[0] = c[0].jb; ctl->index[0] = n0 & SPLIT_SAVE ? P.t[0].count[c[0].jb] - 1 : c[0].is;
+        ctl->act[1] = n1; ctl->h[1] = h1; ctl->body[1] = c[1].jb; ctl->index[1] = n1 & SPLIT_SAVE ? P.t[K].count[c[1].jb] - 1 : c[1].is;
       }
       wsync();
       publish(&ctl->sent, ++sent, lane);
@@ -1320,16 +1356,15 @@ template <int NB, class R> __device__ void split_keep_jac(R& S, double* ws, bool
     }
 }
 
-// The dt/dq rows of a transit (cursor_record), from the final state of its
-// gradient step in the record.
+// The dt/dq rows of a transit (cursor_record) from the final state of its
+// gradient step: its dg/dt, the sky separation and velocity, and the
+// velocity's rate of change.
 template <int NB, class R>
-__device__ void split_gradient(R& S, const SysDesc& D, const SysBufs& B, int jb, int64_t cc, int lane) {
+__device__ void split_gradient_rows(R& S, const SysDesc& D, const SysBufs& B, int jb, int64_t cc, double gd, double dx, double dy,
+                                    double dvx, double dvy, double ax, double ay, int lane) {
   constexpr int N7 = 7 * NB;
   const int n = NB, ti = D.ti, nb = D.ntbv;
   const auto J_ = jj<NB>(S);
-  const double gd = gdot<NB>(S, ti, jb);
-  const double dx = S.x[3 * jb] - S.x[3 * ti], dy = S.x[3 * jb + 1] - S.x[3 * ti + 1];
-  const double dvx = S.v[3 * jb] - S.v[3 * ti], dvy = S.v[3 * jb + 1] - S.v[3 * ti + 1];
   double* dq = B.dq + D.off_dq;
   const int64_t ntt = D.ntt;
   for (int col = lane; col < N7; col += WAVE) {
@@ -1341,12 +1376,18 @@ __device__ void split_gradient(R& S, const SysDesc& D, const SysBufs& B, int jb,
     dq[0 + nb * base] = d0;
     if (nb == 3) {
       const double vsky = __builtin_sqrt(dvx * dvx + dvy * dvy);
-      const double dvdt = (dvx * (S.dqdt[7 * jb + 3] - S.dqdt[7 * ti + 3]) +
-                           dvy * (S.dqdt[7 * jb + 4] - S.dqdt[7 * ti + 4])) / vsky;
+      const double dvdt = (dvx * ax + dvy * ay) / vsky;
       dq[1 + nb * base] = (jvx * dvx + jvy * dvy) / vsky + dvdt * d0;
       dq[2 + nb * base] = 2.0 * (jx * dx + jy * dy);
     }
   }
+}
+template <int NB, class R>
+__device__ void split_gradient(R& S, const SysDesc& D, const SysBufs& B, int jb, int64_t cc, int lane) {
+  const int ti = D.ti;
+  split_gradient_rows<NB>(S, D, B, jb, cc, gdot<NB>(S, ti, jb), S.x[3 * jb] - S.x[3 * ti], S.x[3 * jb + 1] - S.x[3 * ti + 1],
+                          S.v[3 * jb] - S.v[3 * ti], S.v[3 * jb + 1] - S.v[3 * ti + 1], S.dqdt[7 * jb + 3] - S.dqdt[7 * ti + 3],
+                          S.dqdt[7 * jb + 4] - S.dqdt[7 * ti + 4], lane);
 }
 
 template <int NB, bool G> __device__ void split_load_jac(JacRec<NB, G>& S, const SysDesc& D, const SysBufs& B, int lane) {
@@ -1421,6 +1462,8 @@ __device__ void split_jacobian(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0
     }
     wsync();
     publish(&ctl->seen, ++seen, lane);
+    if (D0.mode == MODE_CARTESIAN && j0) split_write_jac<NB>(J0, D0, B, i0, lane);
+    if (TWO && D1.mode == MODE_CARTESIAN && j1) split_write_jac<NB>(J1, D1, B, i1, lane);
     if (n0 & SPLIT_SAVE) split_keep_jac<NB>(J0, B.ws + D0.off_ws, false, lane);
     if (n1 & SPLIT_SAVE) split_keep_jac<NB>(J1, B.ws + D1.off_ws, false, lane);
     if constexpr (L::HALF) {
@@ -1514,16 +1557,240 @@ __device__ void split_jacobian(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0
   }
 }
 
-// calc_dtdelements! (dtdelements) of a finished system, both waves at work:
-// wave w takes the transits w, w + 2, ...; jac_init staged transposed in the
+// ---------------------------------------------------------------------------
+// Three waves (few systems, SplitLds3): the Jacobian wave's work divided in
+// two again.  The pair wave turns the ring's slots into pair Jacobians, builds
+// Phi and carries dq/dt; the row wave follows with everything that touches J.
+// Newton's iterations need the first two only.  Between them: a chunk's pair
+// Jacobians in two buffers, Phi in one, a step's header and a transit's
+// scalars in two of each.  Cycles a step of the two Jacobian parts as one
+// wave: 299k at nine bodies (reference row update; 225k factored) and 64k at
+// three, with 210k and 42k for the state's wave beside it; divided, the
+// longest of the three is the state's or close to it.  80 gradient steps of
+// nine bodies 10.4 -> 8.0 ms, 150 of six with three observables 19.4 -> 11.8.
+// ---------------------------------------------------------------------------
+struct RowHeader {
+  int need, body;
+  int64_t index;
+  double h;
+  double gd, dx, dy, dvx, dvy, ax, ay;  // a gradient step's end (split_gradient)
+};
+struct RowCtl {
+  int chunks, chunks_done;  // published / released, of all sweeps so far
+  int phis, phis_done;
+  int heads, heads_seen;    // steps announced / read
+  int ends, steps_done;     // gradient scalars written; steps finished
+  RowHeader hdr[2];
+};
+
+template <int NB, int LIMIT> struct SplitLds3 {
+  static constexpr int NP = NB * (NB - 1) / 2, N3 = 3 * NB, N4 = 4 * NB, PQ = 13, NS = 1;
+  static constexpr int RR = NP;  // a whole sweep's ring
+  struct Phi {
+    double phi[N3 * N4];
+    double dadq[N3 * N4];
+    double pq[NP * PQ];
+  };
+  struct Work {
+    static constexpr int NP = SplitLds3::NP, PQ = SplitLds3::PQ;
+    Phi f;
+  };
+  static constexpr size_t FIXED = sizeof(StateRec<NB>) + sizeof(JacRec<NB, false>) + sizeof(Work) + RR * sizeof(RingSlot) +
+                                  sizeof(SplitCtl) + sizeof(RowCtl) + sizeof(Schedule<NB>) + 64;
+  static constexpr int FIT = (int)(((size_t)LIMIT - FIXED) / (2 * sizeof(JacSlot)));
+  // pairs per chunk: half a sweep or less, so that the waves overlap
+  static constexpr int CH0 = NP < 4 ? NP : (NP + 1) / 2 < 3 ? 3 : (NP + 1) / 2 > 18 ? 18 : (NP + 1) / 2;
+  static constexpr int CH = CH0 < FIT ? CH0 : FIT;
+  static_assert(FIXED < (size_t)LIMIT && CH >= (NB / 2 < 1 ? 1 : NB / 2), "a level of pairs must fit");
+  StateRec<NB> t[1];
+  JacRec<NB, false> j[1];
+  Work w;
+  JacSlot slot[2][CH];
+  RingSlot ring[1][RR];
+  SplitCtl ctl;
+  RowCtl row;
+  Schedule<NB> sched;
+};
+
+template <int NB, int LIMIT, bool FACT>
+__device__ __attribute__((always_inline)) inline bool pair_wave_sweep(SplitLds3<NB, LIMIT>& P, int& head, int& pos, int& chunk, int dir,
+                                                                      double hh, int need, int lane, int64_t bound,
+                                                                      unsigned long long* err) {
+  using L = SplitLds3<NB, LIMIT>;
+  constexpr int NL = Schedule<NB>::NL;
+  const uint8_t* lw = P.sched.width[dir];
+  const bool needJ = (need & SPLIT_J) != 0, needQ = (need & SPLIT_Q) != 0;
+  JacRec<NB, false>& S = P.j[0];
+  int lev = 0;
+  while (lev < NL) {
+    int cnt = 0;
+    while (lev < NL && cnt + lw[lev] <= L::CH) cnt += lw[lev++];
+    if (!wait_for(&P.ctl.tail, head + cnt, &P.ctl, bound, err, lane)) return false;
+    // the buffer the row wave used two chunks ago
+    if (!wait_for(&P.row.chunks_done, chunk - 1, &P.ctl, bound, err, lane)) return false;
+    JacSlot* slots = P.slot[chunk & 1];
+    if (lane < cnt) {
+      int at = pos + lane;
+      if (at >= L::RR) at -= L::RR;
+      const RingSlot* a = &P.ring[0][at];
+      if (dir == 0) split_pair_jacobian<true>(lds_off(a), lds_off(slots + lane), S.m[a->i], S.m[a->j], hh, FACT);
+      else split_pair_jacobian<false>(lds_off(a), lds_off(slots + lane), S.m[a->i], S.m[a->j], hh, FACT);
+    }
+    wsync();
+    head += cnt;
+    pos += cnt;
+    if (pos >= L::RR) pos -= L::RR;
+    publish(&P.ctl.head, head, lane);
+    if (needJ) publish(&P.row.chunks, ++chunk, lane);
+    if (needQ) split_rows<NB, false, WAVE, FACT>(S, slots, cnt, false, true, lane);
+  }
+  return true;
+}
+
+template <int NB, int LIMIT, bool FACT>
+__device__ void pair_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBufs& B, const Visit& v, int lane, int64_t bound,
+                          int64_t bound_job, unsigned long long* err) {
+  constexpr int N3 = 3 * NB, N7 = 7 * NB;
+  SplitCtl* ctl = &P.ctl;
+  RowCtl* row = &P.row;
+  JacRec<NB, false>& S = P.j[0];
+  int seen = 0, answered = 0, head = 0, pos = 0, chunk = 0, steps = 0;  // steps: announced to the row wave
+#pragma unroll 1
+  while (true) {
+    if (!wait_for(&ctl->sent, seen + 1, ctl, bound_job, err, lane)) return;
+    const int need = __builtin_amdgcn_readfirstlane(ctl->act[0]);
+    const bool needJ = need >= 0 && (need & SPLIT_J) != 0, needQ = need >= 0 && (need & SPLIT_Q) != 0;
+    const double h = ctl->h[0];
+    const int body = ctl->body[0];
+    const int64_t index = ctl->index[0];
+    if (needJ || need < 0) {
+      if (!wait_for(&row->heads_seen, steps - 1, ctl, bound, err, lane)) return;
+      RowHeader& H = row->hdr[steps & 1];
+      if (lane == 0) {
+        H.need = need;
+        H.body = body;
+        H.index = index;
+        H.h = h;
+      }
+      wsync();
+      publish(&row->heads, ++steps, lane);
+    }
+    if (need < 0) break;
+    if (needQ)
+      for (int q = lane; q < N3; q += WAVE) S.v[q] = S.mv[q];
+    wsync();
+    publish(&ctl->seen, ++seen, lane);
+    step_pre<NB, false, WAVE, FACT, false>(S, P.w, h, false, needQ, false, lane);
+    if (!pair_wave_sweep<NB, LIMIT, FACT>(P, head, pos, chunk, 0, 0.5 * h, need, lane, bound, err)) return;
+    if (!wait_for(&ctl->sent, seen + 1, ctl, bound, err, lane)) return;
+    for (int q = lane; q < N3; q += WAVE) S.x[q] = S.mx[q];
+    wsync();
+    publish(&ctl->seen, ++seen, lane);
+    // Phi of the last step that had one for the row wave is used up
+    if (!wait_for(&row->phis_done, needJ ? steps - 1 : steps, ctl, bound, err, lane)) return;
+    split_phi<NB, WAVE, FACT>(S, P.w, h, needQ, lane);
+    wsync();
+    if (needJ) publish(&row->phis, steps, lane);
+    step_mid_rest<NB, false, WAVE, FACT>(S, P.w, false, needQ, lane);
+    if (!pair_wave_sweep<NB, LIMIT, FACT>(P, head, pos, chunk, 1, 0.5 * h, need, lane, bound, err)) return;
+    if (!wait_for(&ctl->sent, seen + 1, ctl, bound, err, lane)) return;
+    if (needQ)
+      for (int q = lane; q < N3; q += WAVE) {
+        S.x[q] = S.qx[q];
+        S.v[q] = S.qv[q];
+      }
+    wsync();
+    publish(&ctl->seen, ++seen, lane);
+    step_post<NB, false, WAVE, FACT, false>(S, P.w, h, false, needQ, false, lane);
+    publish(&ctl->answered, ++answered, lane);
+    if (need & SPLIT_SAVE) {
+      const int ti = D.ti, jb = body;
+      RowHeader& H = row->hdr[(steps - 1) & 1];
+      if (lane == 0) {
+        H.gd = gdot<NB>(S, ti, jb);
+        H.dx = S.x[3 * jb] - S.x[3 * ti];
+        H.dy = S.x[3 * jb + 1] - S.x[3 * ti + 1];
+        H.dvx = S.v[3 * jb] - S.v[3 * ti];
+        H.dvy = S.v[3 * jb + 1] - S.v[3 * ti + 1];
+        H.ax = S.dqdt[7 * jb + 3] - S.dqdt[7 * ti + 3];
+        H.ay = S.dqdt[7 * jb + 4] - S.dqdt[7 * ti + 4];
+      }
+      wsync();
+      publish(&row->ends, steps, lane);
+    } else if ((need & 3) == ACT_MAIN && needQ) {
+      for (int q = lane; q < N7; q += WAVE) S.run_dqdt[q] = S.dqdt[q];
+      wsync();
+    }
+  }
+}
+
+template <int NB, int LIMIT, bool FACT>
+__device__ void row_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBufs& B, const Visit& v, int lane, int64_t bound,
+                         int64_t bound_job, unsigned long long* err) {
+  using L = SplitLds3<NB, LIMIT>;
+  constexpr int NL = Schedule<NB>::NL;
+  SplitCtl* ctl = &P.ctl;
+  RowCtl* row = &P.row;
+  JacRec<NB, false>& S = P.j[0];
+  int steps = 0, chunk = 0;
+#pragma unroll 1
+  while (true) {
+    if (!wait_for(&row->heads, steps + 1, ctl, bound_job, err, lane)) return;
+    const RowHeader& H = row->hdr[steps & 1];
+    const int need = __builtin_amdgcn_readfirstlane(H.need);
+    if (need < 0) break;
+    const double h = H.h;
+    const int body = H.body;
+    const int64_t index = H.index;
+    ++steps;
+    // the header stays until the step's gradient scalars are read from it
+    if (!(need & SPLIT_SAVE)) publish(&row->heads_seen, steps, lane);
+    if (D.mode == MODE_CARTESIAN) split_write_jac<NB>(S, D, B, index, lane);
+    if (need & SPLIT_SAVE) split_keep_jac<NB>(S, B.ws + D.off_ws, false, lane);
+    split_drift<NB, false, WAVE, FACT>(S, 0.5 * h, lane);
+    wsync();
+#pragma unroll 1
+    for (int dir = 0; dir < 2; ++dir) {
+      const uint8_t* lw = P.sched.width[dir];
+      int lev = 0;
+      while (lev < NL) {
+        int cnt = 0;
+        while (lev < NL && cnt + lw[lev] <= L::CH) cnt += lw[lev++];
+        if (!wait_for(&row->chunks, chunk + 1, ctl, bound, err, lane)) return;
+        split_rows<NB, false, WAVE, FACT>(S, P.slot[chunk & 1], cnt, true, false, lane);
+        publish(&row->chunks_done, ++chunk, lane);
+      }
+      if (dir == 0) {
+        if (!wait_for(&row->phis, steps, ctl, bound, err, lane)) return;
+        split_vel_product<NB, false, WAVE, FACT>(S, P.w.f.phi, lane);
+        wsync();
+        publish(&row->phis_done, steps, lane);
+      }
+    }
+    split_drift<NB, false, WAVE, FACT>(S, 0.5 * h, lane);
+    wsync();
+    if (need & SPLIT_SAVE) {
+      if (!wait_for(&row->ends, steps, ctl, bound, err, lane)) return;
+      const RowHeader G = H;
+      split_gradient_rows<NB>(S, D, B, body, index, G.gd, G.dx, G.dy, G.dvx, G.dvy, G.ax, G.ay, lane);
+      split_keep_jac<NB>(S, B.ws + D.off_ws, true, lane);
+      wsync();
+      publish(&row->heads_seen, steps, lane);
+    }
+  }
+  if (v.begin <= D.nsteps) split_store_jac<NB, false>(S, D, B, lane);
+}
+
+// calc_dtdelements! (dtdelements) of a finished system, all NWV waves at work:
+// wave w takes the transits w, w + NWV, ...; jac_init staged transposed in the
 // Jacobian's store (the Jacobian is already stored).
-template <int NB, class L> __device__ void split_elements(L& P, int k, const SysDesc& D, const SysBufs& B, int wave, int lane) {
+template <int NB, int NWV, class L> __device__ void split_elements(L& P, int k, const SysDesc& D, const SysBufs& B, int wave, int lane) {
   constexpr int N7 = 7 * NB;
   const int n = NB, nb = D.ntbv;
   const auto jt = jj<NB>(P.j[k]);
   const double* jinit = B.jac + D.off_jac + 2 * (int64_t)N7 * N7;
   for (int col = lane; col < N7; col += WAVE)
-    for (int cp = wave; cp < N7; cp += 2) jt[(unsigned)(col + N7 * cp)] = jinit[cp + (int64_t)N7 * col];
+    for (int cp = wave; cp < N7; cp += NWV) jt[(unsigned)(col + N7 * cp)] = jinit[cp + (int64_t)N7 * col];
   __syncthreads();
   const double* dq = B.dq + D.off_dq;
   double* del = B.del + D.off_del;
@@ -1532,8 +1799,10 @@ template <int NB, class L> __device__ void split_elements(L& P, int k, const Sys
   for (int b = 0; b < nb; ++b)
     for (int i = 0; i < n; ++i) {
       const int64_t cnt = P.t[k].count[i] < ntt ? P.t[k].count[i] : ntt;
-      for (int64_t t = 0; t < cnt; ++t, turn ^= 1) {
-        if (turn != wave) continue;
+      for (int64_t t = 0; t < cnt; ++t) {
+        const bool mine = turn == wave;
+        turn = turn + 1 < NWV ? turn + 1 : 0;
+        if (!mine) continue;
         for (int col = lane; col < N7; col += WAVE) {
           double acc = 0.0;
           for (int cp = 0; cp < N7; ++cp)
@@ -1542,6 +1811,55 @@ template <int NB, class L> __device__ void split_elements(L& P, int k, const Sys
         }
       }
     }
+}
+
+// Whether a run ever needs the Jacobian wave.
+__device__ inline bool split_follows(const SysDesc& D) { return D.grad || D.mode == MODE_TRANSITS; }
+
+// One visit of a system by a workgroup of three waves.
+template <int NB, int LIMIT>
+__device__ void split_run3(unsigned char* raw, int wave, const SysDesc& D, const SysBufs& B, int64_t chunk, int64_t bound,
+                           int64_t bound_job, unsigned long long* err, int lane) {
+  using L = SplitLds3<NB, LIMIT>;
+  L& P = *reinterpret_cast<L*>(raw);
+  static_assert(sizeof(L) <= (size_t)LIMIT, "LDS");
+  const Visit v = visit_of(D, B, chunk), none{1, 1, 0};
+  if (wave == 0) {
+    split_load_state<NB>(P.t[0], D, B, lane);
+    for (int w = lane; w < (int)(sizeof(SplitCtl) / 4); w += WAVE) reinterpret_cast<int*>(&P.ctl)[w] = 0;
+    for (int w = lane; w < (int)(sizeof(RowCtl) / 4); w += WAVE) reinterpret_cast<int*>(&P.row)[w] = 0;
+  } else if (wave == 1) {
+    for (int w = lane; w < (int)sizeof(Schedule<NB>); w += WAVE)
+      reinterpret_cast<uint8_t*>(&P.sched)[w] = reinterpret_cast<const uint8_t*>(&kSchedule<NB>)[w];
+  } else {
+    split_load_jac<NB, false>(P.j[0], D, B, lane);
+  }
+  __syncthreads();
+  if (wave == 0) {
+    split_state<NB, false>(P, D, D, B, v, none, lane, bound, err);
+  } else if (split_follows(D)) {
+    if (wave == 1) {
+      if (D.rowupd) pair_wave<NB, LIMIT, true>(P, D, B, v, lane, bound, bound_job, err);
+      else pair_wave<NB, LIMIT, false>(P, D, B, v, lane, bound, bound_job, err);
+    } else {
+      if (D.rowupd) row_wave<NB, LIMIT, true>(P, D, B, v, lane, bound, bound_job, err);
+      else row_wave<NB, LIMIT, false>(P, D, B, v, lane, bound, bound_job, err);
+    }
+  }
+  __syncthreads();  // every row is written
+  if (D.mode == MODE_TRANSITS && D.grad && v.begin <= D.nsteps && v.end == v.total) split_elements<NB, 3>(P, 0, D, B, wave, lane);
+  __syncthreads();
+}
+template <int N, int HI, int LIMIT>
+__device__ __forceinline__ void split_dispatch3(unsigned char* raw, int wave, const SysDesc& D, const SysBufs& B, int64_t chunk,
+                                                int64_t bound, int64_t bound_job, unsigned long long* err, int lane) {
+  if constexpr (N <= HI) {
+    if (D.n == N) {
+      split_run3<N, LIMIT>(raw, wave, D, B, chunk, bound, bound_job, err, lane);
+      return;
+    }
+    split_dispatch3<N + 1, HI, LIMIT>(raw, wave, D, B, chunk, bound, bound_job, err, lane);
+  }
 }
 
 // One visit of a system, or of two of equal body count, by a workgroup of two
@@ -1566,16 +1884,16 @@ __device__ void split_run(unsigned char* raw, int wave, const SysDesc& D0, const
   }
   __syncthreads();
   if (wave == 0) {
-    split_state<NB, G, TWO, LIMIT>(P, D0, D1, B, v0, v1, lane, bound, err);
-  } else if (D0.grad || D0.mode == MODE_TRANSITS || (pair && (D1.grad || D1.mode == MODE_TRANSITS))) {
+    split_state<NB, TWO>(P, D0, D1, B, v0, v1, lane, bound, err);
+  } else if (split_follows(D0) || (pair && split_follows(D1))) {
     if (D0.rowupd) split_jacobian<NB, G, TWO, LIMIT, true>(P, D0, D1, B, v0, v1, lane, bound, bound_job, err);
     else split_jacobian<NB, G, TWO, LIMIT, false>(P, D0, D1, B, v0, v1, lane, bound, bound_job, err);
   }
   __syncthreads();  // every row is written
   if (D0.mode == MODE_TRANSITS && D0.grad && v0.begin <= D0.nsteps && v0.end == v0.total)
-    split_elements<NB>(P, 0, D0, B, wave, lane);
+    split_elements<NB, 2>(P, 0, D0, B, wave, lane);
   if (TWO && D1.mode == MODE_TRANSITS && D1.grad && v1.begin <= D1.nsteps && v1.end == v1.total)
-    split_elements<NB>(P, L::NS - 1, D1, B, wave, lane);
+    split_elements<NB, 2>(P, L::NS - 1, D1, B, wave, lane);
   __syncthreads();
 }
 
@@ -1603,7 +1921,7 @@ __device__ __forceinline__ void split_dispatch(unsigned char* raw, int wave, con
 // Persistent two-wave launch of bodies up to HI: like nbg_run (TWO: like
 // nbg_run_duo, one unit of one or two systems at a time).  LIMIT: the
 // workgroup's LDS.  units[13] collects wait failures.
-template <int HI, bool TWO, int LIMIT>
+template <int HI, bool TWO, int LIMIT, bool THREE = false>
 __device__ __forceinline__ void split_body(unsigned char* raw, int* share, const GroupList& gl, const SysBufs& B, int64_t chunk,
                                            int64_t bound, int64_t bound_job, unsigned long long* units,
                                            unsigned long long* err) {
@@ -1636,7 +1954,8 @@ __device__ __forceinline__ void split_body(unsigned char* raw, int* share, const
     const int64_t before1 = ints1[D1.n], tr01 = ints1[D1.n + 1], it01 = ints1[D1.n + 2];
     const int64_t c0 = D0.chunk > 0 ? D0.chunk : chunk, c1 = D1.chunk > 0 ? D1.chunk : chunk;
     __syncthreads();  // both waves have read the counters
-    split_dispatch<2, HI, TWO, LIMIT>(raw, wave, D0, D1, B, c0, c1, two, bound, bound_job, err, lane);
+    if constexpr (THREE) split_dispatch3<2, HI, LIMIT>(raw, wave, D0, B, c0, bound, bound_job, err, lane);
+    else split_dispatch<2, HI, TWO, LIMIT>(raw, wave, D0, D1, B, c0, c1, two, bound, bound_job, err, lane);
     if (threadIdx.x == 0) {
       visit_done(D0, ints0, before0, tr00, it00, B, units);
       if (two) visit_done(D1, ints1, before1, tr01, it01, B, units);

@@ -1,25 +1,24 @@
-// nbg_split_wide.hip -- two-wave launch for few systems (nbg_split.h): one
-// workgroup a compute unit, its two waves on different SIMDs with all their
+// nbg_split_wide.hip -- three-wave launch for few systems (nbg_split.h): one
+// workgroup a compute unit, its waves on different SIMDs with all their
 // registers, the Jacobian in LDS at every body count.
 #include "nbg_split.h"
 
 namespace nbg {
 
 template <int HI, int LIMIT>
-__global__ __launch_bounds__(2 * WAVE, 1) void nbg_run_split_wide(GroupList gl, SysBufs B, int64_t chunk, int64_t bound, int64_t bound_job,
+__global__ __launch_bounds__(3 * WAVE, 1) void nbg_run_split_wide(GroupList gl, SysBufs B, int64_t chunk, int64_t bound, int64_t bound_job,
                                                                   unsigned long long* __restrict__ units,
                                                                   unsigned long long* __restrict__ err) {
-  static_assert(!split_global<HI, false, LIMIT>(), "the Jacobian must fit in LDS");
   __shared__ __attribute__((aligned(16))) unsigned char raw[LIMIT];
   __shared__ int share;
-  split_body<HI, false, LIMIT>(raw, &share, gl, B, chunk, bound, bound_job, units, err);
+  split_body<HI, false, LIMIT, true>(raw, &share, gl, B, chunk, bound, bound_job, units, err);
 }
 
 }  // namespace nbg
 
 extern "C" hipError_t nbg_launch_split_wide(nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int64_t bound_job, int grid,
                                             unsigned long long* units, unsigned long long* err, hipStream_t stream) {
-  hipLaunchKernelGGL((nbg::nbg_run_split_wide<12, 163776>), dim3(grid), dim3(2 * nbg::WAVE), 0, stream, gl, bufs, chunk, bound,
+  hipLaunchKernelGGL((nbg::nbg_run_split_wide<12, 163776>), dim3(grid), dim3(3 * nbg::WAVE), 0, stream, gl, bufs, chunk, bound,
                      bound_job, units, err);
   return hipGetLastError();
 }
