@@ -62,6 +62,10 @@ extern "C" hipError_t nbg_launch_split_wide(nbg::GroupList gl, nbg::SysBufs bufs
 namespace {
 
 constexpr int NB_MIN = 2, NB_MAX = 12;
+// Polls of a wait between the waves of nbg_split.h before it is reported as
+// failed: for another wave's work, and for the next step.
+constexpr int64_t SPLIT_POLLS = (int64_t)1 << 24, SPLIT_JOB_POLLS = (int64_t)1 << 40;
+constexpr const char* WAIT_FAILED = "two-wave workgroup: a wait between its two waves timed out";
 constexpr int SPLIT_PAIR_MAX = 7;  // bodies of the largest systems paired on the two-wave launches
 
 template <class T> struct DevVec {
@@ -83,6 +87,41 @@ template <class T> struct DevVec {
     cap = 0;
   }
 };
+
+// A single run's record on the device and its pinned host mirror: grown as
+// runs need, at most to RUN_OUTPUT_MAX bytes and the 0.2 MB of the largest
+// system's state and Jacobians, and given back with the context.
+constexpr int64_t RUN_OUTPUT_MAX = 1 << 20;
+struct RunRecord {
+  unsigned char* dev = nullptr;
+  unsigned char* host = nullptr;
+  unsigned char* host_dev = nullptr;  // the mirror as kernels address it
+  int64_t cap = 0;
+  void release() {
+    if (dev) (void)hipFree(dev);
+    if (host) (void)hipHostFree(host);
+    dev = host = host_dev = nullptr;
+    cap = 0;
+  }
+  hipError_t ensure(int64_t bytes) {
+    if (bytes <= cap) return hipSuccess;
+    release();
+    void *d = nullptr, *h = nullptr, *a = nullptr;
+    hipError_t e = hipMalloc(&d, bytes);
+    if (e == hipSuccess) e = hipHostMalloc(&h, bytes, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostGetDevicePointer(&a, h, 0);
+    dev = static_cast<unsigned char*>(d);
+    host = static_cast<unsigned char*>(h);
+    host_dev = static_cast<unsigned char*>(a);
+    if (e == hipSuccess) cap = bytes;
+    else release();
+    return e;
+  }
+};
+// Moves 8-byte words between a run's record and its mirror.
+__global__ __launch_bounds__(256) void nbg_move_words(double* __restrict__ dst, const double* __restrict__ src, int64_t count) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x) dst[i] = src[i];
+}
 
 // Device storage of a set of systems.
 struct Store {
@@ -297,6 +336,7 @@ struct nbg_ctx {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t gev[2 * 16] = {};  // start/end of each body-count launch (timed on its own stream)
   Store single;  // reused by the single-system entry points
+  RunRecord rec;  // ... on the three-wave launch
   unsigned char* scratch_dev = nullptr;  // device address of `scratch` on this context's device
 };
 
@@ -403,8 +443,8 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
     if (!split[g] || paired[g]) wide = false;
   }
   bool any_split = false;
-  const int64_t split_bound = ctx->coop_polls > 0 ? ctx->coop_polls : (int64_t)1 << 24;
-  const int64_t split_job = ctx->coop_polls > 0 ? ctx->coop_polls : (int64_t)1 << 40;
+  const int64_t split_bound = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_POLLS;
+  const int64_t split_job = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_JOB_POLLS;
   unsigned long long* const wait_err = S.units.p + 13 * G + 13;
   NBG_HIP(hipEventRecord(ctx->ev0, 0));
   for (int s = 0; s < ns; ++s) NBG_HIP(hipStreamWaitEvent(ctx->streams[s], ctx->ev0, 0));
@@ -584,7 +624,7 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
     unsigned long long werr = 0;
     NBG_HIP(hipMemcpy(&werr, wait_err, sizeof(werr), hipMemcpyDeviceToHost));
     if (werr) {
-      ctx->err = "two-wave workgroup: a wait between its two waves timed out";
+      ctx->err = WAIT_FAILED;
       return -2;
     }
   }
@@ -656,6 +696,185 @@ struct TrajOut {
   double *vsky, *bsky2, *dbvdq0, *dbvdel;
 };
 
+// The trajectory records of a finished run, to the host.
+int fetch_trajectory(nbg_ctx* ctx, const nbg::SysDesc& D, const double* base, const TrajOut& o) {
+  const int64_t n = D.n, ns = D.nsteps;
+  const int f = D.traj;
+  auto get = [&](double* dst, int64_t off, int64_t len) -> int {
+    if (dst) NBG_HIP(hipMemcpy(dst, base + off, (size_t)len * sizeof(double), hipMemcpyDeviceToHost));
+    return 0;
+  };
+  const int64_t n3 = 3 * n * ns, nj = 49 * n * n * ns;
+  if (int rc = get(o.t, 0, ns)) return rc;
+  if (int rc = get(o.x, nbg::traj_off_x(n, ns), n3)) return rc;
+  if (int rc = get(o.v, nbg::traj_off_v(n, ns), n3)) return rc;
+  if (f & nbg::TRAJ_ERR) {
+    if (int rc = get(o.xe, nbg::traj_off_xe(n, ns), n3)) return rc;
+    if (int rc = get(o.ve, nbg::traj_off_ve(n, ns), n3)) return rc;
+  }
+  if (f & nbg::TRAJ_JAC)
+    if (int rc = get(o.jac, nbg::traj_off_jac(n, ns, f), nj)) return rc;
+  if (f & nbg::TRAJ_JACERR)
+    if (int rc = get(o.jace, nbg::traj_off_jacerr(n, ns, f), nj)) return rc;
+  return 0;
+}
+
+// A system on the three-wave launch, its record moved in and out by a kernel
+// each that read and write the pinned mirror, all on one stream with one wait.
+// A short run is the calls around it.  Transit outputs up to RUN_OUTPUT_MAX
+// bytes travel in the record: only the entries of recorded transits are
+// written by a run, so they need not be uploaded and only they are handed on;
+// larger ones are copied from and to the caller's arrays.
+int run_record(nbg_ctx* ctx, const Layout& L, double* x, double* v, double* xe, double* ve, const double* m, double* J,
+               double* JE, double* dqdt, const double* jinit, double* t, double* tt, double* dtdq0, double* dtdel,
+               int64_t* count, const TrajOut* traj) {
+  NBG_HIP(hipSetDevice(ctx->device));
+  nbg::SysDesc D = L.desc[0];
+  Store& S = ctx->single;
+  RunRecord& R = ctx->rec;
+  const int n = D.n, s7 = 7 * n;
+  const int64_t NN = (int64_t)s7 * s7;
+  const bool grad = D.grad != 0, transits = D.mode == nbg::MODE_TRANSITS;
+  const int64_t ntt_len = transits ? L.n_tt : 0, ndq = transits && grad ? L.n_dq : 0;
+  const bool staged = 8 * (ntt_len + 2 * ndq) <= RUN_OUTPUT_MAX;
+  // pieces in 8-byte words, each from a 128-byte line on; what goes in comes
+  // first, what comes out last
+  int64_t words = 0;
+  auto take = [&](int64_t k) {
+    const int64_t o = words;
+    words += (k + 15) / 16 * 16;
+    return o;
+  };
+  const int64_t o_desc = take((sizeof(nbg::SysDesc) + 7) / 8), o_queue = take(1), o_units = take(14);
+  const int64_t o_ints = take(nbg::int_len(n)), o_state = take(nbg::state_len(n));
+  const int64_t o_jac = take(grad ? (transits ? 3 : 2) * NN : 0), in_words = words;  // J, its error, jac_init
+  const int64_t o_tt = take(staged ? ntt_len : 0), o_dq = take(staged ? ndq : 0), o_del = take(staged ? ndq : 0);
+  NBG_HIP(R.ensure(8 * words));
+  NBG_HIP(S.ws.ensure(L.n_ws));
+  if (L.n_traj > 0) NBG_HIP(S.traj.ensure(L.n_traj));
+  double* H = reinterpret_cast<double*>(R.host);
+  double* V = reinterpret_cast<double*>(R.dev);
+  double* HV = reinterpret_cast<double*>(R.host_dev);
+  // each buffer pointer starts at its own piece
+  D.off_state = D.off_jac = D.off_ws = D.off_tt = D.off_dq = D.off_del = D.off_int = D.off_pair = D.off_traj = 0;
+  std::memset(H, 0, 8 * o_jac);
+  std::memcpy(H + o_desc, &D, sizeof(D));
+  double* st = H + o_state;
+  auto put = [](double* dst, const double* src, int64_t k) {
+    if (src) std::memcpy(dst, src, 8 * k);
+  };
+  put(st + nbg::off_x(n), x, 3 * n);
+  put(st + nbg::off_v(n), v, 3 * n);
+  put(st + nbg::off_xe(n), xe, 3 * n);
+  put(st + nbg::off_ve(n), ve, 3 * n);
+  put(st + nbg::off_m(n), m, n);
+  put(st + nbg::off_dqdt(n), dqdt, s7);
+  st[nbg::off_t(n)] = t ? *t : 0.0;
+  auto identity = [&](double* a) {
+    std::fill(a, a + NN, 0.0);
+    for (int q = 0; q < s7; ++q) a[(int64_t)q * (s7 + 1)] = 1.0;
+  };
+  if (grad) {
+    double* a = H + o_jac;
+    if (J) put(a, J, NN);
+    else identity(a);
+    if (JE) put(a + NN, JE, NN);
+    else std::fill(a + NN, a + 2 * NN, 0.0);
+    if (transits) {
+      if (jinit) put(a + 2 * NN, jinit, NN);
+      else identity(a + 2 * NN);
+    }
+  }
+  hipStream_t s = ctx->streams[0];
+  nbg::SysBufs B = bufs_of(S);
+  B.state = V + o_state;
+  B.jac = V + o_jac;
+  B.ints = reinterpret_cast<int64_t*>(V + o_ints);
+  B.pair = nullptr;  // Kepler pairs only
+  if (staged) {
+    B.tt = V + o_tt;
+    B.dq = V + o_dq;
+    B.del = V + o_del;
+  } else {
+    NBG_HIP(S.tt.ensure(ntt_len));
+    NBG_HIP(S.dq.ensure(ndq));
+    NBG_HIP(S.del.ensure(ndq));
+    B.tt = S.tt.p;
+    B.dq = S.dq.p;
+    B.del = S.del.p;
+    NBG_HIP(hipMemcpyAsync(B.tt, tt, 8 * ntt_len, hipMemcpyHostToDevice, s));
+    if (ndq) NBG_HIP(hipMemcpyAsync(B.dq, dtdq0, 8 * ndq, hipMemcpyHostToDevice, s));
+    if (ndq) NBG_HIP(hipMemcpyAsync(B.del, dtdel, 8 * ndq, hipMemcpyHostToDevice, s));
+  }
+  auto move = [&](double* dst, const double* src, int64_t k) {
+    const int grid = (int)std::min<int64_t>((k + 255) / 256, 256);
+    hipLaunchKernelGGL(nbg_move_words, dim3(grid), dim3(256), 0, s, dst, src, k);
+    return hipGetLastError();
+  };
+  nbg::GroupList gl{};
+  gl.rowupd = ctx->row_update;
+  gl.ng = 1;
+  gl.nsys[0] = 1;
+  gl.descs[0] = reinterpret_cast<const nbg::SysDesc*>(V + o_desc);
+  gl.queue[0] = reinterpret_cast<int*>(V + o_queue);
+  unsigned long long* units = reinterpret_cast<unsigned long long*>(V + o_units);
+  const int64_t bound = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_POLLS;
+  const int64_t job = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_JOB_POLLS;
+  NBG_HIP(move(V, HV, in_words));
+  NBG_HIP(nbg_launch_split_wide(gl, B, 0, bound, job, 1, units, units + 13, s));
+  NBG_HIP(move(HV + o_units, V + o_units, words - o_units));
+  NBG_HIP(hipStreamSynchronize(s));
+  unsigned long long werr = 0;
+  std::memcpy(&werr, H + o_units + 13, sizeof(werr));
+  if (werr) {
+    ctx->err = WAIT_FAILED;
+    return -2;
+  }
+  auto get = [](double* dst, const double* src, int64_t k) {
+    if (dst) std::memcpy(dst, src, 8 * k);
+  };
+  get(x, st + nbg::off_x(n), 3 * n);
+  get(v, st + nbg::off_v(n), 3 * n);
+  get(xe, st + nbg::off_xe(n), 3 * n);
+  get(ve, st + nbg::off_ve(n), 3 * n);
+  if (grad) {
+    get(J, H + o_jac, NN);
+    get(JE, H + o_jac + NN, NN);
+    get(dqdt, st + nbg::off_dqdt(n), s7);
+  }
+  if (D.mode == nbg::MODE_CARTESIAN && traj)
+    if (int rc = fetch_trajectory(ctx, D, S.traj.p, *traj)) return rc;
+  if (!transits) return 0;
+  if (t) *t = st[nbg::off_t(n)];
+  std::memcpy(count, H + o_ints, 8 * n);
+  if (!staged) {
+    NBG_HIP(hipMemcpyAsync(tt, B.tt, 8 * ntt_len, hipMemcpyDeviceToHost, s));
+    if (ndq) NBG_HIP(hipMemcpyAsync(dtdq0, B.dq, 8 * ndq, hipMemcpyDeviceToHost, s));
+    if (ndq) NBG_HIP(hipMemcpyAsync(dtdel, B.del, 8 * ndq, hipMemcpyDeviceToHost, s));
+    NBG_HIP(hipStreamSynchronize(s));
+    return 0;
+  }
+  // entries of transit k < count of each body; ntbv of them together, then
+  // the bodies, the transits, and (gradients) the columns
+  const int nb = D.ntbv;
+  const int64_t ntt = D.ntt;
+  auto entries = [&](double* dst, const double* src, int64_t cols) {
+    for (int64_t c = 0; c < cols; ++c)
+      for (int64_t k = 0; k < ntt; ++k)
+        for (int i = 0; i < n; ++i)
+          if (k < count[i]) {
+            const int64_t e = nb * (i + n * (k + ntt * c));
+            for (int b = 0; b < nb; ++b) dst[e + b] = src[e + b];
+          }
+  };
+  entries(tt, H + o_tt, 1);
+  if (ndq) {
+    entries(dtdq0, H + o_dq, s7);
+    entries(dtdel, H + o_del, s7);
+  }
+  return 0;
+}
+
 // Run one system through the single-system store.
 int run_single(nbg_ctx* ctx, nbg::SysDesc d, double* x, double* v, double* xe, double* ve, const double* m,
                const uint8_t* pair, double* J, double* JE, double* dqdt, const double* jinit, double* t,
@@ -664,6 +883,9 @@ int run_single(nbg_ctx* ctx, nbg::SysDesc d, double* x, double* v, double* xe, d
   d.split = split_ok(d, m);
   L.desc.push_back(d);
   finalize_layout(L);
+  // a cooperative workgroup asked for takes transit runs (run_groups)
+  if (d.split && !(ctx->coop_mode == 2 && d.mode == nbg::MODE_TRANSITS))
+    return run_record(ctx, L, x, v, xe, ve, m, J, JE, dqdt, jinit, t, tt, dtdq0, dtdel, count, traj);
   const nbg::SysDesc& D = L.desc[0];
   HostRec R;
   pack_system(D, x, v, xe, ve, m, pair, J, JE, dqdt, jinit, t ? *t : 0.0, nullptr, nullptr, R);
@@ -719,26 +941,8 @@ int run_single(nbg_ctx* ctx, nbg::SysDesc d, double* x, double* v, double* xe, d
     if (traj->dbvdel)
       NBG_HIP(hipMemcpy(traj->dbvdel, base + nbg::snap_off_del(n, nt), nq * sizeof(double), hipMemcpyDeviceToHost));
   }
-  if (D.mode == nbg::MODE_CARTESIAN && traj) {
-    const int64_t ns = D.nsteps;
-    const int f = D.traj;
-    auto get = [&](double* dst, int64_t off, int64_t len) -> int {
-      if (dst) NBG_HIP(hipMemcpy(dst, S.traj.p + D.off_traj + off, (size_t)len * sizeof(double), hipMemcpyDeviceToHost));
-      return 0;
-    };
-    const int64_t n3 = 3 * (int64_t)n * ns, nj = 49 * (int64_t)n * n * ns;
-    if (int rc = get(traj->t, 0, ns)) return rc;
-    if (int rc = get(traj->x, nbg::traj_off_x(n, ns), n3)) return rc;
-    if (int rc = get(traj->v, nbg::traj_off_v(n, ns), n3)) return rc;
-    if (f & nbg::TRAJ_ERR) {
-      if (int rc = get(traj->xe, nbg::traj_off_xe(n, ns), n3)) return rc;
-      if (int rc = get(traj->ve, nbg::traj_off_ve(n, ns), n3)) return rc;
-    }
-    if (f & nbg::TRAJ_JAC)
-      if (int rc = get(traj->jac, nbg::traj_off_jac(n, ns, f), nj)) return rc;
-    if (f & nbg::TRAJ_JACERR)
-      if (int rc = get(traj->jace, nbg::traj_off_jacerr(n, ns, f), nj)) return rc;
-  }
+  if (D.mode == nbg::MODE_CARTESIAN && traj)
+    if (int rc = fetch_trajectory(ctx, D, S.traj.p + D.off_traj, *traj)) return rc;
   if (D.mode == nbg::MODE_TRANSITS) {
     if (t) *t = R.state[nbg::off_t(n)];
     for (int q = 0; q < n; ++q) count[q] = R.ints[q];
@@ -802,6 +1006,7 @@ void nbg_ctx_destroy(nbg_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   (void)hipDeviceSynchronize();
   ctx->single.release();
+  ctx->rec.release();
   for (auto& s : ctx->streams) (void)hipStreamDestroy(s);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
