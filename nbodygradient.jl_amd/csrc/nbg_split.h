@@ -23,8 +23,8 @@
 // Waits are bounded like those of nbg_run_coop: a failure ends both waves and
 // is reported, it never hangs.
 //
-// Systems with Kepler pairs only and no massless pair (their schedule of
-// levels is the same for every system of a body count); every operation is the
+// Systems with Kepler pairs only and no massless pair (the levels of their
+// sweeps are the same for every system of a body count); every operation is the
 // one-wave step's, so results are the same bits.
 #pragma once
 
@@ -34,48 +34,19 @@
 
 namespace nbg {
 
-// The level schedule of both sweeps of NB bodies, every pair a Kepler pair.
-template <int NB> struct Schedule {
-  static constexpr int NP = NB * (NB - 1) / 2, NL = 2 * NB - 3;
-  uint8_t pairs[2][2 * NP];
-  uint8_t width[2][NL];
-};
-template <int NB> constexpr Schedule<NB> make_schedule() {
-  Schedule<NB> s{};
-  constexpr int NP = Schedule<NB>::NP;
-  for (int dir = 0; dir < 2; ++dir) {
-    int pi[NP] = {}, pj[NP] = {}, lv[NP] = {}, last[NB] = {};
-    int np = 0;
-    if (dir == 0) {
-      for (int i = 0; i < NB - 1; ++i)
-        for (int j = i + 1; j < NB; ++j) { pi[np] = i; pj[np] = j; ++np; }
-    } else {
-      for (int i = NB - 2; i >= 0; --i)
-        for (int j = NB - 1; j >= i + 1; --j) { pi[np] = i; pj[np] = j; ++np; }
-    }
-    for (int p = 0; p < NP; ++p) {
-      const int a = last[pi[p]], b = last[pj[p]];
-      lv[p] = (a > b ? a : b) + 1;
-      last[pi[p]] = last[pj[p]] = lv[p];
-    }
-    int w = 0;
-    for (int l = 0; l < Schedule<NB>::NL; ++l)
-      for (int p = 0; p < NP; ++p)
-        if (lv[p] == l + 1) {
-          s.pairs[dir][2 * w] = (uint8_t)pi[p];
-          s.pairs[dir][2 * w + 1] = (uint8_t)pj[p];
-          ++w;
-          s.width[dir][l] += 1;
-        }
-  }
-  return s;
-}
-template <int NB> __device__ constexpr Schedule<NB> kSchedule = make_schedule<NB>();
+// The levels of a sweep over nb bodies whose pairs are all Kepler pairs.  In
+// lexicographic order pair (i, j) waits for (i, j - 1) and (i - 1, j) and no
+// others that are not already behind those, so level L has the pairs with
+// i + j = L + 1; the second sweep's order is the reverse, its levels too.
+// Widths read the same from either end.
+__host__ __device__ constexpr int level_count(int nb) { return 2 * nb - 3; }
+__host__ __device__ constexpr int level_first(int nb, int sum) { return sum - nb + 1 > 0 ? sum - nb + 1 : 0; }  // the smallest i
+__host__ __device__ constexpr int level_width(int nb, int level) { return level / 2 - level_first(nb, level + 1) + 1; }
 
 // What the state wave hands over of a pair's drift; the other quantities of
 // KParams and the drift itself follow from these.
 struct RingSlot {
-  double x0[3], v0[3];
+  double x0[3], v0[3];  // first
   double gamma, g1, g2, g3, h1, h2, r0, r, r0inv, rinv, beta, betainv, eta, sqb;
   double mijinv;
   int i, j;
@@ -218,8 +189,7 @@ struct SplitCtl {
 template <int NB, bool G, bool TWO, int LIMIT> struct SplitLds {
   static constexpr int NS = TWO ? 2 : 1;
   static constexpr bool HALF = TWO && 7 * NB <= 32 && !G;  // every stage on half-waves
-  static constexpr size_t FIXED = NS * (sizeof(StateRec<NB>) + sizeof(JacRec<NB, G>)) + sizeof(SplitCtl) +
-                                  sizeof(Schedule<NB>) + 64;
+  static constexpr size_t FIXED = NS * (sizeof(StateRec<NB>) + sizeof(JacRec<NB, G>)) + sizeof(SplitCtl) + 64;
   static constexpr int NP = NB * (NB - 1) / 2;
   static constexpr int RMIN = NB / 2 < 1 ? 1 : NB / 2;
   using Work = JacWork<NB, (NB <= 4 ? 6 : 1)>;
@@ -243,7 +213,6 @@ template <int NB, bool G, bool TWO, int LIMIT> struct SplitLds {
   Work w[NW];
   RingSlot ring[NS][RR];
   SplitCtl ctl;
-  Schedule<NB> sched;
 };
 
 __device__ __forceinline__ void publish(int* counter, int v, int lane) {
@@ -273,13 +242,19 @@ __device__ __forceinline__ bool wait_for(const int* counter, int v, SplitCtl* ct
 // ---------------------------------------------------------------------------
 // State wave
 // ---------------------------------------------------------------------------
-// A sweep of one system or two of equal body count (act: which have a step):
-// lanes [0, w) the first's pairs of a level, [w, 2w) the second's.  keep: the
-// Jacobian wave follows, so each level's pairs go to the ring once it has room.
-// One out-of-line copy per direction for every body count.
+// A sweep of one system or two of equal body count (act: which have a step).
+// A pair takes eight lanes: the first w groups of eight are the first system's
+// pairs of a level, the next w the second's.  All eight solve the pair's
+// Kepler problem alike (a wave pays for an instruction, not for its lanes);
+// then lane r < 6 moves coordinate r of the two bodies -- the positions' three,
+// the velocities' three -- in 20 instructions where one lane for all of them
+// took 110 and twice the LDS accesses (lanes 6 and 7 repeat 0 and 1).  keep:
+// the Jacobian wave follows, so each level's pairs go to the ring once it has
+// room.  One out-of-line copy per direction for every body count.
+constexpr int PAIR_LANES = 8;
 struct SplitSweep {
-  uint32_t x0, x1, ring0, ring1, pairs, width, ctl;
-  int n3, levels, act0, act1, keep, slots, pos, made;
+  uint32_t x0, x1, ring0, ring1, ctl;
+  int n, act0, act1, keep, slots, pos, made;
   double hh0, hh1;
   int64_t bound;
   unsigned long long* err;
@@ -287,53 +262,68 @@ struct SplitSweep {
 template <bool DF> static __device__ __attribute__((noinline)) bool split_levels(SplitSweep R) {
   const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
-  const int levels = uni(R.levels), n3 = uni(R.n3), slots = uni(R.slots);
+  const int n = uni(R.n), slots = uni(R.slots), n3 = 3 * n, levels = level_count(n);
   const bool a0 = uni(R.act0) != 0, a1 = uni(R.act1) != 0, keep = uni(R.keep) != 0;
   int pos = uni(R.pos), made = uni(R.made);
-  const uint8_t* lw = lds_at<uint8_t>(uni(R.width));
-  const uint8_t* pl = lds_at<uint8_t>(uni(R.pairs));
   SplitCtl* ctl = lds_at<SplitCtl>(uni(R.ctl));
-  // the next level's width and pairs are read while this one is solved
-  int q0 = 0, w = uni((int)lw[0]);
-  bool second = lane >= w;
-  int q = lane - (second ? w : 0);
-  bool on = lane < 2 * w && (second ? a1 : a0);
-  uint32_t ij = 0;
-  if (on) ij = pl[2 * q] | ((uint32_t)pl[2 * q + 1] << 8);
+  const int group = lane / PAIR_LANES, role = lane % PAIR_LANES < 6 ? lane % PAIR_LANES : lane % PAIR_LANES - 6;
+  const bool vel = role >= 3;
+  const int c = vel ? role - 3 : role, mine = vel ? n3 + c : c;
 #pragma unroll 1
   for (int L = 0; L < levels; ++L) {
-    const int w1 = L + 1 < levels ? (int)lw[L + 1] : 0;
+    const int sum = DF ? L + 1 : levels - L, w = level_width(n, sum - 1);
     if (keep && !wait_for(&ctl->head, made + w - slots, ctl, R.bound, R.err, lane)) return false;
-    if (on) {
-      const int i = ij & 0xff, j = ij >> 8;
-      double x0[3], v0[3], d[6], m_i, m_j, mijinv;
+    const bool second = group >= w;
+    const int q = second ? group - w : group;
+    if (q < w && (second ? a1 : a0)) {
+      const int i = level_first(n, sum) + q, j = sum - i;
+      double* x = lds_at<double>(second ? R.x1 : R.x0);
+      const double *bi = x + 3 * i, *bj = x + 3 * j;
+      const double hh = second ? R.hh1 : R.hh0;
+      // every LDS operand is read before anything is written back
+      double x0[3], v0[3];
+      for (int k = 0; k < 3; ++k) {
+        x0[k] = bi[k] - bj[k];
+        v0[k] = bi[n3 + k] - bj[n3 + k];
+      }
+      const double m_i = x[4 * n3 + i], m_j = x[4 * n3 + j];
+      const double x0c = bi[c] - bj[c], v0c = bi[n3 + c] - bj[n3 + c];
+      double si = bi[mine], sj = bj[mine], ei = bi[2 * n3 + mine], ej = bj[2 * n3 + mine];
+      const double gm = NBG_GNEWT * (m_i + m_j);  // not 0: no pair is massless
+      double d[6], mijinv;
       KParams P;
-      pair_state<DF>(lds_at<double>(second ? R.x1 : R.x0), n3, i, j, second ? R.hh1 : R.hh0, x0, v0, P, d, m_i, m_j,
-                     mijinv);
+      if (jac_delxv_gamma_fast<DF>(x0, v0, d, gm, hh, P)) {
+        mijinv = fdiv(1.0, m_i + m_j);  // gm is in the plain range
+      } else {
+        DriftOut o;
+        pair_drift_general(x0[0], x0[1], x0[2], v0[0], v0[1], v0[2], gm, hh, DF, &o);
+        P = o.P;
+        mijinv = 1.0 / (m_i + m_j);
+      }
+      const double delta = (vel ? P.dfdt : P.fm1) * x0c + (vel ? P.dgdtm1 : P.gmh) * v0c;
+      kahan(si, ei, (m_j * mijinv) * delta);
+      kahan(sj, ej, (-(m_i * mijinv)) * delta);
+      x[3 * i + mine] = si;
+      x[3 * j + mine] = sj;
+      x[2 * n3 + 3 * i + mine] = ei;
+      x[2 * n3 + 3 * j + mine] = ej;
       if (keep) {
         int at = pos + q;
         if (at >= slots) at -= slots;
         RingSlot* o = lds_at<RingSlot>((second ? R.ring1 : R.ring0) + (uint32_t)(at * sizeof(RingSlot)));
-        for (int k = 0; k < 3; ++k) {
-          o->x0[k] = x0[k];
-          o->v0[k] = v0[k];
+        reinterpret_cast<double*>(o)[role] = vel ? v0c : x0c;  // x0, then v0
+        if (lane % PAIR_LANES == 0) {
+          o->gamma = P.gamma; o->g1 = P.g1; o->g2 = P.g2; o->g3 = P.g3; o->h1 = P.h1; o->h2 = P.h2;
+          o->r0 = P.r0; o->r = P.r; o->r0inv = P.r0inv; o->rinv = P.rinv;
+          o->beta = P.beta; o->betainv = P.betainv; o->eta = P.eta; o->sqb = P.sqb;
+          o->mijinv = mijinv;
+          o->i = i; o->j = j;
         }
-        o->gamma = P.gamma; o->g1 = P.g1; o->g2 = P.g2; o->g3 = P.g3; o->h1 = P.h1; o->h2 = P.h2;
-        o->r0 = P.r0; o->r = P.r; o->r0inv = P.r0inv; o->rinv = P.rinv;
-        o->beta = P.beta; o->betainv = P.betainv; o->eta = P.eta; o->sqb = P.sqb;
-        o->mijinv = mijinv;
-        o->i = i; o->j = j;
       }
     }
-    q0 += w;
     made += w;
     pos += w;
     if (pos >= slots) pos -= slots;
-    w = uni(w1);
-    second = lane >= w;
-    q = lane - (second ? w : 0);
-    on = lane < 2 * w && (second ? a1 : a0);
-    if (on) ij = pl[2 * (q0 + q)] | ((uint32_t)pl[2 * (q0 + q) + 1] << 8);
     wsync();
     if (keep) publish(&ctl->tail, made, lane);
   }
@@ -662,6 +652,7 @@ __device__ void split_state(L& P, const SysDesc& D0, const SysDesc& D1, const Sy
                             const Visit& v0, const Visit& v1, int lane, int64_t bound, unsigned long long* err) {
   constexpr int N3 = 3 * NB, NP = L::NP, K = TWO ? 1 : 0;
   constexpr int STEP = TWO && N3 <= 32 ? 32 : WAVE;
+  static_assert(L::NS * (NB / 2) * PAIR_LANES <= WAVE, "a level's pairs must fit the wave");
   SplitCtl* ctl = &P.ctl;
   RunCursor c[2];
   const Visit* vs[2] = {&v0, &v1};
@@ -674,7 +665,7 @@ __device__ void split_state(L& P, const SysDesc& D0, const SysDesc& D1, const Sy
   R.x0 = lds_off(P.t[0].x); R.x1 = lds_off(P.t[K].x);
   R.ring0 = lds_off(P.ring[0]); R.ring1 = lds_off(P.ring[K]);
   R.ctl = lds_off(ctl);
-  R.n3 = N3; R.levels = Schedule<NB>::NL; R.slots = L::RR;
+  R.n = NB; R.slots = L::RR;
   R.pos = 0; R.made = 0;
   R.bound = bound; R.err = err;
   int sent = 0, asked = 0;
@@ -716,7 +707,6 @@ __device__ void split_state(L& P, const SysDesc& D0, const SysDesc& D1, const Sy
       wsync();
     };
     drift();
-    R.pairs = lds_off(P.sched.pairs[0]); R.width = lds_off(P.sched.width[0]);
     if (!split_levels<true>(R)) return;
     if (keep) {
       R.made += NP; R.pos = (R.pos + NP) % L::RR;
@@ -735,7 +725,6 @@ __device__ void split_state(L& P, const SysDesc& D0, const SysDesc& D1, const Sy
       if (a1) phi_state<NB, WAVE>(P.t[K], h1, lane);
     }
     wsync();
-    R.pairs = lds_off(P.sched.pairs[1]); R.width = lds_off(P.sched.width[1]);
     if (!split_levels<false>(R)) return;
     drift();
     if (keep) {
@@ -997,15 +986,14 @@ __device__ __attribute__((always_inline)) inline bool split_sweep(SplitLds<NB, G
                                                                   SplitFollow<NB, G, TWO, LIMIT>& F, int dir, double hh0,
                                                                   double hh1, int n0, int n1, int lane) {
   using L = SplitLds<NB, G, TWO, LIMIT>;
-  constexpr int K = TWO ? 1 : 0, NL = Schedule<NB>::NL;
-  const uint8_t* lw = P.sched.width[dir];
+  constexpr int K = TWO ? 1 : 0, NL = level_count(NB);
   const bool p0 = (n0 & (SPLIT_J | SPLIT_Q)) != 0, p1 = TWO && (n1 & (SPLIT_J | SPLIT_Q)) != 0;
   JacSlot* s0 = P.w[0].slot;
   JacSlot* s1 = L::PHI2 ? P.w[L::NW - 1].slot : P.w[0].slot + L::CH;
   int lev = 0;
   while (lev < NL) {
     int cnt = 0;
-    while (lev < NL && cnt + lw[lev] <= L::CH) cnt += lw[lev++];
+    while (lev < NL && cnt + level_width(NB, lev) <= L::CH) cnt += level_width(NB, lev++);
     if (!wait_for(&P.ctl.tail, F.head + cnt, &P.ctl, F.bound, F.err, lane)) return false;
     if (lane < (TWO ? 2 : 1) * cnt) {
       const bool second = lane >= cnt;
@@ -1596,7 +1584,7 @@ template <int NB, int LIMIT> struct SplitLds3 {
     Phi f;
   };
   static constexpr size_t FIXED = sizeof(StateRec<NB>) + sizeof(JacRec<NB, false>) + sizeof(Work) + RR * sizeof(RingSlot) +
-                                  sizeof(SplitCtl) + sizeof(RowCtl) + sizeof(Schedule<NB>) + 64;
+                                  sizeof(SplitCtl) + sizeof(RowCtl) + 64;
   static constexpr int FIT = (int)(((size_t)LIMIT - FIXED) / (2 * sizeof(JacSlot)));
   // pairs per chunk: half a sweep or less, so that the waves overlap
   static constexpr int CH0 = NP < 4 ? NP : (NP + 1) / 2 < 3 ? 3 : (NP + 1) / 2 > 18 ? 18 : (NP + 1) / 2;
@@ -1609,7 +1597,6 @@ template <int NB, int LIMIT> struct SplitLds3 {
   RingSlot ring[1][RR];
   SplitCtl ctl;
   RowCtl row;
-  Schedule<NB> sched;
 };
 
 template <int NB, int LIMIT, bool FACT>
@@ -1617,14 +1604,13 @@ __device__ __attribute__((always_inline)) inline bool pair_wave_sweep(SplitLds3<
                                                                       double hh, int need, int lane, int64_t bound,
                                                                       unsigned long long* err) {
   using L = SplitLds3<NB, LIMIT>;
-  constexpr int NL = Schedule<NB>::NL;
-  const uint8_t* lw = P.sched.width[dir];
+  constexpr int NL = level_count(NB);
   const bool needJ = (need & SPLIT_J) != 0, needQ = (need & SPLIT_Q) != 0;
   JacRec<NB, false>& S = P.j[0];
   int lev = 0;
   while (lev < NL) {
     int cnt = 0;
-    while (lev < NL && cnt + lw[lev] <= L::CH) cnt += lw[lev++];
+    while (lev < NL && cnt + level_width(NB, lev) <= L::CH) cnt += level_width(NB, lev++);
     if (!wait_for(&P.ctl.tail, head + cnt, &P.ctl, bound, err, lane)) return false;
     // the buffer the row wave used two chunks ago
     if (!wait_for(&P.row.chunks_done, chunk - 1, &P.ctl, bound, err, lane)) return false;
@@ -1728,7 +1714,7 @@ template <int NB, int LIMIT, bool FACT>
 __device__ void row_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBufs& B, const Visit& v, int lane, int64_t bound,
                          int64_t bound_job, unsigned long long* err) {
   using L = SplitLds3<NB, LIMIT>;
-  constexpr int NL = Schedule<NB>::NL;
+  constexpr int NL = level_count(NB);
   SplitCtl* ctl = &P.ctl;
   RowCtl* row = &P.row;
   JacRec<NB, false>& S = P.j[0];
@@ -1751,11 +1737,10 @@ __device__ void row_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBuf
     wsync();
 #pragma unroll 1
     for (int dir = 0; dir < 2; ++dir) {
-      const uint8_t* lw = P.sched.width[dir];
       int lev = 0;
       while (lev < NL) {
         int cnt = 0;
-        while (lev < NL && cnt + lw[lev] <= L::CH) cnt += lw[lev++];
+        while (lev < NL && cnt + level_width(NB, lev) <= L::CH) cnt += level_width(NB, lev++);
         if (!wait_for(&row->chunks, chunk + 1, ctl, bound, err, lane)) return;
         split_rows<NB, false, WAVE, FACT>(S, P.slot[chunk & 1], cnt, true, false, lane);
         publish(&row->chunks_done, ++chunk, lane);
@@ -1828,10 +1813,7 @@ __device__ void split_run3(unsigned char* raw, int wave, const SysDesc& D, const
     split_load_state<NB>(P.t[0], D, B, lane);
     for (int w = lane; w < (int)(sizeof(SplitCtl) / 4); w += WAVE) reinterpret_cast<int*>(&P.ctl)[w] = 0;
     for (int w = lane; w < (int)(sizeof(RowCtl) / 4); w += WAVE) reinterpret_cast<int*>(&P.row)[w] = 0;
-  } else if (wave == 1) {
-    for (int w = lane; w < (int)sizeof(Schedule<NB>); w += WAVE)
-      reinterpret_cast<uint8_t*>(&P.sched)[w] = reinterpret_cast<const uint8_t*>(&kSchedule<NB>)[w];
-  } else {
+  } else if (wave == 2) {
     split_load_jac<NB, false>(P.j[0], D, B, lane);
   }
   __syncthreads();
@@ -1876,8 +1858,6 @@ __device__ void split_run(unsigned char* raw, int wave, const SysDesc& D0, const
     split_load_state<NB>(P.t[0], D0, B, lane);
     if (TWO) split_load_state<NB>(P.t[L::NS - 1], D1, B, lane);
     for (int w = lane; w < (int)sizeof(SplitCtl) / 4; w += WAVE) reinterpret_cast<int*>(&P.ctl)[w] = 0;
-    for (int w = lane; w < (int)sizeof(Schedule<NB>); w += WAVE)
-      reinterpret_cast<uint8_t*>(&P.sched)[w] = reinterpret_cast<const uint8_t*>(&kSchedule<NB>)[w];
   } else {
     split_load_jac<NB, G>(P.j[0], D0, B, lane);
     if (TWO) split_load_jac<NB, G>(P.j[L::NS - 1], D1, B, lane);
