@@ -245,9 +245,10 @@ void group_layout(Layout& L) {
   for (size_t g = 0; g < L.gn.size() && budget > 0; ++g) {
     const int off = L.goff[g], cnt = L.gcnt[g], cls = L.gn[g];
     // On the two-wave launches pairs pay up to SPLIT_PAIR_MAX bodies: from 8 on
-    // the Jacobians of twice as many systems overflow the L2 cache (rounds of
-    // 100 steps over 2048 systems of n bodies, one against two a workgroup: 3:
-    // 8.9, 6.1 ms; 5: 17.0, 13.9; 7: 31.6, 26.9; 8: 44.1, 42.3; 9: 52.1, 74.4).
+    // the Jacobians of twice as many systems overflow the L2 cache further
+    // than half the state waves' work is worth (rounds of 100 steps over 2048
+    // systems of n bodies, factored, one against two a workgroup: 6: 21.8,
+    // 20.1 ms; 7: 31.5, 26.3; 8: 38.9, 40.5; 9: 48.0, 66.6).
     bool two_wave = cls == 9;
     for (int k = 0; k < cnt; ++k) two_wave = two_wave && L.desc[L.order[off + k]].split;
     std::vector<std::vector<int>> pos(NB_MAX + 1);  // systems by body count, longest first

@@ -42,6 +42,11 @@ namespace nbg {
 __host__ __device__ constexpr int level_count(int nb) { return 2 * nb - 3; }
 __host__ __device__ constexpr int level_first(int nb, int sum) { return sum - nb + 1 > 0 ? sum - nb + 1 : 0; }  // the smallest i
 __host__ __device__ constexpr int level_width(int nb, int level) { return level / 2 - level_first(nb, level + 1) + 1; }
+// Pairs of the levels before `level` (the sum of their widths).
+__host__ __device__ constexpr int level_start(int nb, int level) {
+  const int left = level_count(nb) - level;
+  return level < nb ? (level + 1) * (level + 1) / 4 : nb * (nb - 1) / 2 - (left + 1) * (left + 1) / 4;
+}
 
 // What the state wave hands over of a pair's drift; the other quantities of
 // KParams and the drift itself follow from these.
@@ -829,145 +834,178 @@ template <bool FACT> __device__ __forceinline__ double split_coef(const JacSlot&
   return rowi == (k < 7) ? v : -v;
 }
 
-// pair_cols from a JacSlot (same operations), STEP lanes a system, every one
+// The row updates of levels [lev0, lev1) of sweep dir (jij_cols' operations),
+// their pair Jacobians in `slots` level by level; STEP lanes a system, every one
 // of them taking part: those past the last column compute it again and store
-// nothing.
+// nothing.  The pairs are taken body by body -- i up and j up, or both down in
+// the second sweep, which keeps every body's order -- so that body i's twelve
+// rows of J and its error stay in registers over its pairs of these levels and
+// body j's next rows are loaded before the arithmetic of the pair at hand.
+// Level by level, each pair loaded and stored both bodies' 24 rows: systems
+// whose J is not in LDS waited for the L2 cache and what lies behind it (302 GB
+// written and 104 read by 250 steps of 4096 systems, 3 TB/s).  Rounds of 200
+// steps over 2048 systems in the reference's order 90.7 -> 70.8 ms; factored,
+// 250 of 4096, 143.7 -> 137.4.
 template <int NB, bool G, int STEP, bool FACT, class R>
-__device__ __attribute__((always_inline)) inline void split_pair_cols(R& S, const JacSlot& sl, int i, int j, int col) {
-  constexpr int N7 = 7 * NB, NC = FACT ? 4 : 6;
-  double cf[NC];
-#pragma unroll
-  for (int r = 0; r < NC; ++r) cf[r] = sl.c[16 * r + (col & 15)];
-  const double mi = sl.mi, mj = sl.mj;
+__device__ __attribute__((always_inline)) inline void split_rows(R& S, const JacSlot* slots, int dir, int lev0, int lev1, int col) {
+  constexpr int N7 = 7 * NB, NC = FACT ? 4 : 6, NL = level_count(NB);
+  const int lo = dir == 0 ? lev0 + 1 : NL - lev1 + 1, hi = dir == 0 ? lev1 : NL - lev0;  // i + j in lo .. hi
+  const int base = level_start(NB, lev0), turn = dir == 0 ? 1 : -1;
+  const int ifirst = level_first(NB, lo), ilast = (hi - 1) / 2;
 #pragma unroll 1
   for (int c0 = 0; c0 < N7; c0 += STEP) {
     const bool on = c0 + col < N7;
     const int c = on ? c0 + col : N7 - 1;
-    double a[12], e[12], o[12];
-    const Column<NB, R> Ci(S, 6 * i, c), Cj(S, 6 * j, c);
+#pragma unroll 1
+    for (int i = dir == 0 ? ifirst : ilast; i >= ifirst && i <= ilast; i += turn) {
+      const int jlo = lo - i > i + 1 ? lo - i : i + 1, jhi = hi - i < NB - 1 ? hi - i : NB - 1;
+      if (jlo > jhi) continue;
+      int j = dir == 0 ? jlo : jhi;
+      const double a6 = (c == 7 * i + 6) ? 1.0 : 0.0;
+      const Column<NB, R> Ci(S, 6 * i, c);
+      double ai[6], ei[6], aj[6], ej[6];
+      auto load = [&](const Column<NB, R>& C, double (&a)[6], double (&e)[6]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      a[k] = Ci.j(k);
-      a[6 + k] = Cj.j(k);
-    }
+        for (int k = 0; k < 6; ++k) a[k] = C.j(k);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      e[k] = Ci.e(k);
-      e[6 + k] = Cj.e(k);
-    }
-    // all 24 rows are in flight before the arithmetic starts (left alone, the
-    // scheduler moves the error rows' loads down to their uses, each with a
-    // wait of its own)
-    __builtin_amdgcn_sched_barrier(0);
-    const double a6 = (c == 7 * i + 6) ? 1.0 : 0.0;
-    const double a13 = (c == 7 * j + 6) ? 1.0 : 0.0;
-    if constexpr (FACT) {
-      double d[6], sk[6];
+        for (int k = 0; k < 6; ++k) e[k] = C.e(k);
+      };
+      load(Ci, ai, ei);
+      if constexpr (G) load(Column<NB, R>(S, 6 * j, c), aj, ej);
+#pragma unroll 1
+      while (true) {
+        const int sum = i + j, at = level_start(NB, dir == 0 ? sum - 1 : NL - sum) - base + i - level_first(NB, sum);
+        const JacSlot& sl = slots[at];
+        double cf[NC];
 #pragma unroll
-      for (int k = 0; k < 6; ++k) {
-        d[k] = a[k] - a[6 + k];
-        sk[k] = 0.0;
+        for (int r = 0; r < NC; ++r) cf[r] = sl.c[16 * r + (col & 15)];
+        const double mi = sl.mi, mj = sl.mj;
+        // G: the next partner's rows are in flight during the arithmetic (the
+        // last pair loads its own again); LDS answers too soon for the copies
+        // that costs
+        const int jn = j + turn < jlo || j + turn > jhi ? j : j + turn;
+        const Column<NB, R> Cj(S, 6 * j, c);
+        double an[6], en[6];
+        if constexpr (G) load(Column<NB, R>(S, 6 * jn, c), an, en);
+        else load(Cj, aj, ej);
+        __builtin_amdgcn_sched_barrier(0);
+        const double a13 = (c == 7 * j + 6) ? 1.0 : 0.0;
+        double oi[6], oj[6];
+        if constexpr (FACT) {
+          double d[6], sk[6];
+#pragma unroll
+          for (int k = 0; k < 6; ++k) {
+            d[k] = ai[k] - aj[k];
+            sk[k] = 0.0;
+          }
+          fmac6<0>(sk, cf, d[0]);
+          fmac6<6>(sk, cf, d[1]);
+          fmac6<12>(sk, cf, d[2]);
+          fmac6<18>(sk, cf, d[3]);
+          fmac6<24>(sk, cf, d[4]);
+          fmac6<30>(sk, cf, d[5]);
+#pragma unroll
+          for (int rk = 0; rk < 6; ++rk) {
+            oi[rk] = mj * sk[rk];
+            oj[rk] = (-mi) * sk[rk];
+          }
+          fmac6<36>(oi, cf, a6);
+          fmac6<42>(oj, cf, a6);
+          fmac6<48>(oi, cf, a13);
+          fmac6<54>(oj, cf, a13);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 6; ++q) oi[q] = oj[q] = 0.0;
+          // k = 0..5: rows of i get +mj*kep * a_i[k], rows of j -mi*kep * a_i[k]
+          fmac6<0>(oi, cf, ai[0]);
+          fmac6<36, true>(oj, cf, ai[0]);
+          fmac6<6>(oi, cf, ai[1]);
+          fmac6<42, true>(oj, cf, ai[1]);
+          fmac6<12>(oi, cf, ai[2]);
+          fmac6<48, true>(oj, cf, ai[2]);
+          fmac6<18>(oi, cf, ai[3]);
+          fmac6<54, true>(oj, cf, ai[3]);
+          fmac6<24>(oi, cf, ai[4]);
+          fmac6<60, true>(oj, cf, ai[4]);
+          fmac6<30>(oi, cf, ai[5]);
+          fmac6<66, true>(oj, cf, ai[5]);
+          fmac6<72>(oi, cf, a6);
+          fmac6<78>(oj, cf, a6);
+          // k = 7..12: rows of i get -mj*kep * a_j[k], rows of j +mi*kep * a_j[k]
+          fmac6<0, true>(oi, cf, aj[0]);
+          fmac6<36>(oj, cf, aj[0]);
+          fmac6<6, true>(oi, cf, aj[1]);
+          fmac6<42>(oj, cf, aj[1]);
+          fmac6<12, true>(oi, cf, aj[2]);
+          fmac6<48>(oj, cf, aj[2]);
+          fmac6<18, true>(oi, cf, aj[3]);
+          fmac6<54>(oj, cf, aj[3]);
+          fmac6<24, true>(oi, cf, aj[4]);
+          fmac6<60>(oj, cf, aj[4]);
+          fmac6<30, true>(oi, cf, aj[5]);
+          fmac6<66>(oj, cf, aj[5]);
+          fmac6<84>(oi, cf, a13);
+          fmac6<90>(oj, cf, a13);
+        }
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+          kahan(ai[q], ei[q], oi[q]);
+          kahan(aj[q], ej[q], oj[q]);
+        }
+        if (on) {
+#pragma unroll
+          for (int k = 0; k < 6; ++k) {
+            Cj.j(k) = aj[k];
+            Cj.e(k) = ej[k];
+          }
+        }
+        if (jn == j) break;
+        j = jn;
+        if constexpr (G) {
+#pragma unroll
+          for (int k = 0; k < 6; ++k) {
+            aj[k] = an[k];
+            ej[k] = en[k];
+          }
+        }
       }
-      fmac6<0>(sk, cf, d[0]);
-      fmac6<6>(sk, cf, d[1]);
-      fmac6<12>(sk, cf, d[2]);
-      fmac6<18>(sk, cf, d[3]);
-      fmac6<24>(sk, cf, d[4]);
-      fmac6<30>(sk, cf, d[5]);
+      if (on) {
 #pragma unroll
-      for (int rk = 0; rk < 6; ++rk) {
-        o[rk] = mj * sk[rk];
-        o[6 + rk] = (-mi) * sk[rk];
-      }
-      fmac6<36>(o, cf, a6);
-      fmac6<42>(o + 6, cf, a6);
-      fmac6<48>(o, cf, a13);
-      fmac6<54>(o + 6, cf, a13);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 12; ++q) o[q] = 0.0;
-      // k = 0..5: rows of i get +mj*kep * a_i[k], rows of j -mi*kep * a_i[k]
-      fmac6<0>(o, cf, a[0]);
-      fmac6<36, true>(o + 6, cf, a[0]);
-      fmac6<6>(o, cf, a[1]);
-      fmac6<42, true>(o + 6, cf, a[1]);
-      fmac6<12>(o, cf, a[2]);
-      fmac6<48, true>(o + 6, cf, a[2]);
-      fmac6<18>(o, cf, a[3]);
-      fmac6<54, true>(o + 6, cf, a[3]);
-      fmac6<24>(o, cf, a[4]);
-      fmac6<60, true>(o + 6, cf, a[4]);
-      fmac6<30>(o, cf, a[5]);
-      fmac6<66, true>(o + 6, cf, a[5]);
-      fmac6<72>(o, cf, a6);
-      fmac6<78>(o + 6, cf, a6);
-      // k = 7..12: rows of i get -mj*kep * a_j[k], rows of j +mi*kep * a_j[k]
-      fmac6<0, true>(o, cf, a[6]);
-      fmac6<36>(o + 6, cf, a[6]);
-      fmac6<6, true>(o, cf, a[7]);
-      fmac6<42>(o + 6, cf, a[7]);
-      fmac6<12, true>(o, cf, a[8]);
-      fmac6<48>(o + 6, cf, a[8]);
-      fmac6<18, true>(o, cf, a[9]);
-      fmac6<54>(o + 6, cf, a[9]);
-      fmac6<24, true>(o, cf, a[10]);
-      fmac6<60>(o + 6, cf, a[10]);
-      fmac6<30, true>(o, cf, a[11]);
-      fmac6<66>(o + 6, cf, a[11]);
-      fmac6<84>(o, cf, a13);
-      fmac6<90>(o + 6, cf, a13);
-    }
-#pragma unroll
-    for (int q = 0; q < 12; ++q) {
-      double sv = a[q], se = e[q];
-      se += o[q];
-      const double t = sv + se;
-      se += sv - t;
-      a[q] = t;
-      e[q] = se;
-    }
-    if (on) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) {
-        Ci.j(k) = a[k];
-        Cj.j(k) = a[6 + k];
-        Ci.e(k) = e[k];
-        Cj.e(k) = e[6 + k];
+        for (int k = 0; k < 6; ++k) {
+          Ci.j(k) = ai[k];
+          Ci.e(k) = ei[k];
+        }
       }
     }
   }
 }
 
-// Phase C of a chunk (sweep_rows).
-template <int NB, bool G, int STEP, bool FACT, class R>
-__device__ __attribute__((always_inline)) inline void split_rows(R& S, const JacSlot* slots, int cnt, bool needJ, bool needQ, int col) {
+// dqdt_ij (ahl21.jl:743-748) and dq/dt's rows, of cnt pairs level by level.
+template <int NB, bool FACT, class R>
+__device__ __attribute__((always_inline)) inline void split_rates(R& S, const JacSlot* slots, int cnt, int col) {
 #pragma unroll 1
   for (int q = 0; q < cnt; ++q) {
     const JacSlot& sl = slots[q];
     const int i = sl.i, j = sl.j;
-    if (needJ) split_pair_cols<NB, G, STEP, FACT>(S, sl, i, j, col);
-    if (needQ) {
-      // dqdt_ij (ahl21.jl:743-748) and dq/dt's rows
-      if (col < 14) {
-        const bool rowi = col < 7;
-        const int rk = rowi ? col : col - 7;
-        double q1[14];
-        for (int k = 0; k < 7; ++k) {
-          q1[k] = S.dqdt[7 * i + k];
-          q1[7 + k] = S.dqdt[7 * j + k];
-        }
-        double s2 = 0.0, dq = S.dqij[col];
-        const double mine = S.dqdt[rowi ? 7 * i + rk : 7 * j + rk];
-        if (rk < 6) {
-          dq = (rowi ? sl.mj : -sl.mi) * sl.kh[rk];
-          for (int k = 0; k < 14; ++k) s2 = fmad(split_coef<FACT>(sl, rowi, rk, k), q1[k], s2);
-        } else {
-          for (int k = 0; k < 14; ++k) s2 = fmad(0.0, q1[k], s2);
-        }
-        const double nd = (dq * 0.5) + (mine + s2);
-        S.dqij[col] = nd;
-        S.dqdt[rowi ? 7 * i + rk : 7 * j + rk] = nd;
+    if (col < 14) {
+      const bool rowi = col < 7;
+      const int rk = rowi ? col : col - 7;
+      double q1[14];
+      for (int k = 0; k < 7; ++k) {
+        q1[k] = S.dqdt[7 * i + k];
+        q1[7 + k] = S.dqdt[7 * j + k];
       }
+      double s2 = 0.0, dq = S.dqij[col];
+      const double mine = S.dqdt[rowi ? 7 * i + rk : 7 * j + rk];
+      if (rk < 6) {
+        dq = (rowi ? sl.mj : -sl.mi) * sl.kh[rk];
+        for (int k = 0; k < 14; ++k) s2 = fmad(split_coef<FACT>(sl, rowi, rk, k), q1[k], s2);
+      } else {
+        for (int k = 0; k < 14; ++k) s2 = fmad(0.0, q1[k], s2);
+      }
+      const double nd = (dq * 0.5) + (mine + s2);
+      S.dqij[col] = nd;
+      S.dqdt[rowi ? 7 * i + rk : 7 * j + rk] = nd;
     }
     wsync();
   }
@@ -992,6 +1030,7 @@ __device__ __attribute__((always_inline)) inline bool split_sweep(SplitLds<NB, G
   JacSlot* s1 = L::PHI2 ? P.w[L::NW - 1].slot : P.w[0].slot + L::CH;
   int lev = 0;
   while (lev < NL) {
+    const int lev0 = lev;
     int cnt = 0;
     while (lev < NL && cnt + level_width(NB, lev) <= L::CH) cnt += level_width(NB, lev++);
     if (!wait_for(&P.ctl.tail, F.head + cnt, &P.ctl, F.bound, F.err, lane)) return false;
@@ -1014,15 +1053,18 @@ __device__ __attribute__((always_inline)) inline bool split_sweep(SplitLds<NB, G
     F.pos += cnt;
     if (F.pos >= L::RR) F.pos -= L::RR;
     publish(&P.ctl.head, F.head, lane);
+    const bool j0 = (n0 & SPLIT_J) != 0, q0 = (n0 & SPLIT_Q) != 0, j1 = (n1 & SPLIT_J) != 0, q1 = (n1 & SPLIT_Q) != 0;
     if constexpr (L::HALF) {
       const bool sys = lane >= 32;
-      if (sys ? p1 : p0)
-        split_rows<NB, G, 32, FACT>(sys ? P.j[K] : P.j[0], sys ? s1 : s0, cnt, ((sys ? n1 : n0) & SPLIT_J) != 0,
-                                    ((sys ? n1 : n0) & SPLIT_Q) != 0, lane & 31);
+      if (sys ? j1 : j0) split_rows<NB, G, 32, FACT>(sys ? P.j[K] : P.j[0], sys ? s1 : s0, dir, lev0, lev, lane & 31);
+      if (sys ? q1 : q0) split_rates<NB, FACT>(sys ? P.j[K] : P.j[0], sys ? s1 : s0, cnt, lane & 31);
       wsync();
     } else {
-      if (p0) split_rows<NB, G, WAVE, FACT>(P.j[0], s0, cnt, (n0 & SPLIT_J) != 0, (n0 & SPLIT_Q) != 0, lane);
-      if (p1) split_rows<NB, G, WAVE, FACT>(P.j[K], s1, cnt, (n1 & SPLIT_J) != 0, (n1 & SPLIT_Q) != 0, lane);
+      if (j0) split_rows<NB, G, WAVE, FACT>(P.j[0], s0, dir, lev0, lev, lane);
+      if (q0) split_rates<NB, FACT>(P.j[0], s0, cnt, lane);
+      if (TWO && j1) split_rows<NB, G, WAVE, FACT>(P.j[K], s1, dir, lev0, lev, lane);
+      if (TWO && q1) split_rates<NB, FACT>(P.j[K], s1, cnt, lane);
+      wsync();
     }
   }
   return true;
@@ -1609,6 +1651,7 @@ __device__ __attribute__((always_inline)) inline bool pair_wave_sweep(SplitLds3<
   JacRec<NB, false>& S = P.j[0];
   int lev = 0;
   while (lev < NL) {
+    const int lev0 = lev;
     int cnt = 0;
     while (lev < NL && cnt + level_width(NB, lev) <= L::CH) cnt += level_width(NB, lev++);
     if (!wait_for(&P.ctl.tail, head + cnt, &P.ctl, bound, err, lane)) return false;
@@ -1628,7 +1671,7 @@ __device__ __attribute__((always_inline)) inline bool pair_wave_sweep(SplitLds3<
     if (pos >= L::RR) pos -= L::RR;
     publish(&P.ctl.head, head, lane);
     if (needJ) publish(&P.row.chunks, ++chunk, lane);
-    if (needQ) split_rows<NB, false, WAVE, FACT>(S, slots, cnt, false, true, lane);
+    if (needQ) split_rates<NB, FACT>(S, slots, cnt, lane);
   }
   return true;
 }
@@ -1739,10 +1782,12 @@ __device__ void row_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBuf
     for (int dir = 0; dir < 2; ++dir) {
       int lev = 0;
       while (lev < NL) {
+        const int lev0 = lev;
         int cnt = 0;
         while (lev < NL && cnt + level_width(NB, lev) <= L::CH) cnt += level_width(NB, lev++);
         if (!wait_for(&row->chunks, chunk + 1, ctl, bound, err, lane)) return;
-        split_rows<NB, false, WAVE, FACT>(S, P.slot[chunk & 1], cnt, true, false, lane);
+        split_rows<NB, false, WAVE, FACT>(S, P.slot[chunk & 1], dir, lev0, lev, lane);
+        wsync();
         publish(&row->chunks_done, ++chunk, lane);
       }
       if (dir == 0) {
