@@ -440,41 +440,55 @@ template <int NB> __device__ inline void split_restore_prior(StateRec<NB>& S, in
   wsync();
 }
 
-// detect_transits! from body c.body on (cursor_detect).
+// detect_transits! from body c.body on (cursor_detect), a lane a body: the
+// first that transits starts a search, those before it keep their g; the ones
+// after it are looked at again when the search has ended.  One body after the
+// other, each took its own chain of LDS reads and a square root.
 template <int NB> __device__ void split_detect(StateRec<NB>& S, const SysDesc& D, RunCursor& c, int lane) {
   const int ti = D.ti;
   int act = c.is < c.iend ? ACT_MAIN : ACT_DONE;
-  int body = NB;
+  int body = NB, from = c.body;
 #pragma unroll 1
-  for (int i = c.body; i < NB; ++i) {
-    if (i == ti) continue;
-    const double gi = gsky<NB>(S, i, ti);
-    const double ri = __builtin_sqrt((S.x[3 * i] * S.x[3 * i] + S.x[3 * i + 1] * S.x[3 * i + 1]) + S.x[3 * i + 2] * S.x[3 * i + 2]);
-    if (gi > 0.0 && S.gsave[i] < 0.0 && -S.x[3 * i + 2] > 0.25 * ri && ri < 1e12) {
-      const int64_t cnt = S.count[i] + 1;
-      wsync();
-      if (lane == 0) S.count[i] = cnt;
-      wsync();
-      if (cnt >= 1 && cnt <= D.ntt) {
-        if (!c.saved) {
-          split_save_prior<NB>(S, lane);
-          c.saved = 1;
-        }
-        c.dt0 = ((-gi) * D.hstep) / (gi - S.gsave[i]);
-        c.gi = gi;
-        c.jb = i;
-        c.iter = 0;
-        c.stmp = 0.0;
-        c.tt1 = c.dt0 + 1.0;
-        c.tt2 = c.dt0 + 2.0;
-        act = ACT_NEWTON;
-        body = i;  // gsave[i] is written when the search ends
-        break;
-      }
+  while (from < NB) {
+    const bool mine = lane >= from && lane < NB && lane != ti;
+    double g = 0.0;
+    bool hit = false;
+    if (mine) {
+      const double *x = S.x + 3 * lane;
+      g = gsky<NB>(S, lane, ti);
+      const double r = __builtin_sqrt((x[0] * x[0] + x[1] * x[1]) + x[2] * x[2]);
+      hit = g > 0.0 && S.gsave[lane] < 0.0 && -x[2] > 0.25 * r && r < 1e12;
     }
+    const uint64_t hits = __builtin_amdgcn_ballot_w64(hit);
+    const int i = hits ? __builtin_ctzll(hits) : NB;
     wsync();
-    if (lane == 0) S.gsave[i] = gi;
+    if (mine && lane < i) S.gsave[lane] = g;
     wsync();
+    if (i == NB) break;
+    const int64_t cnt = S.count[i] + 1;
+    wsync();
+    if (lane == 0) S.count[i] = cnt;
+    wsync();
+    if (cnt >= 1 && cnt <= D.ntt) {
+      if (!c.saved) {
+        split_save_prior<NB>(S, lane);
+        c.saved = 1;
+      }
+      const double gi = gsky<NB>(S, i, ti);
+      c.dt0 = ((-gi) * D.hstep) / (gi - S.gsave[i]);
+      c.gi = gi;
+      c.jb = i;
+      c.iter = 0;
+      c.stmp = 0.0;
+      c.tt1 = c.dt0 + 1.0;
+      c.tt2 = c.dt0 + 2.0;
+      act = ACT_NEWTON;
+      body = i;  // gsave[i] is written when the search ends
+      break;
+    }
+    if (lane == i) S.gsave[i] = g;
+    wsync();
+    from = i + 1;
   }
   c.act = __builtin_amdgcn_readfirstlane(act);
   c.body = __builtin_amdgcn_readfirstlane(body);
