@@ -55,10 +55,11 @@ FP64_PEAK_TFLOPS = 78.6
 # batch, by kernel and row update (0 reference order, 1 factored), from
 # rocprofv3 FETCH_SIZE and WRITE_SIZE passes scaled by the same counters'
 # reading of nbg_copy_kernel of known size (the figures and the commands are
-# in profiles/nbg_run_duo_c2_round_counters.md and
-# nbg_run_duo_c2_round_factored_counters.md); a configuration without a
+# in profiles/nbg_run_split_c2_round.md and
+# nbg_run_split_duo_c2_round_counters.md); a configuration without a
 # measurement of the current kernels reports traffic null
-HBM_BYTES_PER_UNIT = {("nbg_run_duo<9>", 0): 470.3e3, ("nbg_run_duo<9>", 1): 354.7e3}
+HBM_BYTES_PER_UNIT = {("nbg_run_split<11>", 0): 282.7e3, ("nbg_run_split<11>", 1): 258.8e3,
+                      ("nbg_run_split_duo<9>", 0): 447.0e3, ("nbg_run_split_duo<9>", 1): 398.6e3}
 METRIC = "system-steps/s w/ Jacobian, batched vs plain GPU; p50/p99 request latency"
 T_START = time.perf_counter()
 
@@ -332,7 +333,8 @@ def main():
     lrep = {}
     for cls, L in launches.items():
         flops = sum(W(n) * u for n, u in L["units"].items())
-        kname = "nbg_run_coop<10>" if cls == 1 else ("nbg_run_duo<%d>" if spw == 2 else "nbg_run<%d>") % cls
+        # this workload's pairs are all Kepler pairs: two waves a workgroup
+        kname = "nbg_run_coop<10>" if cls == 1 else "nbg_run_split_duo<9>" if spw == 2 else "nbg_run_split<%d>" % max(cls, 11)
         lrep[str(cls)] = {"kernel": kname, "ms_total": L["ms"], "ms_per_round": L["ms"] / args.steps,
                           "grid": L["grid"], "units": sum(L["units"].values()),
                           "units_by_n": {str(n): u for n, u in sorted(L["units"].items())}, "flops": flops,
