@@ -561,6 +561,10 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
     if (g == 1 && chunk == 0) std::this_thread::sleep_for(std::chrono::microseconds(2000));
     nbg::GroupList gl{};
     gl.rowupd = ctx->row_update;
+    // Two-per-wave launches take units (ustart) of a group's whole queue; the
+    // two- and three-wave launches of a class without pairs take its systems
+    // one by one, from the first that is not a cooperative one.
+    const bool by_unit = L.pairs && (!split[g] || paired[g]);
     // own class, then the smaller ones whose launch takes systems the same way
     for (size_t h = g; h < G; ++h) {
       if (h > g && !wide && (split[h] != split[g] || (split[g] && (paired[h] || paired[g])))) continue;
@@ -568,7 +572,7 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
       gl.nsys[gl.ng] = L.gcnt[h] - skip;
       gl.descs[gl.ng] = S.desc.p + L.goff[h] + skip;
       gl.queue[gl.ng] = S.queue.p + h;
-      if (L.pairs) {  // units from the first one after the cooperative systems; offsets from the group's start
+      if (by_unit) {  // units from the first one after the cooperative systems; offsets from the group's start
         const int* us = L.ustart.data() + L.uoff[h];
         const int nu = (int)((h + 1 < G ? L.uoff[h + 1] : (int)L.ustart.size()) - L.uoff[h]) - 1;
         int u0 = 0;
@@ -597,7 +601,7 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
               : paired[g] ? nbg_launch_split_duo(gl, B, chunk, split_bound, split_job, grid, un, wait_err, st)
                           : nbg_launch_split(L.gn[g], gl, B, chunk, split_bound, split_job, grid, un, wait_err, st));
     } else if (work > 0)
-      NBG_HIP(L.pairs ? nbg_launch_group_duo(L.gn[g], gl, B, chunk, grid, S.units.p + 13 * g, st)
+      NBG_HIP(by_unit ? nbg_launch_group_duo(L.gn[g], gl, B, chunk, grid, S.units.p + 13 * g, st)
                       : nbg_launch_group(L.gn[g], gl, B, chunk, grid, S.units.p + 13 * g, st));
     if (timed) NBG_HIP(hipEventRecord(ctx->gev[2 * g + 1], st));
   }
