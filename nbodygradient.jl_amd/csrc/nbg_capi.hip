@@ -2006,6 +2006,7 @@ int nbg_batch_cartesian(nbg_ctx* ctx, int32_t nsys, const int32_t* n, const doub
     d.traj = records;
     d.nsteps = nstep[s]; d.ntt = 0; d.h = h[s] * check_step(t0[s], tmax[s]); d.hstep = h[s]; d.hlast = 0.0;
     d.t0 = t0[s];
+    d.split = split_ok(d, m + ob[s]);
   }
   finalize_layout(L);
   Store S;
