@@ -2417,10 +2417,10 @@ template <int HI> struct TransitRing {
   double st[COOP_RQ][19 * HI + 1];  // x, v, xe, ve (3n each), dqdt (7n), t
 };
 
-__device__ __forceinline__ int ring_load(const int* p) {
+template <class T> __device__ __forceinline__ T ring_load(const T* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ __forceinline__ void ring_store(int* p, int v) {
+template <class T> __device__ __forceinline__ void ring_store(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 

@@ -181,9 +181,10 @@ template <int NB, int CHMIN> struct JacWork {
 // Steps of a system as the Jacobian wave sees them (RunCursor's act).
 enum : int { SPLIT_J = 4, SPLIT_Q = 8, SPLIT_SAVE = 16 };
 struct SplitCtl {
-  int tail, head;     // pairs published / released, per system
-  int sent, seen;     // messages published / copied
-  int answered;       // steps whose dq/dt is complete
+  // counters (counter_reached), from COUNTER_START on
+  uint32_t tail, head;  // pairs published / released, per system
+  uint32_t sent, seen;  // messages published / copied
+  uint32_t answered;    // steps whose dq/dt is complete
   int quit;           // the state wave is done, or a wait ran out
   int act[2];         // PRE: what the step is
   int body[2];        // PRE: a gradient step's body ...
@@ -220,16 +221,21 @@ template <int NB, bool G, bool TWO, int LIMIT> struct SplitLds {
   SplitCtl ctl;
 };
 
-__device__ __forceinline__ void publish(int* counter, int v, int lane) {
+__device__ __forceinline__ void start_counters(SplitCtl& c, int lane) {
+  if (lane != 0) return;
+  c.tail = c.head = c.sent = c.seen = c.answered = COUNTER_START;
+  c.quit = 0;
+}
+__device__ __forceinline__ void publish(uint32_t* counter, uint32_t v, int lane) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   if (lane == 0) ring_store(counter, v);
 }
-// Waits until *counter >= v (as a difference); false when the other wave has
-// quit or the bound runs out.
-__device__ __forceinline__ bool wait_for(const int* counter, int v, SplitCtl* ctl, int64_t bound, unsigned long long* err,
-                                         int lane) {
+// Waits until the counter has reached v; false when the other wave has quit or
+// the bound runs out.
+__device__ __forceinline__ bool wait_for(const uint32_t* counter, uint32_t v, SplitCtl* ctl, int64_t bound,
+                                         unsigned long long* err, int lane) {
   int64_t spins = 0;
-  while (ring_load(counter) - v < 0) {
+  while (!counter_reached(ring_load(counter), v)) {
     if (ring_load(&ctl->quit) == 2) return false;
     if (++spins > bound) {
       if (lane == 0) {
@@ -259,7 +265,8 @@ __device__ __forceinline__ bool wait_for(const int* counter, int v, SplitCtl* ct
 constexpr int PAIR_LANES = 8;
 struct SplitSweep {
   uint32_t x0, x1, ring0, ring1, ctl;
-  int n, act0, act1, keep, slots, pos, made;
+  int n, act0, act1, keep, slots, pos;
+  uint32_t made;
   double hh0, hh1;
   int64_t bound;
   unsigned long long* err;
@@ -269,7 +276,8 @@ template <bool DF> static __device__ __attribute__((noinline)) bool split_levels
   auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   const int n = uni(R.n), slots = uni(R.slots), n3 = 3 * n, levels = level_count(n);
   const bool a0 = uni(R.act0) != 0, a1 = uni(R.act1) != 0, keep = uni(R.keep) != 0;
-  int pos = uni(R.pos), made = uni(R.made);
+  int pos = uni(R.pos);
+  uint32_t made = uni(R.made);
   SplitCtl* ctl = lds_at<SplitCtl>(uni(R.ctl));
   const int group = lane / PAIR_LANES, role = lane % PAIR_LANES < 6 ? lane % PAIR_LANES : lane % PAIR_LANES - 6;
   const bool vel = role >= 3;
@@ -685,9 +693,9 @@ __device__ void split_state(L& P, const SysDesc& D0, const SysDesc& D1, const Sy
   R.ring0 = lds_off(P.ring[0]); R.ring1 = lds_off(P.ring[K]);
   R.ctl = lds_off(ctl);
   R.n = NB; R.slots = L::RR;
-  R.pos = 0; R.made = 0;
+  R.pos = 0; R.made = COUNTER_START;
   R.bound = bound; R.err = err;
-  int sent = 0, asked = 0;
+  uint32_t sent = COUNTER_START, asked = COUNTER_START;
   const int half = STEP == 32 ? lane >> 5 : 0, col = STEP == 32 ? lane & 31 : lane;
 #pragma unroll 1
   while (c[0].act != ACT_DONE || c[1].act != ACT_DONE) {
@@ -1026,7 +1034,8 @@ __device__ __attribute__((always_inline)) inline void split_rates(R& S, const Ja
 }
 
 template <int NB, bool G, bool TWO, int LIMIT> struct SplitFollow {
-  int head, pos;
+  uint32_t head;
+  int pos;
   int64_t bound;
   unsigned long long* err;
 };
@@ -1482,14 +1491,14 @@ __device__ void split_jacobian(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0
   constexpr int N3 = 3 * NB, N7 = 7 * NB, K = TWO ? 1 : 0;
   constexpr int STEP = L::HALF ? 32 : WAVE;
   SplitCtl* ctl = &P.ctl;
-  SplitFollow<NB, G, TWO, LIMIT> F{0, 0, bound, err};
+  SplitFollow<NB, G, TWO, LIMIT> F{COUNTER_START, 0, bound, err};
   JacRec<NB, G>& J0 = P.j[0];
   JacRec<NB, G>& J1 = P.j[K];
   typename L::Work& W0 = P.w[0];
   typename L::Work& W1 = P.w[L::NW - 1];
   const bool sys = L::HALF && lane >= 32;
   const int col = L::HALF ? lane & 31 : lane;
-  int seen = 0, answered = 0;
+  uint32_t seen = COUNTER_START, answered = COUNTER_START;
 #pragma unroll 1
   while (true) {
     if (!wait_for(&ctl->sent, seen + 1, ctl, bound_job, err, lane)) return;
@@ -1620,10 +1629,11 @@ struct RowHeader {
   double gd, dx, dy, dvx, dvy, ax, ay;  // a gradient step's end (split_gradient)
 };
 struct RowCtl {
-  int chunks, chunks_done;  // published / released, of all sweeps so far
-  int phis, phis_done;
-  int heads, heads_seen;    // steps announced / read
-  int ends, steps_done;     // gradient scalars written; steps finished
+  // counters (counter_reached), from COUNTER_START on
+  uint32_t chunks, chunks_done;  // published / released, of all sweeps so far
+  uint32_t phis, phis_done;
+  uint32_t heads, heads_seen;    // steps announced / read
+  uint32_t ends;                 // gradient steps whose scalars are written
   RowHeader hdr[2];
 };
 
@@ -1656,7 +1666,7 @@ template <int NB, int LIMIT> struct SplitLds3 {
 };
 
 template <int NB, int LIMIT, bool FACT>
-__device__ __attribute__((always_inline)) inline bool pair_wave_sweep(SplitLds3<NB, LIMIT>& P, int& head, int& pos, int& chunk, int dir,
+__device__ __attribute__((always_inline)) inline bool pair_wave_sweep(SplitLds3<NB, LIMIT>& P, uint32_t& head, int& pos, uint32_t& chunk, int dir,
                                                                       double hh, int need, int lane, int64_t bound,
                                                                       unsigned long long* err) {
   using L = SplitLds3<NB, LIMIT>;
@@ -1697,7 +1707,9 @@ __device__ void pair_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBu
   SplitCtl* ctl = &P.ctl;
   RowCtl* row = &P.row;
   JacRec<NB, false>& S = P.j[0];
-  int seen = 0, answered = 0, head = 0, pos = 0, chunk = 0, steps = 0;  // steps: announced to the row wave
+  uint32_t seen = COUNTER_START, answered = COUNTER_START, head = COUNTER_START, chunk = COUNTER_START;
+  uint32_t steps = COUNTER_START, ends = COUNTER_START;  // announced to the row wave; gradient steps' ends
+  int pos = 0;
 #pragma unroll 1
   while (true) {
     if (!wait_for(&ctl->sent, seen + 1, ctl, bound_job, err, lane)) return;
@@ -1759,7 +1771,7 @@ __device__ void pair_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBu
         H.ay = S.dqdt[7 * jb + 4] - S.dqdt[7 * ti + 4];
       }
       wsync();
-      publish(&row->ends, steps, lane);
+      publish(&row->ends, ++ends, lane);
     } else if ((need & 3) == ACT_MAIN && needQ) {
       for (int q = lane; q < N7; q += WAVE) S.run_dqdt[q] = S.dqdt[q];
       wsync();
@@ -1775,7 +1787,7 @@ __device__ void row_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBuf
   SplitCtl* ctl = &P.ctl;
   RowCtl* row = &P.row;
   JacRec<NB, false>& S = P.j[0];
-  int steps = 0, chunk = 0;
+  uint32_t steps = COUNTER_START, ends = COUNTER_START, chunk = COUNTER_START;
 #pragma unroll 1
   while (true) {
     if (!wait_for(&row->heads, steps + 1, ctl, bound_job, err, lane)) return;
@@ -1814,7 +1826,7 @@ __device__ void row_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBuf
     split_drift<NB, false, WAVE, FACT>(S, 0.5 * h, lane);
     wsync();
     if (need & SPLIT_SAVE) {
-      if (!wait_for(&row->ends, steps, ctl, bound, err, lane)) return;
+      if (!wait_for(&row->ends, ++ends, ctl, bound, err, lane)) return;
       const RowHeader G = H;
       split_gradient_rows<NB>(S, D, B, body, index, G.gd, G.dx, G.dy, G.dvx, G.dvy, G.ax, G.ay, lane);
       split_keep_jac<NB>(S, B.ws + D.off_ws, true, lane);
@@ -1870,8 +1882,11 @@ __device__ void split_run3(unsigned char* raw, int wave, const SysDesc& D, const
   const Visit v = visit_of(D, B, chunk), none{1, 1, 0};
   if (wave == 0) {
     split_load_state<NB>(P.t[0], D, B, lane);
-    for (int w = lane; w < (int)(sizeof(SplitCtl) / 4); w += WAVE) reinterpret_cast<int*>(&P.ctl)[w] = 0;
-    for (int w = lane; w < (int)(sizeof(RowCtl) / 4); w += WAVE) reinterpret_cast<int*>(&P.row)[w] = 0;
+    start_counters(P.ctl, lane);
+    if (lane == 0) {
+      RowCtl& r = P.row;
+      r.chunks = r.chunks_done = r.phis = r.phis_done = r.heads = r.heads_seen = r.ends = COUNTER_START;
+    }
   } else if (wave == 2) {
     split_load_jac<NB, false>(P.j[0], D, B, lane);
   }
@@ -1916,7 +1931,7 @@ __device__ void split_run(unsigned char* raw, int wave, const SysDesc& D0, const
   if (wave == 0) {
     split_load_state<NB>(P.t[0], D0, B, lane);
     if (TWO) split_load_state<NB>(P.t[L::NS - 1], D1, B, lane);
-    for (int w = lane; w < (int)sizeof(SplitCtl) / 4; w += WAVE) reinterpret_cast<int*>(&P.ctl)[w] = 0;
+    start_counters(P.ctl, lane);
   } else {
     split_load_jac<NB, G>(P.j[0], D0, B, lane);
     if (TWO) split_load_jac<NB, G>(P.j[L::NS - 1], D1, B, lane);

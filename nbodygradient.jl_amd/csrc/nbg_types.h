@@ -88,6 +88,16 @@ struct SysBufs {
   int32_t* done_list;  // during a launch are appended here
 };
 
+// Counters that the waves of a workgroup publish to each other (nbg_split.h).
+// They count over a whole visit, n (n - 1) pairs a step, and wrap after 2^32
+// (30 million steps of 12 bodies): a counter has reached a value when their
+// difference, taken modulo 2^32, is not negative.  The two are never further
+// apart than a ring.
+NBG_TD bool counter_reached(uint32_t have, uint32_t want) { return (int32_t)(have - want) >= 0; }
+// Where they start: 32 short of 2^31, so that every run of some steps passes
+// the point where a signed comparison goes wrong.
+constexpr uint32_t COUNTER_START = 0x7fffffe0u;
+
 // Cooperative workgroups (two waves per system, batch launches only): the
 // HBM slots that carry a transit search's Jacobian snapshot from the wave
 // that integrates to the wave that searches.  Each workgroup owns `stride`
