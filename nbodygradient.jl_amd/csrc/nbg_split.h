@@ -74,7 +74,9 @@ struct JacSlot {
 // bytes -- 16 cycles of the compute unit's LDS per pair of coefficients -- and a wait:
 // an update of 9 bodies' rows took 2,850 cycles of which its arithmetic
 // issues 1,000.  Every lane of the row must be active.  The leading wait keeps
-// a coefficient that was just copied between registers readable by DPP.
+// a coefficient that was just copied between registers readable by DPP.  The
+// accumulators are written before the last inputs are read ("&"), so none may
+// share a register with an input of the same value.
 template <int I, bool NEG = false> __device__ __forceinline__ void fmac6(double* acc, const double* cf, double x) {
 #define NBG_FMAC6(SIGN)                                                                              \
   asm("s_nop 1\n\t"                                                                                  \
@@ -84,7 +86,7 @@ template <int I, bool NEG = false> __device__ __forceinline__ void fmac6(double*
       "v_fmac_f64_dpp %3, %9, " SIGN "%12 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"           \
       "v_fmac_f64_dpp %4, %10, " SIGN "%12 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"          \
       "v_fmac_f64_dpp %5, %11, " SIGN "%12 row_newbcast:%18 row_mask:0xf bank_mask:0xf"              \
-      : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5])           \
+      : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3]), "+&v"(acc[4]), "+&v"(acc[5])     \
       : "v"(cf[I / 16]), "v"(cf[(I + 1) / 16]), "v"(cf[(I + 2) / 16]), "v"(cf[(I + 3) / 16]),        \
         "v"(cf[(I + 4) / 16]), "v"(cf[(I + 5) / 16]), "v"(x), "n"(I % 16), "n"((I + 1) % 16),        \
         "n"((I + 2) % 16), "n"((I + 3) % 16), "n"((I + 4) % 16), "n"((I + 5) % 16))
@@ -99,7 +101,7 @@ template <int I, int M> __device__ __forceinline__ double fmac_body(double s, co
       "v_fmac_f64_dpp %0, %2, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
       "v_fmac_f64_dpp %0, %3, %7 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
       "v_fmac_f64_dpp %0, %4, %8 row_newbcast:%12 row_mask:0xf bank_mask:0xf"
-      : "+v"(s)
+      : "+&v"(s)
       : "v"(cf[I / 16]), "v"(cf[(I + 1) / 16]), "v"(cf[(I + 2) / 16]), "v"(cf[M / 16]), "v"(x[0]), "v"(x[1]), "v"(x[2]),
         "v"(u), "n"(I % 16), "n"((I + 1) % 16), "n"((I + 2) % 16), "n"(M % 16));
   return s;
