@@ -52,20 +52,20 @@ extern "C" hipError_t nbg_launch_group_duo(int cls, nbg::GroupList gl, nbg::SysB
 extern "C" int nbg_duo_pairs(int cls, int n);
 // two waves a workgroup, the state on one and the Jacobian on the other: one
 // system per workgroup, two, or few systems on the whole GPU
-extern "C" hipError_t nbg_launch_split(int cls, nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int64_t bound_job,
+extern "C" hipError_t nbg_launch_split(int cls, nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound,
                                        int grid, unsigned long long* units, unsigned long long* err, hipStream_t stream);
-extern "C" hipError_t nbg_launch_split_duo(nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int64_t bound_job, int grid,
+extern "C" hipError_t nbg_launch_split_duo(nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int grid,
                                            unsigned long long* units, unsigned long long* err, hipStream_t stream);
-extern "C" hipError_t nbg_launch_split_wide(nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int64_t bound_job, int grid,
+extern "C" hipError_t nbg_launch_split_wide(nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int grid,
                                             unsigned long long* units, unsigned long long* err, hipStream_t stream);
 
 namespace {
 
 constexpr int NB_MIN = 2, NB_MAX = 12;
-// Polls of a wait between the waves of nbg_split.h before it is reported as
-// failed: for another wave's work, and for the next step.
-constexpr int64_t SPLIT_POLLS = (int64_t)1 << 24, SPLIT_JOB_POLLS = (int64_t)1 << 40;
-constexpr const char* WAIT_FAILED = "two-wave workgroup: a wait between its two waves timed out";
+// Polls (of 100 to 200 cycles) of a wait between the waves of nbg_split.h
+// before it is reported as failed: about a second, thousands of steps.
+constexpr int64_t SPLIT_POLLS = (int64_t)1 << 24;
+constexpr const char* WAIT_FAILED = "workgroup of several waves: a wait between its waves timed out";
 constexpr int SPLIT_PAIR_MAX = 7;  // bodies of the largest systems paired on the two-wave launches
 
 template <class T> struct DevVec {
@@ -445,7 +445,6 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
   }
   bool any_split = false;
   const int64_t split_bound = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_POLLS;
-  const int64_t split_job = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_JOB_POLLS;
   unsigned long long* const wait_err = S.units.p + 13 * G + 13;
   NBG_HIP(hipEventRecord(ctx->ev0, 0));
   for (int s = 0; s < ns; ++s) NBG_HIP(hipStreamWaitEvent(ctx->streams[s], ctx->ev0, 0));
@@ -597,9 +596,9 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
     if (work > 0 && split[g]) {
       any_split = true;
       unsigned long long* un = S.units.p + 13 * g;
-      NBG_HIP(wide ? nbg_launch_split_wide(gl, B, chunk, split_bound, split_job, grid, un, wait_err, st)
-              : paired[g] ? nbg_launch_split_duo(gl, B, chunk, split_bound, split_job, grid, un, wait_err, st)
-                          : nbg_launch_split(L.gn[g], gl, B, chunk, split_bound, split_job, grid, un, wait_err, st));
+      NBG_HIP(wide ? nbg_launch_split_wide(gl, B, chunk, split_bound, grid, un, wait_err, st)
+              : paired[g] ? nbg_launch_split_duo(gl, B, chunk, split_bound, grid, un, wait_err, st)
+                          : nbg_launch_split(L.gn[g], gl, B, chunk, split_bound, grid, un, wait_err, st));
     } else if (work > 0)
       NBG_HIP(by_unit ? nbg_launch_group_duo(L.gn[g], gl, B, chunk, grid, S.units.p + 13 * g, st)
                       : nbg_launch_group(L.gn[g], gl, B, chunk, grid, S.units.p + 13 * g, st));
@@ -824,9 +823,8 @@ int run_record(nbg_ctx* ctx, const Layout& L, double* x, double* v, double* xe, 
   gl.queue[0] = reinterpret_cast<int*>(V + o_queue);
   unsigned long long* units = reinterpret_cast<unsigned long long*>(V + o_units);
   const int64_t bound = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_POLLS;
-  const int64_t job = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_JOB_POLLS;
   NBG_HIP(move(V, HV, in_words));
-  NBG_HIP(nbg_launch_split_wide(gl, B, 0, bound, job, 1, units, units + 13, s));
+  NBG_HIP(nbg_launch_split_wide(gl, B, 0, bound, 1, units, units + 13, s));
   NBG_HIP(move(HV + o_units, V + o_units, words - o_units));
   NBG_HIP(hipStreamSynchronize(s));
   unsigned long long werr = 0;

@@ -20,8 +20,9 @@
 // three messages a step (PRE: the step's kind, size and velocities; MID: the
 // positions between the sweeps; POST: the final state), each buffer with one
 // writer and one reader, published by workgroup-scope release of a counter.
-// Waits are bounded like those of nbg_run_coop: a failure ends both waves and
-// is reported, it never hangs.
+// Waits are bounded (wait_for, wait_next): one that has polled about a second
+// without an answer, or without a new step of the state wave, ends the
+// workgroup's waves and is reported as an error.
 //
 // Systems with Kepler pairs only and no massless pair (the levels of their
 // sweeps are the same for every system of a body count); every operation is the
@@ -187,6 +188,7 @@ struct SplitCtl {
   uint32_t tail, head;  // pairs published / released, per system
   uint32_t sent, seen;  // messages published / copied
   uint32_t answered;    // steps whose dq/dt is complete
+  uint32_t begun;       // steps the state wave has begun, followed or not (wait_next)
   int quit;           // the state wave is done, or a wait ran out
   int act[2];         // PRE: what the step is
   int body[2];        // PRE: a gradient step's body ...
@@ -225,14 +227,21 @@ template <int NB, bool G, bool TWO, int LIMIT> struct SplitLds {
 
 __device__ __forceinline__ void start_counters(SplitCtl& c, int lane) {
   if (lane != 0) return;
-  c.tail = c.head = c.sent = c.seen = c.answered = COUNTER_START;
+  c.tail = c.head = c.sent = c.seen = c.answered = c.begun = COUNTER_START;
   c.quit = 0;
 }
 __device__ __forceinline__ void publish(uint32_t* counter, uint32_t v, int lane) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   if (lane == 0) ring_store(counter, v);
 }
-// Waits until the counter has reached v; false when the other wave has quit or
+// Ends a wait that found nothing in `bound` polls.
+__device__ __forceinline__ void wait_failed(SplitCtl* ctl, unsigned long long* err, int lane) {
+  if (lane == 0) {
+    atomicOr(err, 4ull);
+    ring_store(&ctl->quit, 2);
+  }
+}
+// Waits until the counter has reached v; false when another wave has quit or
 // the bound runs out.
 __device__ __forceinline__ bool wait_for(const uint32_t* counter, uint32_t v, SplitCtl* ctl, int64_t bound,
                                          unsigned long long* err, int lane) {
@@ -240,10 +249,28 @@ __device__ __forceinline__ bool wait_for(const uint32_t* counter, uint32_t v, Sp
   while (!counter_reached(ring_load(counter), v)) {
     if (ring_load(&ctl->quit) == 2) return false;
     if (++spins > bound) {
-      if (lane == 0) {
-        atomicOr(err, 4ull);
-        ring_store(&ctl->quit, 2);
-      }
+      wait_failed(ctl, err, lane);
+      return false;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  return true;
+}
+// The same for the next step that needs the waiting wave, which may be a whole
+// run away: the bound counts polls since the state wave last began a step.
+__device__ __forceinline__ bool wait_next(const uint32_t* counter, uint32_t v, SplitCtl* ctl, int64_t bound,
+                                          unsigned long long* err, int lane) {
+  int64_t spins = 0;
+  uint32_t begun = ring_load(&ctl->begun);
+  while (!counter_reached(ring_load(counter), v)) {
+    if (ring_load(&ctl->quit) == 2) return false;
+    const uint32_t b = ring_load(&ctl->begun);
+    if (b != begun) {
+      begun = b;
+      spins = 0;
+    } else if (++spins > bound) {
+      wait_failed(ctl, err, lane);
       return false;
     }
     __builtin_amdgcn_s_sleep(1);
@@ -697,10 +724,12 @@ __device__ void split_state(L& P, const SysDesc& D0, const SysDesc& D1, const Sy
   R.n = NB; R.slots = L::RR;
   R.pos = 0; R.made = COUNTER_START;
   R.bound = bound; R.err = err;
-  uint32_t sent = COUNTER_START, asked = COUNTER_START;
+  uint32_t sent = COUNTER_START, asked = COUNTER_START, begun = COUNTER_START;
   const int half = STEP == 32 ? lane >> 5 : 0, col = STEP == 32 ? lane & 31 : lane;
 #pragma unroll 1
   while (c[0].act != ACT_DONE || c[1].act != ACT_DONE) {
+    ++begun;
+    if (lane == 0) ring_store(&ctl->begun, begun);
     const bool a0 = c[0].act != ACT_DONE, a1 = TWO && c[1].act != ACT_DONE;
     double h0 = 0.0, h1 = 0.0;
     int n0 = ACT_DONE, n1 = ACT_DONE;
@@ -1487,7 +1516,7 @@ template <int NB, bool G> __device__ void split_store_jac(JacRec<NB, G>& S, cons
 
 template <int NB, bool G, bool TWO, int LIMIT, bool FACT>
 __device__ void split_jacobian(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0, const SysDesc& D1, const SysBufs& B,
-                               const Visit& v0, const Visit& v1, int lane, int64_t bound, int64_t bound_job,
+                               const Visit& v0, const Visit& v1, int lane, int64_t bound,
                                unsigned long long* err) {
   using L = SplitLds<NB, G, TWO, LIMIT>;
   constexpr int N3 = 3 * NB, N7 = 7 * NB, K = TWO ? 1 : 0;
@@ -1503,7 +1532,7 @@ __device__ void split_jacobian(SplitLds<NB, G, TWO, LIMIT>& P, const SysDesc& D0
   uint32_t seen = COUNTER_START, answered = COUNTER_START;
 #pragma unroll 1
   while (true) {
-    if (!wait_for(&ctl->sent, seen + 1, ctl, bound_job, err, lane)) return;
+    if (!wait_next(&ctl->sent, seen + 1, ctl, bound, err, lane)) return;
     const int n0 = __builtin_amdgcn_readfirstlane(ctl->act[0]);
     if (n0 < 0) break;
     const int n1 = TWO ? __builtin_amdgcn_readfirstlane(ctl->act[1]) : (int)ACT_DONE;
@@ -1703,8 +1732,7 @@ __device__ __attribute__((always_inline)) inline bool pair_wave_sweep(SplitLds3<
 }
 
 template <int NB, int LIMIT, bool FACT>
-__device__ void pair_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBufs& B, const Visit& v, int lane, int64_t bound,
-                          int64_t bound_job, unsigned long long* err) {
+__device__ void pair_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBufs& B, const Visit& v, int lane, int64_t bound, unsigned long long* err) {
   constexpr int N3 = 3 * NB, N7 = 7 * NB;
   SplitCtl* ctl = &P.ctl;
   RowCtl* row = &P.row;
@@ -1714,7 +1742,7 @@ __device__ void pair_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBu
   int pos = 0;
 #pragma unroll 1
   while (true) {
-    if (!wait_for(&ctl->sent, seen + 1, ctl, bound_job, err, lane)) return;
+    if (!wait_next(&ctl->sent, seen + 1, ctl, bound, err, lane)) return;
     const int need = __builtin_amdgcn_readfirstlane(ctl->act[0]);
     const bool needJ = need >= 0 && (need & SPLIT_J) != 0, needQ = need >= 0 && (need & SPLIT_Q) != 0;
     const double h = ctl->h[0];
@@ -1782,8 +1810,7 @@ __device__ void pair_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBu
 }
 
 template <int NB, int LIMIT, bool FACT>
-__device__ void row_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBufs& B, const Visit& v, int lane, int64_t bound,
-                         int64_t bound_job, unsigned long long* err) {
+__device__ void row_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBufs& B, const Visit& v, int lane, int64_t bound, unsigned long long* err) {
   using L = SplitLds3<NB, LIMIT>;
   constexpr int NL = level_count(NB);
   SplitCtl* ctl = &P.ctl;
@@ -1792,7 +1819,7 @@ __device__ void row_wave(SplitLds3<NB, LIMIT>& P, const SysDesc& D, const SysBuf
   uint32_t steps = COUNTER_START, ends = COUNTER_START, chunk = COUNTER_START;
 #pragma unroll 1
   while (true) {
-    if (!wait_for(&row->heads, steps + 1, ctl, bound_job, err, lane)) return;
+    if (!wait_next(&row->heads, steps + 1, ctl, bound, err, lane)) return;
     const RowHeader& H = row->hdr[steps & 1];
     const int need = __builtin_amdgcn_readfirstlane(H.need);
     if (need < 0) break;
@@ -1876,8 +1903,7 @@ __device__ inline bool split_follows(const SysDesc& D) { return D.grad || D.mode
 
 // One visit of a system by a workgroup of three waves.
 template <int NB, int LIMIT>
-__device__ void split_run3(unsigned char* raw, int wave, const SysDesc& D, const SysBufs& B, int64_t chunk, int64_t bound,
-                           int64_t bound_job, unsigned long long* err, int lane) {
+__device__ void split_run3(unsigned char* raw, int wave, const SysDesc& D, const SysBufs& B, int64_t chunk, int64_t bound, unsigned long long* err, int lane) {
   using L = SplitLds3<NB, LIMIT>;
   L& P = *reinterpret_cast<L*>(raw);
   static_assert(sizeof(L) <= (size_t)LIMIT, "LDS");
@@ -1897,11 +1923,11 @@ __device__ void split_run3(unsigned char* raw, int wave, const SysDesc& D, const
     split_state<NB, false>(P, D, D, B, v, none, lane, bound, err);
   } else if (split_follows(D)) {
     if (wave == 1) {
-      if (D.rowupd) pair_wave<NB, LIMIT, true>(P, D, B, v, lane, bound, bound_job, err);
-      else pair_wave<NB, LIMIT, false>(P, D, B, v, lane, bound, bound_job, err);
+      if (D.rowupd) pair_wave<NB, LIMIT, true>(P, D, B, v, lane, bound, err);
+      else pair_wave<NB, LIMIT, false>(P, D, B, v, lane, bound, err);
     } else {
-      if (D.rowupd) row_wave<NB, LIMIT, true>(P, D, B, v, lane, bound, bound_job, err);
-      else row_wave<NB, LIMIT, false>(P, D, B, v, lane, bound, bound_job, err);
+      if (D.rowupd) row_wave<NB, LIMIT, true>(P, D, B, v, lane, bound, err);
+      else row_wave<NB, LIMIT, false>(P, D, B, v, lane, bound, err);
     }
   }
   __syncthreads();  // every row is written
@@ -1910,13 +1936,13 @@ __device__ void split_run3(unsigned char* raw, int wave, const SysDesc& D, const
 }
 template <int N, int HI, int LIMIT>
 __device__ __forceinline__ void split_dispatch3(unsigned char* raw, int wave, const SysDesc& D, const SysBufs& B, int64_t chunk,
-                                                int64_t bound, int64_t bound_job, unsigned long long* err, int lane) {
+                                                int64_t bound, unsigned long long* err, int lane) {
   if constexpr (N <= HI) {
     if (D.n == N) {
-      split_run3<N, LIMIT>(raw, wave, D, B, chunk, bound, bound_job, err, lane);
+      split_run3<N, LIMIT>(raw, wave, D, B, chunk, bound, err, lane);
       return;
     }
-    split_dispatch3<N + 1, HI, LIMIT>(raw, wave, D, B, chunk, bound, bound_job, err, lane);
+    split_dispatch3<N + 1, HI, LIMIT>(raw, wave, D, B, chunk, bound, err, lane);
   }
 }
 
@@ -1924,7 +1950,7 @@ __device__ __forceinline__ void split_dispatch3(unsigned char* raw, int wave, co
 // waves.
 template <int NB, bool G, bool TWO, int LIMIT>
 __device__ void split_run(unsigned char* raw, int wave, const SysDesc& D0, const SysDesc& D1, const SysBufs& B, int64_t chunk0,
-                          int64_t chunk1, bool pair, int64_t bound, int64_t bound_job, unsigned long long* err, int lane) {
+                          int64_t chunk1, bool pair, int64_t bound, unsigned long long* err, int lane) {
   using L = SplitLds<NB, G, TWO, LIMIT>;
   L& P = *reinterpret_cast<L*>(raw);
   const Visit v0 = visit_of(D0, B, chunk0);
@@ -1942,8 +1968,8 @@ __device__ void split_run(unsigned char* raw, int wave, const SysDesc& D0, const
   if (wave == 0) {
     split_state<NB, TWO>(P, D0, D1, B, v0, v1, lane, bound, err);
   } else if (split_follows(D0) || (pair && split_follows(D1))) {
-    if (D0.rowupd) split_jacobian<NB, G, TWO, LIMIT, true>(P, D0, D1, B, v0, v1, lane, bound, bound_job, err);
-    else split_jacobian<NB, G, TWO, LIMIT, false>(P, D0, D1, B, v0, v1, lane, bound, bound_job, err);
+    if (D0.rowupd) split_jacobian<NB, G, TWO, LIMIT, true>(P, D0, D1, B, v0, v1, lane, bound, err);
+    else split_jacobian<NB, G, TWO, LIMIT, false>(P, D0, D1, B, v0, v1, lane, bound, err);
   }
   __syncthreads();  // every row is written
   if (D0.mode == MODE_TRANSITS && D0.grad && v0.begin <= D0.nsteps && v0.end == v0.total)
@@ -1963,14 +1989,14 @@ template <int NB, int LIMIT> constexpr bool split_pairs() {
 }
 template <int N, int HI, bool TWO, int LIMIT>
 __device__ __forceinline__ void split_dispatch(unsigned char* raw, int wave, const SysDesc& D0, const SysDesc& D1,
-                                               const SysBufs& B, int64_t c0, int64_t c1, bool pair, int64_t bound, int64_t bound_job,
+                                               const SysBufs& B, int64_t c0, int64_t c1, bool pair, int64_t bound,
                                                unsigned long long* err, int lane) {
   if constexpr (N <= HI) {
     if (D0.n == N) {
-      split_run<N, split_global<N, TWO, LIMIT>(), TWO, LIMIT>(raw, wave, D0, D1, B, c0, c1, pair, bound, bound_job, err, lane);
+      split_run<N, split_global<N, TWO, LIMIT>(), TWO, LIMIT>(raw, wave, D0, D1, B, c0, c1, pair, bound, err, lane);
       return;
     }
-    split_dispatch<N + 1, HI, TWO, LIMIT>(raw, wave, D0, D1, B, c0, c1, pair, bound, bound_job, err, lane);
+    split_dispatch<N + 1, HI, TWO, LIMIT>(raw, wave, D0, D1, B, c0, c1, pair, bound, err, lane);
   }
 }
 
@@ -1979,7 +2005,7 @@ __device__ __forceinline__ void split_dispatch(unsigned char* raw, int wave, con
 // workgroup's LDS.  units[13] collects wait failures.
 template <int HI, bool TWO, int LIMIT, bool THREE = false>
 __device__ __forceinline__ void split_body(unsigned char* raw, int* share, const GroupList& gl, const SysBufs& B, int64_t chunk,
-                                           int64_t bound, int64_t bound_job, unsigned long long* units,
+                                           int64_t bound, unsigned long long* units,
                                            unsigned long long* err) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE;
@@ -2010,8 +2036,8 @@ __device__ __forceinline__ void split_body(unsigned char* raw, int* share, const
     const int64_t before1 = ints1[D1.n], tr01 = ints1[D1.n + 1], it01 = ints1[D1.n + 2];
     const int64_t c0 = D0.chunk > 0 ? D0.chunk : chunk, c1 = D1.chunk > 0 ? D1.chunk : chunk;
     __syncthreads();  // both waves have read the counters
-    if constexpr (THREE) split_dispatch3<2, HI, LIMIT>(raw, wave, D0, B, c0, bound, bound_job, err, lane);
-    else split_dispatch<2, HI, TWO, LIMIT>(raw, wave, D0, D1, B, c0, c1, two, bound, bound_job, err, lane);
+    if constexpr (THREE) split_dispatch3<2, HI, LIMIT>(raw, wave, D0, B, c0, bound, err, lane);
+    else split_dispatch<2, HI, TWO, LIMIT>(raw, wave, D0, D1, B, c0, c1, two, bound, err, lane);
     if (threadIdx.x == 0) {
       visit_done(D0, ints0, before0, tr00, it00, B, units);
       if (two) visit_done(D1, ints1, before1, tr01, it01, B, units);

@@ -6,19 +6,18 @@
 namespace nbg {
 
 template <int HI, int LIMIT>
-__global__ __launch_bounds__(3 * WAVE, 1) void nbg_run_split_wide(GroupList gl, SysBufs B, int64_t chunk, int64_t bound, int64_t bound_job,
+__global__ __launch_bounds__(3 * WAVE, 1) void nbg_run_split_wide(GroupList gl, SysBufs B, int64_t chunk, int64_t bound,
                                                                   unsigned long long* __restrict__ units,
                                                                   unsigned long long* __restrict__ err) {
   __shared__ __attribute__((aligned(16))) unsigned char raw[LIMIT];
   __shared__ int share;
-  split_body<HI, false, LIMIT, true>(raw, &share, gl, B, chunk, bound, bound_job, units, err);
+  split_body<HI, false, LIMIT, true>(raw, &share, gl, B, chunk, bound, units, err);
 }
 
 }  // namespace nbg
 
-extern "C" hipError_t nbg_launch_split_wide(nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int64_t bound_job, int grid,
+extern "C" hipError_t nbg_launch_split_wide(nbg::GroupList gl, nbg::SysBufs bufs, int64_t chunk, int64_t bound, int grid,
                                             unsigned long long* units, unsigned long long* err, hipStream_t stream) {
-  hipLaunchKernelGGL((nbg::nbg_run_split_wide<12, 163776>), dim3(grid), dim3(3 * nbg::WAVE), 0, stream, gl, bufs, chunk, bound,
-                     bound_job, units, err);
+  hipLaunchKernelGGL((nbg::nbg_run_split_wide<12, 163776>), dim3(grid), dim3(3 * nbg::WAVE), 0, stream, gl, bufs, chunk, bound, units, err);
   return hipGetLastError();
 }
