@@ -328,10 +328,13 @@ int nbg_set_systems_per_wave(nbg_ctx* ctx, int32_t k);
  * neither, stay bitwise. */
 int nbg_set_row_update(nbg_ctx* ctx, int32_t mode);
 /* Diagnostic only (no counterpart in the reference): bound every wait between
- * the two waves of a cooperative workgroup to `polls` polls (0: the defaults,
- * ~1 s for a free search slot and ~2 min for the next search).  A wait that
- * runs out makes the launch return an error instead of hanging; tests use a
- * tiny bound to check that path. */
+ * the waves of a workgroup, in runs with a transit search, to `polls` polls
+ * (0: the defaults; cooperative workgroups ~1 s for a free search slot and
+ * ~2 min for the next search, workgroups that divide a step between two or
+ * three waves ~1 s without an answer or a new step).  A wait that runs out
+ * makes the launch return an error instead of hanging; tests use a tiny bound
+ * to check that path.  Steps and trajectories, and every run with
+ * nbg_set_coop mode 0, keep the defaults. */
 int nbg_set_coop_wait(nbg_ctx* ctx, int64_t polls);
 
 /* Diagnostic only (no counterpart in the reference): a plain device copy of

@@ -331,7 +331,7 @@ struct nbg_ctx {
   int coop_max = 128;  // at most this many cooperative systems per batch
   int systems_per_wave = 1;  // batches: 2 runs transit systems of equal body count two per wave (nbg_run_duo)
   int row_update = 0;        // Jacobian row update: 0 the reference's order (bitwise), 1 factored
-  int64_t coop_polls = 0;  // > 0: bound on every inter-wave wait (diagnostic); 0: the defaults
+  int64_t coop_polls = 0;  // > 0: bound on the inter-wave waits of transit runs (diagnostic); 0: the defaults
   int nstreams = 4;
   std::vector<hipStream_t> streams;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -369,6 +369,13 @@ struct nbg_batch {
   } while (0)
 
 namespace {
+
+// Polls of a wait on the two- and three-wave launches.  nbg_set_coop_wait
+// bounds runs that may take cooperative workgroups: with a transit search, and
+// not turned off.
+int64_t wait_bound(const nbg_ctx* ctx, int mode) {
+  return ctx->coop_polls > 0 && ctx->coop_mode != 0 && mode == nbg::MODE_TRANSITS ? ctx->coop_polls : SPLIT_POLLS;
+}
 
 int grid_for(nbg_ctx* ctx, int nb, int nsys) {
   const size_t lds = nbg_lds_bytes(nb);
@@ -444,7 +451,7 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
     if (!split[g] || paired[g]) wide = false;
   }
   bool any_split = false;
-  const int64_t split_bound = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_POLLS;
+  const int64_t split_bound = wait_bound(ctx, L.desc[0].mode);  // a layout's systems are of one mode
   unsigned long long* const wait_err = S.units.p + 13 * G + 13;
   NBG_HIP(hipEventRecord(ctx->ev0, 0));
   for (int s = 0; s < ns; ++s) NBG_HIP(hipStreamWaitEvent(ctx->streams[s], ctx->ev0, 0));
@@ -822,7 +829,7 @@ int run_record(nbg_ctx* ctx, const Layout& L, double* x, double* v, double* xe, 
   gl.descs[0] = reinterpret_cast<const nbg::SysDesc*>(V + o_desc);
   gl.queue[0] = reinterpret_cast<int*>(V + o_queue);
   unsigned long long* units = reinterpret_cast<unsigned long long*>(V + o_units);
-  const int64_t bound = ctx->coop_polls > 0 ? ctx->coop_polls : SPLIT_POLLS;
+  const int64_t bound = wait_bound(ctx, D.mode);
   NBG_HIP(move(V, HV, in_words));
   NBG_HIP(nbg_launch_split_wide(gl, B, 0, bound, 1, units, units + 13, s));
   NBG_HIP(move(HV + o_units, V + o_units, words - o_units));

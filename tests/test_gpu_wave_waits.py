@@ -3,14 +3,15 @@ wait bounded to a single poll, a run on each of the launches -- a compute unit a
 system, more systems than compute units, two systems a workgroup -- ends and
 reports the failure, and the next one, with the default bounds, gives the usual
 results.  A wave that has nothing to do for a whole run (no gradient, no
-transit) does not run out of its bound while the state wave steps on."""
+transit) does not run out of its bound while the state wave steps on.  The bound
+is one on transit runs with cooperative workgroups allowed: others never had it."""
 import numpy as np
 import pytest
 
 import oracle_lib as O
 import nbodygradient_amd as nb
 from nbodygradient_amd import workloads as W
-from nbodygradient_amd.batch import Batch
+from nbodygradient_amd.batch import Batch, cartesian_batch
 
 pytestmark = pytest.mark.gpu
 
@@ -95,3 +96,28 @@ def test_a_run_without_work_for_a_wave_is_no_failure(copies):
     for q, s in enumerate(specs):
         _check(s, states[q], res[q], False)
         assert res[q]["count"].sum() == 0
+
+
+def test_other_runs_are_not_bounded():
+    print("gpu: a wait bound and runs it does not reach", flush=True)
+    spec = _specs([4], 820, 60)[0]
+    (x, v, j), = W.initial_states([spec], processes=1)
+    ctx = nb.default_context()
+    ctx.set_coop_wait(1)
+    try:
+        st = nb.State(nb.ElementsIC(spec.t0, spec.n, spec.elements))
+        os_ = O.OState(st.x.copy(), st.v.copy(), spec.elements[:, 0], t=spec.t0)
+        end = spec.t0 + 10 * spec.h
+        nb.Integrator(spec.h, spec.t0, end)(st, end, grad=True)
+        O.integrate_to(os_, spec.h, end, grad=True)
+        for k in ("x", "v", "jac_step", "jac_error", "dqdt"):
+            assert np.array_equal(getattr(st, k), getattr(os_, k)), k
+        got = cartesian_batch([spec], [7], states=[(x, v, j)], jacobian=True)[0]
+        os_ = O.OState(x, v, spec.elements[:, 0], t=spec.t0, jac_init=j)
+        rec = O.cartesian_output(os_, spec.h, spec.tmax, 7)
+        assert np.array_equal(got["x"], rec["x"]) and np.array_equal(got["jac_step"], rec["jac_step"])
+        ctx.set_coop(0, 0)  # no cooperative workgroups, no bound
+        _check(spec, (x, v, j), _run([spec], [(x, v, j)])[0], True)
+    finally:
+        ctx.set_coop(1, 128)
+        ctx.set_coop_wait(0)
