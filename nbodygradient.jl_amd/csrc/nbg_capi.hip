@@ -591,7 +591,10 @@ int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* k
     }
     const int grid = wide ? std::max(1, std::min({(int)L.desc.size(), ctx->cu_count, ctx->grid_cap > 0 ? ctx->grid_cap : INT_MAX}))
                           : grids[g];
-    if (wide && group_grid) (*group_grid)[g] = grid;
+    if (wide && group_grid) {  // the one launch there is
+      group_grid->assign(G, 0);
+      (*group_grid)[g] = grid;
+    }
     if (K > 0) load[0] += 1e30;  // the cooperative launch holds stream 0
     const int si = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     load[si] += L.gcost[g] / grid;
