@@ -431,15 +431,10 @@ template <int NB, bool G> __device__ void kick_build(Smem<NB, G>& S, Swork<NB>& 
 // col = lane) or two on its halves (STEP = 32, phi_build2).  The lane of
 // body d's coordinate p writes the acceleration a[p, d]; col 0 writes the
 // other uniform values (v, dqdt_phi).  FACT: jac_phi in the factored form.
-// STATE: the velocities are updated too (a record that carries them).
-template <int NB, bool G, int STEP, bool FACT = false, bool STATE = true, class R, class WK>
-__device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W, double h, bool anyKick, bool needQ,
-                                                                     int col) {
+template <int NB, bool G, int STEP, bool FACT = false>
+__device__ __attribute__((always_inline)) inline void phisalpha_cols(Smem<NB, G>& S, Swork<NB>& W, double h, bool anyKick,
+                                                                     bool needQ, int col) {
   constexpr int N3 = 3 * NB, N4 = 4 * NB;
-  auto kicked = [](const R& rec, bool any, int i, int j) {
-    if constexpr (STATE) return any && rec.pair[i + NB * j];
-    else return false;
-  };
   const bool own = col < N4;
   int myd = -1, myp = -1;
   if (own) col_dp<NB>(col, myd, myp);
@@ -457,7 +452,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
   // order; looping over the partner c in increasing order therefore repeats
   // every accumulation in the reference's order.  a and dadq start at zero
   // (ahl21.jl:559-563); jac_phi keeps phic!'s terms.
-  constexpr int NP = WK::NP, PQ = WK::PQ;
+  constexpr int NP = Swork<NB>::NP, PQ = Swork<NB>::PQ;
   double* pq = W.f.pq;
   auto pidx = [](int i, int j) { return i * (2 * NB - i - 1) / 2 + (j - i - 1); };
   const double coeff = (((2.0 * (h * h * h)) / 96.0) * 2.0) * NBG_GNEWT;
@@ -500,7 +495,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
       const int i = b < myd ? b : myd, j = b < myd ? myd : b;
       const bool bi = (b == i);
       double t[3] = {0.0, 0.0, 0.0};
-      if (!kicked(S, anyKick, i, j)) {
+      if (!(anyKick && S.pair[i + NB * j])) {
         const double* o = pq + pidx(i, j) * PQ;
         const double m = S.m[myd];  // b's partner's mass
         const double f2m = o[0] * m;
@@ -522,7 +517,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
     for (int c = 0; c < NB; ++c) {
       if (c == myd) continue;
       const int i = c < myd ? c : myd, j = c < myd ? myd : c;
-      if (kicked(S, anyKick, i, j)) continue;
+      if (anyKick && S.pair[i + NB * j]) continue;
       const double* o = pq + pidx(i, j) * PQ;
       const bool bi = (myd == i);
       const double m = S.m[c];  // the partner's mass
@@ -595,11 +590,8 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
     for (int i = 0; i < NB - 1; ++i) {
       double vi[3], vie[3], qi[3], pi[3], xi[3], Di[3];
       for (int k = 0; k < 3; ++k) {
-        vi[k] = vie[k] = 0.0;
-        if constexpr (STATE) {
-          vi[k] = S.v[3 * i + k];
-          vie[k] = S.ve[3 * i + k];
-        }
+        vi[k] = S.v[3 * i + k];
+        vie[k] = S.ve[3 * i + k];
         qi[k] = needQ ? S.dqdt_phi[7 * i + 3 + k] : 0.0;
         pi[k] = own ? PHI[(3 * i + k) * N4 + col] : 0.0;
         xi[k] = S.x[3 * i + k];
@@ -609,18 +601,15 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
       const bool di = myd == i;
 #pragma unroll 1
       for (int j = i + 1; j < NB; ++j, ++p) {
-        if (kicked(S, anyKick, i, j)) continue;
+        if (anyKick && S.pair[i + NB * j]) continue;
         const double* o = pq + p * PQ;
         const double mj = S.m[j];
         double rij[3], Dj[3], vj[3], vje[3], qj[3], pj[3];
         for (int k = 0; k < 3; ++k) {
           rij[k] = xi[k] - S.x[3 * j + k];
           Dj[k] = own ? D[(3 * j + k) * N4 + col] : 0.0;
-          vj[k] = vje[k] = 0.0;
-          if constexpr (STATE) {
-            vj[k] = S.v[3 * j + k];
-            vje[k] = S.ve[3 * j + k];
-          }
+          vj[k] = S.v[3 * j + k];
+          vje[k] = S.ve[3 * j + k];
           qj[k] = needQ ? S.dqdt_phi[7 * j + 3 + k] : 0.0;
           pj[k] = own ? PHI[(3 * j + k) * N4 + col] : 0.0;
         }
@@ -633,10 +622,8 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
           const double fac = o[k];
-          if constexpr (STATE) {
-            kahan(vi[k], vie[k], mj * fac);
-            kahan(vj[k], vje[k], -(mi * fac));
-          }
+          kahan(vi[k], vie[k], mj * fac);
+          kahan(vj[k], vje[k], -(mi * fac));
           if (needQ) {
             qi[k] += (q3h * mj) * fac;
             qj[k] += -((q3h * mi) * fac);
@@ -651,10 +638,8 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
         for (int k = 0; k < 3; ++k) {
           if (own) PHI[(3 * j + k) * N4 + col] = pj[k];
           if (col == 0) {
-            if constexpr (STATE) {
-              S.v[3 * j + k] = vj[k];
-              S.ve[3 * j + k] = vje[k];
-            }
+            S.v[3 * j + k] = vj[k];
+            S.ve[3 * j + k] = vje[k];
             if (needQ) S.dqdt_phi[7 * j + 3 + k] = qj[k];
           }
         }
@@ -662,10 +647,8 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
       for (int k = 0; k < 3; ++k) {
         if (own) PHI[(3 * i + k) * N4 + col] = pi[k];
         if (col == 0) {
-          if constexpr (STATE) {
-            S.v[3 * i + k] = vi[k];
-            S.ve[3 * i + k] = vie[k];
-          }
+          S.v[3 * i + k] = vi[k];
+          S.ve[3 * i + k] = vie[k];
           if (needQ) S.dqdt_phi[7 * i + 3 + k] = qi[k];
         }
       }
@@ -675,11 +658,8 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
   for (int b = 0; b < NB; ++b) {
     double vb[3], veb[3], qb[3], pb[3];
     for (int k = 0; k < 3; ++k) {
-      vb[k] = veb[k] = 0.0;
-      if constexpr (STATE) {
-        vb[k] = S.v[3 * b + k];
-        veb[k] = S.ve[3 * b + k];
-      }
+      vb[k] = S.v[3 * b + k];
+      veb[k] = S.ve[3 * b + k];
       qb[k] = needQ ? S.dqdt_phi[7 * b + 3 + k] : 0.0;
       pb[k] = (anyKick && own) ? PHI[(3 * b + k) * N4 + col] : 0.0;
     }
@@ -687,7 +667,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
     for (int c = 0; c < NB; ++c) {
       if (c == b) continue;
       const int i = c < b ? c : b, j = c < b ? b : c;
-      if (kicked(S, anyKick, i, j)) continue;
+      if (anyKick && S.pair[i + NB * j]) continue;
       const double* o = pq + pidx(i, j) * PQ;
       double rij[3], Di[3], Dj[3];
       for (int k = 0; k < 3; ++k) {
@@ -709,7 +689,7 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
       for (int k = 0; k < 3; ++k) {
         const double fac = o[k], f5 = fac * o[3], fm = o[4 + k], fr = o[7 + k], ff = o[10] * rij[k];
         const double mf = m * fac;
-        if constexpr (STATE) kahan(vb[k], veb[k], bi ? mf : -mf);
+        kahan(vb[k], veb[k], bi ? mf : -mf);
         if (needQ) {
           const double qm = (q3h * m) * fac;
           qb[k] += bi ? qm : -qm;
@@ -733,10 +713,8 @@ __device__ __attribute__((always_inline)) inline void phisalpha_cols(R& S, WK& W
       for (int k = 0; k < 3; ++k) PHI[(3 * b + k) * N4 + col] = pb[k];
     if (col == 0)
       for (int k = 0; k < 3; ++k) {
-        if constexpr (STATE) {
-          S.v[3 * b + k] = vb[k];
-          S.ve[3 * b + k] = veb[k];
-        }
+        S.v[3 * b + k] = vb[k];
+        S.ve[3 * b + k] = veb[k];
         if (needQ) S.dqdt_phi[7 * b + 3 + k] = qb[k];
       }
   }
@@ -969,8 +947,8 @@ template <int NB, class R> __device__ inline void drift_cols(R& S, int c, double
 // running sum starts at +0 and can never become -0, so the sign of a zero
 // coefficient cannot change it), and the mass columns 6 and 13 take their
 // coefficients from the slot, where pair_jacobian stored them.
-template <int NB, bool G, bool FACT = false, class R, class SL>
-__device__ inline void pair_cols(R& S, const SL& sl, int i, int j, int c) {
+template <int NB, bool G, bool FACT = false>
+__device__ inline void pair_cols(Smem<NB, G>& S, const PairSlot& sl, int i, int j, int c) {
   const auto J_ = jj<NB>(S);
   constexpr int N7 = 7 * NB;
   const int ri = 6 * i, rj = 6 * j;
