@@ -419,7 +419,7 @@ def main():
             (out["rounds_reference_order"]["value"], np.mean(rms)))
     ctx.set_row_update(0)  # the side legs below run the library's default form
     if not args.no_makespan and fits(45, "c2_makespan"):
-        ctx.set_coop(1, 128)  # whole runs: the automatic two-wave selection, four one-wave groups per CU
+        ctx.set_coop(1, 128)  # whole runs: the automatic cooperative selection, four workgroups per CU
         ctx.set_launch(0)
         batch.reset()
         t = time.perf_counter()
@@ -428,7 +428,7 @@ def main():
         out["c2_makespan"] = {"wall_s": wall, "device_s": st["kernel_ms"] / 1e3, "system_steps": st["system_steps"],
                               "transits": st["transits"], "system_steps_per_s": st["system_steps"] / wall,
                               "what": "the 4096-system batch once to completion (every system to its tmax), "
-                                      "the longest systems on two-wave workgroups (automatic)"}
+                                      "cooperative workgroups selected automatically"}
         log("makespan: %.2f s wall, %d system-steps, %d transits" % (wall, st["system_steps"], st["transits"]))
     plain_rate = None
     if not args.no_plain and fits(15, "plain_gpu"):

@@ -138,15 +138,17 @@ typedef struct {
   double kernel_ms;        /* device time of the last run (HIP events, all launches) */
   /* Per launch, indexed by its class c (the largest body count it serves:
    * n = 2..9 share class 9, every larger n has its own; index 1 is the
-   * two-wave launch of nbg_set_coop): device time (HIP
+   * cooperative launch of nbg_set_coop): device time (HIP
    * events on the stream it ran on) and the work units it completed per body
    * count n, launch_units[c][n] (main steps + one per recorded transit when
    * grad != 0).  A launch runs its own class first, then takes systems of
-   * smaller classes.  Entries of absent classes are 0. */
+   * smaller classes; a batch of Kepler pairs with a compute unit to each
+   * system is one launch, its largest class's.  Entries of classes without a
+   * launch are 0. */
   double launch_ms[13];
   int64_t launch_units[13][13];
-  int32_t launch_grid[13];  /* workgroups (one wave each) of that launch */
-  int32_t paired_systems;   /* systems the queues paired two per wave (nbg_set_systems_per_wave) */
+  int32_t launch_grid[13];  /* workgroups of that launch (a wave each; two or three where a step is divided, nbg_batch_run) */
+  int32_t paired_systems;   /* systems the queues paired (nbg_set_systems_per_wave) */
 } nbg_batch_stats;
 
 int nbg_batch_create(nbg_ctx* ctx, int32_t nsys, const int32_t* n, const double* h, const double* tmax,
@@ -177,10 +179,10 @@ int nbg_batch_initial(nbg_batch* b, double* x, double* v, double* jac_init);
 int nbg_batch_autotune_round(nbg_batch* b, int64_t steps, int32_t* best, double* cand_ms, int32_t max_cand);
 /* Autotuner (no counterpart in the reference): runs a copy of batch b with
  * every system's step count scaled by frac (0 < frac <= 1) under each
- * candidate launch configuration -- the workgroup form (two-wave workgroups
- * for the longest systems: off, automatic, or the 16/32/64 longest), the
- * one-wave workgroups per CU and the systems per wave (one, or two for the
- * paired body counts) -- and keeps the fastest in b's context (the values
+ * candidate launch configuration -- cooperative workgroups for the longest
+ * systems (off, automatic, or the 16/32/64 longest), the workgroups per CU
+ * and the systems per workgroup (one, or two for the paired body counts) --
+ * and keeps the fastest in b's context (the values
  * nbg_set_coop, nbg_set_launch and nbg_set_systems_per_wave set).  cand_ms[c] receives candidate
  * c's device time for c < max_cand (may be NULL), *best the chosen index.
  * The copy needs as much device memory as b.  The batch itself is not run. */
@@ -189,15 +191,20 @@ int nbg_batch_autotune(nbg_batch* b, double frac, int32_t* best, double* cand_ms
  * and its workgroups per CU, 0 = as LDS allows); returns the number of
  * candidates. */
 int nbg_batch_autotune_candidate(int32_t index, int32_t* coop_mode, int32_t* coop_max, int32_t* groups_per_cu);
-/* The systems per wave (1 or 2) of autotuner candidate `index`; -1 when
+/* The systems per workgroup (1 or 2) of autotuner candidate `index`; -1 when
  * there is no such candidate. */
 int32_t nbg_batch_autotune_systems_per_wave(int32_t index);
 /* Restore every system to its initial state (device-side copy). */
 int nbg_batch_reset(nbg_batch* b);
 /* Integrate all systems to completion: one persistent launch per class of
  * body counts (2..9 together, then 10, 11, 12 alone), systems longest first
- * within a launch, launches overlapped on streams; the longest systems may
- * run on two-wave workgroups in a launch of their own (nbg_set_coop). */
+ * within a launch, launches overlapped on streams.  A class whose pairs are
+ * all Kepler pairs, none of them massless, divides every step between two
+ * waves of a workgroup, the state on one and the Jacobian on the other (three
+ * waves, all classes in one launch, where the batch leaves a compute unit to
+ * each system); one kicked or massless pair keeps its class on one wave a
+ * system, whose longest systems may run on cooperative workgroups in a launch
+ * of their own (nbg_set_coop).  Results are the same bits either way. */
 int nbg_batch_run(nbg_batch* b, nbg_batch_stats* stats);
 /* One round of a batch (the unit of the throughput benchmark; no
  * counterpart in the reference): every system advances at most `steps`
@@ -290,26 +297,30 @@ int nbg_set_launch(nbg_ctx* ctx, int32_t max_groups_per_cu, int32_t streams);
 /* Upper bound on persistent workgroups per launch (0 = no bound). */
 int nbg_set_grid_cap(nbg_ctx* ctx, int32_t grid_cap);
 /* Cooperative workgroups of batch runs (no counterpart in the reference):
- * a system of at most 9 bodies with a transit search can run on a workgroup
+ * a system of at most 10 bodies with a transit search can run on a workgroup
  * of two waves, the second running its transit searches (findtransit!,
  * timing.jl:30-110) from snapshots while the first integrates; results are
  * bitwise those of the one-wave kernel.  mode 0: off; 1 (default): in
  * batch runs, the systems whose estimated time exceeds the batch's work
  * spread over every wave slot of the GPU (the ones that would set the
- * batch's end); 2: the longest ones regardless, in batch runs and serving
- * rounds.  At most max_systems per launch (default 128); n <= 10. */
+ * batch's end), of classes on one wave a system (nbg_batch_run: the others
+ * have a second wave already); 2: the longest ones regardless of that, in
+ * batch runs, serving rounds and single runs.  At most max_systems per launch
+ * (default 128). */
 int nbg_set_coop(nbg_ctx* ctx, int32_t mode, int32_t max_systems);
 /* Systems per wave of batch runs and rounds (no counterpart in the
  * reference; the pair-to-lane mapping of the pair sweeps ahl21.jl:25-78).
- * k = 1 (default): one system per wave, a level's Kepler pairs one per lane.
- * k = 2: transit runs of equal body count run two per wave in lockstep
- * (every n <= 9; n = 10 too where the n = 12 launch takes it; two records
- * with their Jacobians in HBM and one shared work area fit the LDS of the
- * launch's one-system layouts, so occupancy is unchanged): the Kepler drifts
- * and pair Jacobians of both systems' levels share the lanes; the rest of
- * each step, and the transit searches, run for one system, then the other.
- * Results are bitwise those of k = 1.  Serving rounds keep one system per
- * wave. */
+ * k = 1 (default): one system a workgroup.  k = 2: transit runs of equal body
+ * count may run two a workgroup in lockstep, where the batch is larger than
+ * what the GPU holds at once: the Kepler drifts and pair Jacobians of both
+ * systems' levels share a wave's lanes; the rest of each step, and the
+ * transit searches, run for one system, then the other (small systems: on
+ * half a wave each).  Classes that divide a step between two waves
+ * (nbg_batch_run) pair up to n = 7; classes on one wave every n <= 9, and
+ * n = 10 where the n = 12 launch takes it (two records with their Jacobians
+ * in HBM and one shared work area fit the LDS of the launch's one-system
+ * layouts, so occupancy is unchanged).  Results are bitwise those of k = 1.
+ * Serving rounds keep one system a workgroup. */
 int nbg_set_systems_per_wave(nbg_ctx* ctx, int32_t k);
 /* Form of the Jacobian updates (every launch of ctx): the chain product
  * J += jac_ij * J of the pair sweeps (ahl21.jl:31-42,60-72) and phisalpha!'s

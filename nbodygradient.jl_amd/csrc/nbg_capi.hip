@@ -329,7 +329,7 @@ struct nbg_ctx {
   int grid_cap = 0;
   int coop_mode = 1;   // 0 off, 1 systems longer than the batch's throughput bound, 2 the longest ones
   int coop_max = 128;  // at most this many cooperative systems per batch
-  int systems_per_wave = 1;  // batches: 2 runs transit systems of equal body count two per wave (nbg_run_duo)
+  int systems_per_wave = 1;  // batches: 2 runs transit systems of equal body count two a workgroup (nbg_run_duo, nbg_run_split_duo)
   int row_update = 0;        // Jacobian row update: 0 the reference's order (bitwise), 1 factored
   int64_t coop_polls = 0;  // > 0: bound on the inter-wave waits of transit runs (diagnostic); 0: the defaults
   int nstreams = 4;
@@ -420,7 +420,7 @@ nbg::SysBufs bufs_of(Store& S) {
   return B;
 }
 
-// Launch every group (one persistent kernel per body count) and wait.
+// Launch every group (one persistent kernel a class, or one for all) and wait.
 int run_groups(nbg_ctx* ctx, Store& S, const Layout& L, int64_t chunk, double* kernel_ms,
                std::vector<float>* group_ms = nullptr, std::vector<unsigned long long>* units = nullptr,
                const nbg::SysBufs* bufs = nullptr, std::vector<int>* group_grid = nullptr) {

@@ -1,5 +1,6 @@
-// nbg_split.h -- device code of the two-wave launches (nbg_run_split): the
-// state of a system, or of two, on one wave and its Jacobian on another.
+// nbg_split.h -- device code of the two- and three-wave launches
+// (nbg_run_split, nbg_run_split_duo, nbg_run_split_wide): the state of a
+// system, or of two, on one wave and its Jacobian on another, or on two.
 //
 // The state of AHL21 never reads the Jacobian, so a workgroup divides every
 // step between two waves:
@@ -8,12 +9,13 @@
 //  * the Jacobian wave follows: the pairs' analytic Jacobians, the row
 //    updates, Phi and its product, the drifts of J, dq/dt, and the transits'
 //    gradients.
-// Alone on a compute unit the two run on different SIMDs and a step takes the
-// longer of the two instead of their sum; with four workgroups a compute unit
-// each SIMD holds two waves, so that one issues while the other waits (a lone
-// wave issues vector instructions about 40 % of the time).  The half of the
-// code that each wave runs also keeps registers within the 256 that two waves
-// per SIMD leave each.
+// With four workgroups a compute unit each SIMD holds two waves, so that one
+// issues while the other waits (a lone wave issues vector instructions about
+// 40 % of the time); the half of the code that each wave runs also keeps
+// registers within the 256 that two waves per SIMD leave each.  Few systems
+// have a compute unit each: there the waves run on different SIMDs, a step
+// takes the longest of them instead of their sum, and the Jacobian wave's work
+// is divided between two (a pair wave and a row wave, at SplitLds3 below).
 //
 // The waves talk through LDS: a ring of pair slots (22 doubles each; the rest
 // of a pair's drift is formed again from them, with the same operations) and

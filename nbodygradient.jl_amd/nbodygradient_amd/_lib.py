@@ -161,10 +161,10 @@ class Context:
         self.check(lib().nbg_set_grid_cap(self._h, int(grid_cap)), "nbg_set_grid_cap")
 
     def set_systems_per_wave(self, k=1):
-        """Batch runs and rounds: 1 system per wave, or 2 (transit runs of
-        equal body count, n <= 9) in lockstep with their Kepler pairs sharing
-        the wave's lanes; results are the same bits either way (C ABI:
-        nbg_set_systems_per_wave)."""
+        """Batch runs and rounds: 1 system a workgroup, or 2 (transit runs of
+        equal body count, n <= 7; n <= 9 in classes on one wave a system) in
+        lockstep with their Kepler pairs sharing a wave's lanes; results are
+        the same bits either way (C ABI: nbg_set_systems_per_wave)."""
         self.check(lib().nbg_set_systems_per_wave(self._h, int(k)), "nbg_set_systems_per_wave")
 
     def set_row_update(self, mode=0):
@@ -176,13 +176,16 @@ class Context:
         self.check(lib().nbg_set_row_update(self._h, int(mode)), "nbg_set_row_update")
 
     def set_coop(self, mode=1, max_systems=128):
-        """Two-wave workgroups for the longest transit-search systems of batch
-        runs: 0 off, 1 automatic (default), 2 the longest max_systems."""
+        """Cooperative workgroups (transit search on a second wave) for the
+        longest systems of batch runs: 0 off, 1 automatic (default; classes
+        that divide their steps between waves are left out), 2 the longest
+        max_systems."""
         self.check(lib().nbg_set_coop(self._h, int(mode), int(max_systems)), "nbg_set_coop")
 
     def set_coop_wait(self, polls=0):
-        """Diagnostic: bound each wait between the two waves of a cooperative
-        workgroup (0: defaults)."""
+        """Diagnostic: bound each wait between the waves of a workgroup, in
+        runs with a transit search and cooperative workgroups not turned off
+        (0: defaults)."""
         self.check(lib().nbg_set_coop_wait(self._h, int(polls)), "nbg_set_coop_wait")
 
     def close(self):

@@ -93,10 +93,11 @@ class Batch:
 
     def autotune(self, frac=0.05):
         """nbg_batch_autotune: time a copy of this batch with every step count
-        scaled by frac under each candidate launch configuration (two-wave
+        scaled by frac under each candidate launch configuration (cooperative
         workgroups off / automatic / for the 16, 32, 64 longest systems;
-        four or three one-wave workgroups per CU; one or two systems per
-        wave) and keep the fastest in the context.  Returns the candidates with their times and the choice."""
+        four or three workgroups per CU; one or two systems a workgroup) and
+        keep the fastest in the context.  Returns the candidates with their
+        times and the choice."""
         L = _lib.lib()
         nc = L.nbg_batch_autotune_candidate(-1, None, None, None)
         ms = np.zeros(nc)
