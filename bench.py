@@ -58,8 +58,8 @@ FP64_PEAK_TFLOPS = 78.6
 # in profiles/nbg_run_split_c2_round.md and
 # nbg_run_split_duo_c2_round_counters.md); a configuration without a
 # measurement of the current kernels reports traffic null
-HBM_BYTES_PER_UNIT = {("nbg_run_split<11>", 0): 282.7e3, ("nbg_run_split<11>", 1): 258.8e3,
-                      ("nbg_run_split_duo<9>", 0): 447.0e3, ("nbg_run_split_duo<9>", 1): 398.6e3}
+HBM_BYTES_PER_UNIT = {("nbg_run_split<11>", 0): 282.3e3, ("nbg_run_split<11>", 1): 257.8e3,
+                      ("nbg_run_split_duo<9>", 0): 446.7e3, ("nbg_run_split_duo<9>", 1): 399.4e3}
 METRIC = "system-steps/s w/ Jacobian, batched vs plain GPU; p50/p99 request latency"
 T_START = time.perf_counter()
 
